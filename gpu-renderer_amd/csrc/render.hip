@@ -218,16 +218,14 @@ __global__ __launch_bounds__(256) void k_gen(RenderArgs a) {
     }
 }
 
-template <class Stack>
-GPR_D gpr_hit trace_one(const RenderArgs& a, const SceneView& sv, const Ray3& r, Stack& st, bool any,
-                        bool ref_order) {
+template <bool ANY, bool REF_ORDER, class Stack>
+GPR_D gpr_hit trace_one(const RenderArgs& a, const SceneView& sv, const Ray3& r, Stack& st) {
     gpr_hit h;
-    if (ref_order) {
+    if constexpr (REF_ORDER) {
         uint32_t nv = 0, nt = 0;
-        h = any ? ref_trace<true>(sv, r, &nv, &nt) : ref_trace<false>(sv, r, &nv, &nt);
+        h = ref_trace<ANY>(sv, r, &nv, &nt);
     } else {
-        const bool ok = any ? fast_trace<true>(sv, r, st, h) : fast_trace<false>(sv, r, st, h);
-        if (!ok) atomicOr(&a.ctrl->error, 1u);
+        if (!fast_trace<ANY>(sv, r, st, h)) atomicOr(&a.ctrl->error, 1u);
     }
     return h;
 }
@@ -397,11 +395,11 @@ GPR_D void shadow_finish(const RenderArgs& a, const QueueView& q, uint32_t i, co
 // REFILL: per-lane ray refill (BVH4 traversal only).
 template <bool PRIMARY, bool REF_ORDER, bool MULTI, int NT, int SL, bool REFILL = false>
 __global__ __launch_bounds__(NT) void k_extend(RenderArgs a, uint32_t bounce) {
-    __shared__ int2 lds[SL * NT];
-    LaneStackT<NT, SL> st;
+    using Stack = LaneStack<false, NT, SL>;
+    __shared__ typename Stack::Entry lds[SL * NT];
+    Stack st;
     st.lds = lds + threadIdx.x;
-    st.spill = a.spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal;
-    st.sp = 0;
+    st.spill = reinterpret_cast<typename Stack::Entry*>(a.spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal);
     // queue: primary = A; at bounce b the scatter queue is q[(b+1)&1]
     const QueueView& q = a.q[PRIMARY ? 0 : ((bounce + 1) & 1)];
     const uint32_t n = PRIMARY ? npaths_of<MULTI>(a) : a.ctrl->scatter_size[bounce];
@@ -415,14 +413,15 @@ __global__ __launch_bounds__(NT) void k_extend(RenderArgs a, uint32_t bounce) {
             [&](uint32_t i) {
                 ei = i;
                 sv = scene_of<MULTI>(a, q, i);
-                if (!trav_begin<false>(sv, queue_ray(q, i), st, t)) return false;
+                trav_begin<false>(sv, queue_ray(q, i), st, t);
+                if (trav_live(sv, t)) return false;
                 extend_finish<PRIMARY, MULTI>(a, q, i, sv, t.r, t.hit, bounce);
                 return true;
             },
             [&]() {
-                const int rc = trav_step<false>(sv, st, t);
-                if (rc == kTravMore) return false;
-                if (rc == kTravOverflow) atomicOr(&a.ctrl->error, 1u);
+                trav_step<false>(sv, st, t);
+                if (trav_live(sv, t)) return false;
+                if (t.node != kTravDone) atomicOr(&a.ctrl->error, 1u);
                 extend_finish<PRIMARY, MULTI>(a, q, ei, sv, t.r, t.hit, bounce);
                 return true;
             });
@@ -430,7 +429,7 @@ __global__ __launch_bounds__(NT) void k_extend(RenderArgs a, uint32_t bounce) {
         for_each_claimed(cur, n, a.chunk, [&](uint32_t i) {
             const SceneView sv = scene_of<MULTI>(a, q, i);
             const Ray3 r = queue_ray(q, i);
-            const gpr_hit h = trace_one(a, sv, r, st, false, REF_ORDER);
+            const gpr_hit h = trace_one<false, REF_ORDER>(a, sv, r, st);
             extend_finish<PRIMARY, MULTI>(a, q, i, sv, r, h, bounce);
         });
     }
@@ -439,11 +438,11 @@ __global__ __launch_bounds__(NT) void k_extend(RenderArgs a, uint32_t bounce) {
 // shadow: any hit + accumulate_light_sampling_contribution (pathtracer_kernel.h:642-664)
 template <bool REF_ORDER, bool MULTI, int NT, int SL, bool REFILL = false>
 __global__ __launch_bounds__(NT) void k_shadow(RenderArgs a, uint32_t bounce) {
-    __shared__ int2 lds[SL * NT];
-    LaneStackT<NT, SL> st;
+    using Stack = LaneStack<true, NT, SL>;
+    __shared__ typename Stack::Entry lds[SL * NT];
+    Stack st;
     st.lds = lds + threadIdx.x;
-    st.spill = a.spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal;
-    st.sp = 0;
+    st.spill = reinterpret_cast<typename Stack::Entry*>(a.spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal);
     const QueueView& q = a.q[2];
     const uint32_t n = a.ctrl->shadow_size[bounce];
     uint32_t* cur = &a.ctrl->sh_cursor[bounce];
@@ -456,21 +455,22 @@ __global__ __launch_bounds__(NT) void k_shadow(RenderArgs a, uint32_t bounce) {
             [&](uint32_t i) {
                 ei = i;
                 sv = scene_of<MULTI>(a, q, i);
-                if (!trav_begin<true>(sv, queue_ray(q, i), st, t)) return false;
+                trav_begin<true>(sv, queue_ray(q, i), st, t);
+                if (trav_live(sv, t)) return false;
                 shadow_finish(a, q, i, t.hit);
                 return true;
             },
             [&]() {
-                const int rc = trav_step<true>(sv, st, t);
-                if (rc == kTravMore) return false;
-                if (rc == kTravOverflow) atomicOr(&a.ctrl->error, 1u);
+                trav_step<true>(sv, st, t);
+                if (trav_live(sv, t)) return false;
+                if (t.node != kTravDone) atomicOr(&a.ctrl->error, 1u);
                 shadow_finish(a, q, ei, t.hit);
                 return true;
             });
     } else {
         for_each_claimed(cur, n, a.chunk, [&](uint32_t i) {
             const SceneView sv = scene_of<MULTI>(a, q, i);
-            const gpr_hit h = trace_one(a, sv, queue_ray(q, i), st, true, REF_ORDER);
+            const gpr_hit h = trace_one<true, REF_ORDER>(a, sv, queue_ray(q, i), st);
             shadow_finish(a, q, i, h);
         });
     }

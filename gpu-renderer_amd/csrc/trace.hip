@@ -44,11 +44,11 @@ __global__ __launch_bounds__(NT) void k_trace_fast(SceneView sv, const gpr_ray* 
                                                    gpr_hit* __restrict__ hits, uint64_t n,
                                                    unsigned long long* __restrict__ cursor,
                                                    int2* __restrict__ spill, uint32_t chunk) {
-    __shared__ int2 lds[SL * NT];
-    LaneStackT<NT, SL> st;
+    using Stack = LaneStack<ANY, NT, SL>;
+    __shared__ typename Stack::Entry lds[SL * NT];
+    Stack st;
     st.lds = lds + threadIdx.x;
-    st.spill = spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal;
-    st.sp = 0;
+    st.spill = reinterpret_cast<typename Stack::Entry*>(spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal);
     const int lane = threadIdx.x & 63;
     while (true) {
         unsigned long long base = 0;
@@ -72,8 +72,8 @@ __global__ __launch_bounds__(NT) void k_trace_fast(SceneView sv, const gpr_ray* 
 // of `chunk` ray indices (one global atomic per chunk), so no lane idles while
 // the slowest ray of the wave finishes.  A closest-hit ray takes the same
 // node steps as in k_trace_fast, so the hits are identical.  Any hit parks
-// leaf children and tests them in wave-wide leaf rounds (TravD): the
-// occlusion answer is the same, the occluder reported may differ.
+// leaf children and tests them in wave-wide leaf rounds (TravD), before the
+// lane's next node: its hits are those of k_trace_fast too.
 constexpr int kLeafRound = 32;  // parked lanes of a wave that start an any-hit leaf round
 
 template <bool ANY, int NT, int SL>
@@ -81,11 +81,11 @@ __global__ __launch_bounds__(NT) void k_trace_refill(SceneView sv, const gpr_ray
                                                      gpr_hit* __restrict__ hits, uint64_t n,
                                                      unsigned long long* __restrict__ cursor,
                                                      int2* __restrict__ spill, uint32_t chunk) {
-    __shared__ int2 lds[SL * NT];
-    LaneStackT<NT, SL> st;
+    using Stack = LaneStack<ANY, NT, SL>;
+    __shared__ typename Stack::Entry lds[SL * NT];
+    Stack st;
     st.lds = lds + threadIdx.x;
-    st.spill = spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal;
-    st.sp = 0;
+    st.spill = reinterpret_cast<typename Stack::Entry*>(spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal);
     const int lane = threadIdx.x & 63;
     uint64_t pb = 0, pe = 0;  // wave-local pool [pb, pe) of ray indices (wave-uniform)
     bool drained = false;     // the global cursor has passed n (wave-uniform)
@@ -114,12 +114,9 @@ __global__ __launch_bounds__(NT) void k_trace_refill(SceneView sv, const gpr_ray
                 const uint64_t idx = from_old ? pb + rank : nb + (rank - avail);
                 if (from_old || idx < ne) {
                     ri = idx;
-                    const Ray3 r = load_ray(rays, ri);
-                    bool done;
-                    if constexpr (ANY) done = travd_begin<ANY>(sv, r, st, t);
-                    else done = trav_begin<ANY>(sv, r, st, t);
-                    if (done) store_hit(hits, ri, t.hit);
-                    else active = true;
+                    trav_begin<ANY>(sv, load_ray(rays, ri), st, t);
+                    if constexpr (ANY) t.pmask = 0;
+                    active = true;
                 }
             }
             if (avail >= cnt) {
@@ -135,27 +132,26 @@ __global__ __launch_bounds__(NT) void k_trace_refill(SceneView sv, const gpr_ray
             continue;
         }
         if constexpr (ANY) {
-            if (active && t.pmask == 0) {
-                const int rc = travd_step<ANY>(sv, st, t);
-                if (rc != kTravMore) {
-                    if (rc == kTravOverflow) atomicAdd(cursor + 1, 1ull);  // stack overflow count
-                    store_hit(hits, ri, t.hit);
-                    active = false;
-                }
-            }
+            if (active && t.pmask == 0 && trav_live(sv, t)) travd_step(sv, st, t);
             // leaf round: when enough lanes have parked leaves, or no lane can step
             const unsigned long long parked = __ballot(active && t.pmask != 0);
-            if (parked != 0ull && (__popcll(parked) >= kLeafRound || __ballot(active && t.pmask == 0) == 0ull)) {
-                if (active && t.pmask != 0 && travd_leaves<ANY>(sv, t)) {
-                    store_hit(hits, ri, t.hit);
-                    active = false;
+            if (parked != 0ull &&
+                (__popcll(parked) >= kLeafRound || __ballot(active && t.pmask == 0 && trav_live(sv, t)) == 0ull)) {
+                if (active && t.pmask != 0) {
+                    travd_leaves(sv, t);
+                    if (t.found) t.node = kTravDone;
                 }
+            }
+            if (active && t.pmask == 0 && !trav_live(sv, t)) {
+                if (t.node != kTravDone) atomicAdd(cursor + 1, 1ull);  // stack overflow count
+                store_hit(hits, ri, t.hit);
+                active = false;
             }
         } else {
             if (active) {
-                const int rc = trav_step<ANY>(sv, st, t);
-                if (rc != kTravMore) {
-                    if (rc == kTravOverflow) atomicAdd(cursor + 1, 1ull);  // stack overflow count
+                if (trav_live(sv, t)) trav_step<ANY>(sv, st, t);
+                if (!trav_live(sv, t)) {
+                    if (t.node != kTravDone) atomicAdd(cursor + 1, 1ull);  // stack overflow count
                     store_hit(hits, ri, t.hit);
                     active = false;
                 }
@@ -195,19 +191,19 @@ template <bool ANY>
 __global__ __launch_bounds__(256) void k_trace_stats(SceneView sv, const gpr_ray* __restrict__ rays, uint64_t n,
                                                      unsigned long long* __restrict__ stats,
                                                      int2* __restrict__ spill) {
-    __shared__ int2 lds[16 * 256];
-    LaneStackT<256, 16> st;
+    using Stack = LaneStack<ANY, 256, 16>;
+    __shared__ typename Stack::Entry lds[16 * 256];
+    Stack st;
     st.lds = lds + threadIdx.x;
-    st.spill = spill + (uint64_t)(blockIdx.x * 256 + threadIdx.x) * kStackGlobal;
-    st.sp = 0;
+    st.spill = reinterpret_cast<typename Stack::Entry*>(spill + (uint64_t)(blockIdx.x * 256 + threadIdx.x) * kStackGlobal);
     unsigned long long nf = 0, nt = 0, ov = 0;
     for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) {
         Trav t;
-        int rc = trav_begin<ANY>(sv, load_ray(rays, i), st, t) ? kTravDone : kTravMore;
-        while (rc == kTravMore) rc = trav_step<ANY>(sv, st, t);
+        trav_begin<ANY>(sv, load_ray(rays, i), st, t);
+        while (trav_live(sv, t)) trav_step<ANY>(sv, st, t);
         nf += t.fetched;
         nt += t.tested + (sv.root4 < 0 ? 1u : 0u);
-        ov += rc == kTravOverflow ? 1u : 0u;
+        ov += t.node != kTravDone ? 1u : 0u;
     }
     for (int o = 32; o > 0; o >>= 1) {
         nf += __shfl_down(nf, o, 64);

@@ -9,8 +9,8 @@
 //              test on all four children, nearest-first descent, leaf triangles
 //              tested as soon as their parent is visited (the persistent any-hit
 //              kernel instead parks them for wave-wide leaf rounds, TravD), and a
-//              short per-lane stack in LDS that spills its oldest entries to a
-//              global overflow area.  Closest-hit results equal the reference's up
+//              short per-lane stack in LDS whose youngest entries go to a global
+//              overflow area when it is full.  Closest-hit results equal the reference's up
 //              to ties of t.
 #pragma once
 
@@ -19,9 +19,7 @@
 
 namespace gpr {
 
-constexpr int kStackLds = 16;      // LDS stack entries per lane (power of two)
 constexpr int kStackGlobal = 96;   // global overflow entries per lane
-constexpr int kTraceBlock = 256;
 
 struct Ray3 {
     v3 o, d;
@@ -119,32 +117,48 @@ GPR_D gpr_hit ref_trace(const SceneView& sv, Ray3 r, uint32_t* nvisit, uint32_t*
 }
 
 // ------------------------------------------------------ BVH4 traversal ---
-// Per-lane traversal stack: the top SL entries in an LDS column of a block of
-// NT lanes (entry k at lds[k * NT]), older entries spilled to a per-lane global
-// slab of kStackGlobal entries.
-template <int NT, int SL>
+// Per-lane traversal stack: the oldest SL entries in an LDS column of a block
+// of NT lanes (entry k at lds[k * NT]), the rest in a per-lane global slab of
+// kStackGlobal entries (walks rarely reach it).  Entry 0 is a sentinel that
+// every pop accepts and that ends the walk, so popping needs no empty test.
+// Closest hit keeps 8 bytes per entry (the order key and the child), any hit
+// only the child.
+template <class E, int NT, int SL>
 struct LaneStackT {
-    static_assert((SL & (SL - 1)) == 0, "LDS stack depth must be a power of two");
-    int2* lds;    // this lane's column
-    int2* spill;  // this lane's overflow area (kStackGlobal entries)
+    static constexpr int kNT = NT, kSL = SL;
+    using Entry = E;
+    E* lds;    // this lane's column
+    E* spill;  // this lane's overflow area (kStackGlobal entries)
     int sp;
-    GPR_D bool push(int2 e) {
-        if (sp >= SL + kStackGlobal) return false;
-        const int slot = sp & (SL - 1);
-        if (sp >= SL) spill[sp - SL] = lds[slot * NT];
-        lds[slot * NT] = e;
-        ++sp;
-        return true;
+    GPR_D void reset(E sentinel) {
+        lds[0] = sentinel;
+        sp = 1;
     }
-    GPR_D int2 pop() {
+    GPR_D void put(int at, E e) {
+        if (at < SL) lds[at * NT] = e;
+        else spill[at - SL] = e;
+    }
+    GPR_D E pop() {
         --sp;
-        const int slot = sp & (SL - 1);
-        const int2 e = lds[slot * NT];
-        if (sp >= SL) lds[slot * NT] = spill[sp - SL];
-        return e;
+        if (sp >= SL) return spill[sp - SL];
+        return lds[sp * NT];
     }
+    // true when no active lane of the wave could leave the LDS part by pushing k entries
+    GPR_D bool roomy(int k) const { return __ballot(sp + k > SL) == 0ull; }
+    GPR_D bool full(int k) const { return sp + k > SL + kStackGlobal; }
 };
-using LaneStack = LaneStackT<kTraceBlock, kStackLds>;
+// Stack entry of a walk: closest hit (order key, child << 2 | low bits of the
+// entry distance), any hit (child).
+template <bool ANY>
+struct StackEntry {
+    using type = uint2;
+};
+template <>
+struct StackEntry<true> {
+    using type = int32_t;
+};
+template <bool ANY, int NT, int SL>
+using LaneStack = LaneStackT<typename StackEntry<ANY>::type, NT, SL>;
 
 GPR_D void tri_rec_hit(const TriRec* tris, uint32_t ntri, int32_t leaf, const Ray3& r, float& tmax,
                        gpr_hit& hit, bool& found) {
@@ -164,11 +178,13 @@ GPR_D void tri_rec_hit(const TriRec* tris, uint32_t ntri, int32_t leaf, const Ra
 // each trav_step visits one node (its leaf children are tested first, they
 // tighten tmax before the descent decision), so a caller can either run a ray
 // to completion (fast_trace) or interleave the steps of many rays and give a
-// lane a new ray as soon as its ray is done.
+// lane a new ray as soon as its ray is done.  The walk goes on while
+// trav_live(); node is then kTravDone, or anything else outside the tree when
+// the stack ran out (or the tree is malformed).
 struct Trav {
     Ray3 r;
     v3 inv;
-    int sx, sy, sz;  // 1 where the direction component is negative: the far plane comes first
+    uint32_t ox, oy, oz;  // byte offset of each axis' near planes in a node (far planes: offset ^ 16)
     float tmax;
     gpr_hit hit;
     int32_t node;
@@ -177,266 +193,232 @@ struct Trav {
     bool found;
 };
 constexpr float kSlabCons = 1.0f + 2.0f * 1.7881394e-07f;  // 1 + 2*gamma(3)
-enum : int { kTravMore = 0, kTravDone = 1, kTravOverflow = 2 };
+enum : int32_t { kTravDone = 0x3fffffff, kTravOverflow = -1 };  // no node: a tree holds fewer than 2^30 - 1 nodes (137 GB)
+constexpr uint32_t kKeyNone = 0x7fefffffu;  // order key of a child not taken: above every key, and no NaN as a double's high word
 
-// Returns true when the ray is already finished (single-triangle scene).
 template <bool ANY, class Stack>
-GPR_D bool trav_begin(const SceneView& sv, const Ray3& r, Stack& st, Trav& t) {
+GPR_D void trav_begin(const SceneView& sv, const Ray3& r, Stack& st, Trav& t) {
     t.r = r;
     t.hit = gpr_hit{INFINITY, -1, 0.f, 0.f};
     t.tmax = r.tmax;
     t.found = false;
     t.fetched = 0;
     t.tested = 0;
-    st.sp = 0;
-    if (sv.root4 < 0) {
-        tri_rec_hit(sv.tris, sv.ntri, ~sv.root4, r, t.tmax, t.hit, t.found);
-        return true;
-    }
+    // the sentinel's entry distance is -inf: no limit culls it
+    if constexpr (ANY) st.reset(kTravDone);
+    else st.reset(make_uint2((uint32_t)kTravDone << 2, 0xff800000u));
     t.inv = V(1 / r.d.x, 1 / r.d.y, 1 / r.d.z);
-    t.sx = __builtin_signbit(t.inv.x) ? 1 : 0;
-    t.sy = __builtin_signbit(t.inv.y) ? 1 : 0;
-    t.sz = __builtin_signbit(t.inv.z) ? 1 : 0;
+    t.ox = __builtin_signbit(t.inv.x) ? 16u : 0u;
+    t.oy = __builtin_signbit(t.inv.y) ? 48u : 32u;
+    t.oz = __builtin_signbit(t.inv.z) ? 80u : 64u;
     t.node = sv.root4;
-    return false;
+    if (sv.root4 < 0) {  // single-triangle scene: finished at once
+        tri_rec_hit(sv.tris, sv.ntri, ~sv.root4, r, t.tmax, t.hit, t.found);
+        t.node = kTravDone;
+    }
 }
 
-template <bool ANY, class Stack>
-GPR_D int trav_step(const SceneView& sv, Stack& st, Trav& t) {
-    // a depth-first walk fetches every node at most once: the cap only trips on a malformed tree
-    if ((uint32_t)t.node >= sv.nbvh4 || t.fetched > sv.nbvh4) return kTravOverflow;
-    const Ray3& r = t.r;
-    const float4* np = reinterpret_cast<const float4*>(sv.bvh4 + t.node);
+// Whether the walk goes on.  A depth-first walk fetches every node at most
+// once: the second bound only trips on a malformed tree.
+GPR_D bool trav_live(const SceneView& sv, const Trav& t) {
+    return (uint32_t)t.node < sv.nbvh4 && t.fetched <= sv.nbvh4;
+}
+
+// 64-bit minimum / maximum of two (order key, payload) pairs as doubles: keys
+// are float bit patterns below 0x7ff00000, so the pairs are non-negative
+// doubles that order by key; one instruction each instead of a compare and
+// two selects, and the payload travels with its key.
+GPR_D void key_sort2(double& a, double& b) {
+    double lo, hi;
+    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+    a = lo;
+    b = hi;
+}
+GPR_D double key_pair(uint32_t key, uint32_t payload) { return __hiloint2double((int)key, (int)payload); }
+GPR_D uint32_t key_of(double e) { return (uint32_t)__double2hiint(e); }
+
+// One node's box tests: leaf children in leaf_mask (slot order), inner
+// children that the ray meets in hitc, entry distances in tn.
+struct NodeHits {
+    float tn[4];
+    int32_t ch[4];
+    bool hitc[4];
+    uint32_t leaf_mask;
+};
+GPR_D void trav_boxes(const SceneView& sv, const Trav& t, NodeHits& h) {
     // the ray enters each slab at the plane its direction meets first: near
-    // and far planes are loaded by the direction's signs (lx/hx at np[0]/np[1],
-    // ly/hy at np[2]/np[3], lz/hz at np[4]/np[5]), so no per-axis min / max.
-    // A 0 * inf (ray in a slab plane) gives NaN, which fmaxf / fminf ignore:
-    // that axis then does not cull the child.
-    const float4 nx = ldg(np + 0 + t.sx), fx = ldg(np + 1 - t.sx), ny = ldg(np + 2 + t.sy), fy = ldg(np + 3 - t.sy);
-    const float4 nz = ldg(np + 4 + t.sz), fz = ldg(np + 5 - t.sz);
-    const int4 ch = ldg(reinterpret_cast<const int4*>(np + 6));
+    // and far planes are loaded by the direction's signs, so no per-axis min
+    // / max.  A 0 * inf (ray in a slab plane) gives NaN, which fmaxf / fminf
+    // ignore: that axis then does not cull the child.
+    const char* np = reinterpret_cast<const char*>(sv.bvh4) + ((uint64_t)(uint32_t)t.node << 7);
+    const auto plane = [&](uint32_t off) { return ldg(reinterpret_cast<const float4*>(np + off)); };
+    const float4 nx = plane(t.ox), fx = plane(t.ox ^ 16u), ny = plane(t.oy), fy = plane(t.oy ^ 16u);
+    const float4 nz = plane(t.oz), fz = plane(t.oz ^ 16u);
+    const int4 ch = ldg(reinterpret_cast<const int4*>(np + 96));
     const float nxa[4] = {nx.x, nx.y, nx.z, nx.w}, fxa[4] = {fx.x, fx.y, fx.z, fx.w};
     const float nya[4] = {ny.x, ny.y, ny.z, ny.w}, fya[4] = {fy.x, fy.y, fy.z, fy.w};
     const float nza[4] = {nz.x, nz.y, nz.z, nz.w}, fza[4] = {fz.x, fz.y, fz.z, fz.w};
-    const int32_t cha[4] = {ch.x, ch.y, ch.z, ch.w};
-    float tn[4];
-    bool hitc[4];
+    h.ch[0] = ch.x;
+    h.ch[1] = ch.y;
+    h.ch[2] = ch.z;
+    h.ch[3] = ch.w;
+    h.leaf_mask = 0;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-        const float x0 = (nxa[c] - r.o.x) * t.inv.x, x1 = (fxa[c] - r.o.x) * t.inv.x;
-        const float y0 = (nya[c] - r.o.y) * t.inv.y, y1 = (fya[c] - r.o.y) * t.inv.y;
-        const float z0 = (nza[c] - r.o.z) * t.inv.z, z1 = (fza[c] - r.o.z) * t.inv.z;
-        const float tnear = fmaxf(fmaxf(x0, y0), fmaxf(z0, r.tmin));
+        const float x0 = (nxa[c] - t.r.o.x) * t.inv.x, x1 = (fxa[c] - t.r.o.x) * t.inv.x;
+        const float y0 = (nya[c] - t.r.o.y) * t.inv.y, y1 = (fya[c] - t.r.o.y) * t.inv.y;
+        const float z0 = (nza[c] - t.r.o.z) * t.inv.z, z1 = (fza[c] - t.r.o.z) * t.inv.z;
+        const float tnear = fmaxf(fmaxf(x0, y0), fmaxf(z0, t.r.tmin));
         const float tfar = fminf(fminf(x1, y1), fminf(z1, t.tmax));
-        tn[c] = tnear;
-        hitc[c] = tnear <= tfar * kSlabCons && cha[c] != kEmptyChild;
+        h.tn[c] = tnear;
+        const bool in = tnear <= tfar * kSlabCons;
+        h.hitc[c] = in && h.ch[c] >= 0;
+        h.leaf_mask |= (in && (uint32_t)h.ch[c] > (uint32_t)kEmptyChild) ? 1u << c : 0u;
     }
+}
+// child reference of the lowest slot set in m (m != 0)
+GPR_D int32_t lowest_child(const NodeHits& h, uint32_t m) {
+    const int c = __builtin_ctz(m);
+    const int32_t lo = (c & 1) ? h.ch[1] : h.ch[0], hi = (c & 1) ? h.ch[3] : h.ch[2];
+    return (c & 2) ? hi : lo;
+}
+
+// Descends after a closest-hit node's leaves: the nearest inner child next,
+// the others pushed far to near, or the nearest pending node that can still
+// hold a closer hit.  Children order by their entry distance with the slot in
+// its two low bits; those bits travel with the child, so a pop compares the
+// distance as computed.  The walk is bound by instruction issue as much as by
+// the cache (a wave runs ~490 vector instructions per node it steps), so the
+// pushes carry no loop and no branch: against a push loop over a sorted key
+// list with child selects, 4M incoherent rays at 1M triangles take 3.47 ms
+// instead of 3.97 wave-synchronous and 2.78 instead of 2.82 refilled, 700K
+// any-hit rays at 262K triangles 0.69 ms instead of 0.79.
+template <class Stack>
+GPR_D void trav_descend(Stack& st, Trav& t, const NodeHits& h) {
+    const float lim = t.tmax * kSlabCons;
+    double e[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const bool go = h.hitc[c] && h.tn[c] <= lim;
+        const uint32_t tb = __float_as_uint(h.tn[c]);
+        const uint32_t key = go ? ((__float_as_uint(fmaxf(h.tn[c], 0.f)) & ~3u) | (uint32_t)c) : kKeyNone;
+        e[c] = key_pair(key, ((uint32_t)h.ch[c] << 2) | (tb & 3u));
+    }
+    key_sort2(e[0], e[1]);
+    key_sort2(e[2], e[3]);
+    key_sort2(e[0], e[2]);
+    key_sort2(e[1], e[3]);
+    key_sort2(e[1], e[2]);
+    ++t.fetched;
+    using E = typename Stack::Entry;
+    const auto entry = [](double v) { return make_uint2((uint32_t)__double2loint(v), (uint32_t)__double2hiint(v)); };
+    if (st.roomy(3)) {
+        // written without a branch: a slot whose child is not taken is
+        // overwritten by the next entry (or left above the top)
+#pragma unroll
+        for (int k = 3; k >= 1; --k) {
+            st.lds[st.sp * Stack::kNT] = entry(e[k]);
+            st.sp += key_of(e[k]) != kKeyNone ? 1 : 0;
+        }
+    } else {
+        if (st.full(3)) {
+            t.node = kTravOverflow;
+            return;
+        }
+#pragma unroll
+        for (int k = 3; k >= 1; --k)
+            if (key_of(e[k]) != kKeyNone) st.put(st.sp++, entry(e[k]));
+    }
+    uint32_t next = (uint32_t)__double2loint(e[0]);
+    if (key_of(e[0]) == kKeyNone) {
+        // distances below 0 (rays with tmin < 0) order and compare as 0
+        const float plim = fmaxf(lim, __uint_as_float(4u));
+        E p;
+        do {
+            p = st.pop();
+        } while (__uint_as_float((p.y & ~3u) | (p.x & 3u)) > plim);
+        next = p.x;
+    }
+    t.node = (int32_t)(next >> 2);
+}
+
+// Any hit needs no near-to-far order (any occluder ends the walk): the lowest
+// hit slot is visited first and the others pushed, with no sorting network.
+template <class Stack>
+GPR_D void trav_descend_any(Stack& st, Trav& t, const NodeHits& h) {
+    ++t.fetched;
+    int32_t next = -1;
+    if (st.roomy(3)) {
+#pragma unroll
+        for (int c = 3; c >= 0; --c) {
+            if (c < 3) st.lds[st.sp * Stack::kNT] = next;
+            st.sp += (c < 3 && h.hitc[c] && next >= 0) ? 1 : 0;
+            next = h.hitc[c] ? h.ch[c] : next;
+        }
+    } else {
+        if (st.full(3)) {
+            t.node = kTravOverflow;
+            return;
+        }
+#pragma unroll
+        for (int c = 3; c >= 0; --c) {
+            if (c < 3 && h.hitc[c] && next >= 0) st.put(st.sp++, next);
+            next = h.hitc[c] ? h.ch[c] : next;
+        }
+    }
+    t.node = next >= 0 ? next : st.pop();
+}
+
+// One node of a live walk.
+template <bool ANY, class Stack>
+GPR_D void trav_step(const SceneView& sv, Stack& st, Trav& t) {
+    NodeHits h;
+    trav_boxes(sv, t, h);
     // leaf children in ascending slot order, as a loop over this lane's own
     // leaves: a wave runs the triangle test as often as its busiest lane
     // needs it, not once per slot that any lane has a leaf in
-    uint32_t leaves = 0;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) leaves |= (hitc[c] && cha[c] < 0) ? 1u << c : 0u;
+    uint32_t leaves = h.leaf_mask;
     while (leaves != 0) {
-        const int c = __builtin_ctz(leaves);
+        const int32_t leaf = lowest_child(h, leaves);
         leaves &= leaves - 1;
-        const int32_t leaf = c == 0 ? cha[0] : c == 1 ? cha[1] : c == 2 ? cha[2] : cha[3];
-        tri_rec_hit(sv.tris, sv.ntri, ~leaf, r, t.tmax, t.hit, t.found);
-        ++t.tested;
-        if (ANY && t.found) return kTravDone;
-    }
-    if constexpr (ANY) {
-        // any hit needs no near-to-far order (any occluder ends the walk): the
-        // lowest hit slot is visited first and the others pushed, with no
-        // sorting network
-        uint32_t m = 0;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) m |= (hitc[c] && cha[c] >= 0) ? 1u << c : 0u;
-        ++t.fetched;
-        if (m != 0) {
-            const int c0 = __builtin_ctz(m);
-            m &= m - 1;
-            while (m != 0) {
-                const int c = 31 - __builtin_clz(m);
-                m &= ~(1u << c);
-                const int32_t ref = c == 1 ? cha[1] : c == 2 ? cha[2] : cha[3];
-                if (!st.push(make_int2(ref, 0))) return kTravOverflow;
-            }
-            t.node = c0 == 0 ? cha[0] : c0 == 1 ? cha[1] : c0 == 2 ? cha[2] : cha[3];
-            return kTravMore;
-        }
-        if (st.sp > 0) {
-            t.node = st.pop().x;
-            return kTravMore;
-        }
-        return kTravDone;
-    }
-    uint32_t key[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const bool go = hitc[c] && cha[c] >= 0 && tn[c] <= t.tmax * kSlabCons;
-        key[c] = go ? ((__float_as_uint(fmaxf(tn[c], 0.f)) & ~3u) | (uint32_t)c) : 0xffffffffu;
-    }
-    // 4-key sorting network, ascending
-#define GPR_CSWAP(a, b)                           \
-    {                                             \
-        const uint32_t lo_ = min(key[a], key[b]); \
-        const uint32_t hi_ = max(key[a], key[b]); \
-        key[a] = lo_;                             \
-        key[b] = hi_;                             \
-    }
-    GPR_CSWAP(0, 1) GPR_CSWAP(2, 3) GPR_CSWAP(0, 2) GPR_CSWAP(1, 3) GPR_CSWAP(1, 2)
-#undef GPR_CSWAP
-    const int cnt = (key[0] != 0xffffffffu) + (key[1] != 0xffffffffu) + (key[2] != 0xffffffffu) +
-                    (key[3] != 0xffffffffu);
-    ++t.fetched;
-    if (cnt > 0) {
-        for (int k = cnt - 1; k >= 1; --k) {
-            const int c = key[k] & 3;
-            if (!st.push(make_int2(cha[c], __float_as_int(tn[c])))) return kTravOverflow;
-        }
-        t.node = cha[key[0] & 3];
-        return kTravMore;
-    }
-    // pop the nearest pending node that can still hold a closer hit
-    while (st.sp > 0) {
-        const int2 e = st.pop();
-        if (ANY || __int_as_float(e.y) <= t.tmax * kSlabCons) {
-            t.node = e.x;
-            return kTravMore;
-        }
-    }
-    return kTravDone;
-}
-
-// Postponed-leaf form of the BVH4 walk, used by the persistent any-hit
-// kernel.  A node step does not test its leaf children: it parks them (slot
-// mask + references) and the lane pauses; the wave tests the parked leaves of
-// its lanes together in one leaf round, so the (double precision) triangle
-// test runs with many lanes active instead of the few whose node held
-// leaves.  A lane descends before its leaves are tested; pops wait for the
-// round.  For an any-hit query the answer (occluded or not) is unchanged; the
-// occluder reported may be a different triangle than in the immediate order.
-struct TravD : Trav {
-    uint32_t pmask;    // parked leaf slots of the last visited node
-    int32_t pleaf[4];  // that node's child references
-};
-
-template <bool ANY, class Stack>
-GPR_D bool travd_begin(const SceneView& sv, const Ray3& r, Stack& st, TravD& t) {
-    t.pmask = 0;
-    return trav_begin<ANY>(sv, r, st, t);
-}
-
-// One node; pops first when the lane has no node to visit (kTravDone when the
-// stack is empty).  Leaves hit are parked in t.pmask / t.pleaf.
-template <bool ANY, class Stack>
-GPR_D int travd_step(const SceneView& sv, Stack& st, TravD& t) {
-    if (t.node < 0) {
-        bool got = false;
-        while (st.sp > 0) {
-            const int2 e = st.pop();
-            if (ANY || __int_as_float(e.y) <= t.tmax * kSlabCons) {
-                t.node = e.x;
-                got = true;
-                break;
-            }
-        }
-        if (!got) return kTravDone;
-    }
-    if ((uint32_t)t.node >= sv.nbvh4 || t.fetched > sv.nbvh4) return kTravOverflow;
-    const Ray3& r = t.r;
-    const float4* np = reinterpret_cast<const float4*>(sv.bvh4 + t.node);
-    const float4 nx = ldg(np + 0 + t.sx), fx = ldg(np + 1 - t.sx), ny = ldg(np + 2 + t.sy), fy = ldg(np + 3 - t.sy);
-    const float4 nz = ldg(np + 4 + t.sz), fz = ldg(np + 5 - t.sz);
-    const int4 ch = ldg(reinterpret_cast<const int4*>(np + 6));
-    const float nxa[4] = {nx.x, nx.y, nx.z, nx.w}, fxa[4] = {fx.x, fx.y, fx.z, fx.w};
-    const float nya[4] = {ny.x, ny.y, ny.z, ny.w}, fya[4] = {fy.x, fy.y, fy.z, fy.w};
-    const float nza[4] = {nz.x, nz.y, nz.z, nz.w}, fza[4] = {fz.x, fz.y, fz.z, fz.w};
-    const int32_t cha[4] = {ch.x, ch.y, ch.z, ch.w};
-    float tn[4];
-    bool hitc[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const float x0 = (nxa[c] - r.o.x) * t.inv.x, x1 = (fxa[c] - r.o.x) * t.inv.x;
-        const float y0 = (nya[c] - r.o.y) * t.inv.y, y1 = (fya[c] - r.o.y) * t.inv.y;
-        const float z0 = (nza[c] - r.o.z) * t.inv.z, z1 = (fza[c] - r.o.z) * t.inv.z;
-        const float tnear = fmaxf(fmaxf(x0, y0), fmaxf(z0, r.tmin));
-        const float tfar = fminf(fminf(x1, y1), fminf(z1, t.tmax));
-        tn[c] = tnear;
-        hitc[c] = tnear <= tfar * kSlabCons && cha[c] != kEmptyChild;
-    }
-    uint32_t leaves = 0;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        leaves |= (hitc[c] && cha[c] < 0) ? 1u << c : 0u;
-        t.pleaf[c] = cha[c];
-    }
-    t.pmask = leaves;
-    if constexpr (ANY) {
-        // as in trav_step: no distance order for any hit
-        uint32_t m = 0;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) m |= (hitc[c] && cha[c] >= 0) ? 1u << c : 0u;
-        ++t.fetched;
-        if (m != 0) {
-            const int c0 = __builtin_ctz(m);
-            m &= m - 1;
-            while (m != 0) {
-                const int c = 31 - __builtin_clz(m);
-                m &= ~(1u << c);
-                const int32_t ref = c == 1 ? cha[1] : c == 2 ? cha[2] : cha[3];
-                if (!st.push(make_int2(ref, 0))) return kTravOverflow;
-            }
-            t.node = c0 == 0 ? cha[0] : c0 == 1 ? cha[1] : c0 == 2 ? cha[2] : cha[3];
-        } else {
-            t.node = -1;
-        }
-        return kTravMore;
-    }
-    uint32_t key[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const bool go = hitc[c] && cha[c] >= 0 && tn[c] <= t.tmax * kSlabCons;
-        key[c] = go ? ((__float_as_uint(fmaxf(tn[c], 0.f)) & ~3u) | (uint32_t)c) : 0xffffffffu;
-    }
-#define GPR_CSWAP(a, b)                           \
-    {                                             \
-        const uint32_t lo_ = min(key[a], key[b]); \
-        const uint32_t hi_ = max(key[a], key[b]); \
-        key[a] = lo_;                             \
-        key[b] = hi_;                             \
-    }
-    GPR_CSWAP(0, 1) GPR_CSWAP(2, 3) GPR_CSWAP(0, 2) GPR_CSWAP(1, 3) GPR_CSWAP(1, 2)
-#undef GPR_CSWAP
-    const int cnt = (key[0] != 0xffffffffu) + (key[1] != 0xffffffffu) + (key[2] != 0xffffffffu) +
-                    (key[3] != 0xffffffffu);
-    ++t.fetched;
-    if (cnt > 0) {
-        for (int k = cnt - 1; k >= 1; --k) {
-            const int c = key[k] & 3;
-            if (!st.push(make_int2(cha[c], __float_as_int(tn[c])))) return kTravOverflow;
-        }
-        t.node = cha[key[0] & 3];
-    } else {
-        t.node = -1;
-    }
-    return kTravMore;
-}
-
-// Tests the parked leaves in slot order; true when an any-hit query is done.
-template <bool ANY>
-GPR_D bool travd_leaves(const SceneView& sv, TravD& t) {
-    uint32_t m = t.pmask;
-    t.pmask = 0;
-    while (m != 0) {
-        const int c = __builtin_ctz(m);
-        m &= m - 1;
-        const int32_t leaf = c == 0 ? t.pleaf[0] : c == 1 ? t.pleaf[1] : c == 2 ? t.pleaf[2] : t.pleaf[3];
         tri_rec_hit(sv.tris, sv.ntri, ~leaf, t.r, t.tmax, t.hit, t.found);
-        if (ANY && t.found) return true;
+        ++t.tested;
+        if (ANY && t.found) leaves = 0;
     }
-    return false;
+    if constexpr (ANY) {
+        if (t.found) t.node = kTravDone;
+        else trav_descend_any(st, t, h);
+    } else {
+        trav_descend(st, t, h);
+    }
+}
+
+// Postponed-leaf form of the any-hit walk, used by the persistent kernel.  A
+// node step does not test its leaf children: it parks them (slot mask +
+// references) and the lane pauses; the wave tests the parked leaves of its
+// lanes together in one leaf round, so the (double precision) triangle test
+// runs with many lanes active instead of the few whose node held leaves.  A
+// lane descends before its leaves are tested, and visits the next node only
+// after them: the walk and its occluder are those of trav_step.
+struct TravD : Trav {
+    uint32_t pmask;  // parked leaf slots of the last visited node
+    NodeHits h;      // that node's children
+};
+template <class Stack>
+GPR_D void travd_step(const SceneView& sv, Stack& st, TravD& t) {
+    trav_boxes(sv, t, t.h);
+    t.pmask = t.h.leaf_mask;
+    trav_descend_any(st, t, t.h);
+}
+// Tests the parked leaves in slot order.
+GPR_D void travd_leaves(const SceneView& sv, TravD& t) {
+    while (t.pmask != 0) {
+        const int32_t leaf = lowest_child(t.h, t.pmask);
+        t.pmask &= t.pmask - 1;
+        tri_rec_hit(sv.tris, sv.ntri, ~leaf, t.r, t.tmax, t.hit, t.found);
+        if (t.found) t.pmask = 0;
+    }
 }
 
 // Closest hit (ANY=false) or any hit (ANY=true) against the BVH4.  Returns
@@ -445,10 +427,10 @@ GPR_D bool travd_leaves(const SceneView& sv, TravD& t) {
 template <bool ANY, class Stack>
 GPR_D bool fast_trace(const SceneView& sv, const Ray3& r, Stack& st, gpr_hit& hit) {
     Trav t;
-    int rc = trav_begin<ANY>(sv, r, st, t) ? kTravDone : kTravMore;
-    while (rc == kTravMore) rc = trav_step<ANY>(sv, st, t);
+    trav_begin<ANY>(sv, r, st, t);
+    while (trav_live(sv, t)) trav_step<ANY>(sv, st, t);
     hit = t.hit;
-    return rc != kTravOverflow;
+    return t.node == kTravDone;
 }
 
 }  // namespace gpr
