@@ -1,8 +1,8 @@
 // engine.h -- multi-job wavefront engine shared by the batched and served
-// forms.  One pass renders one sample of every job it holds: the jobs' paths
-// are concatenated in the ray queues (each entry carries its job id), scenes
-// live in one device arena, and the pass is a fixed launch sequence replayed
-// from a hipGraph.  In PCG mode a job's image does not depend on which other
+// forms.  One pass renders the next 2^log_s samples of every job it holds: the
+// jobs' paths are concatenated in the ray queues (each entry carries its job
+// id), scenes live in one device arena, and the pass is a fixed launch sequence
+// replayed from a hipGraph.  In PCG mode a job's image does not depend on which other
 // jobs share its passes: every path keeps its own RNG stream (job seed,
 // sample, pixel) and each pixel receives its terms in the same kernel order as
 // in the single-scene renderer.
@@ -22,10 +22,10 @@ struct EngineJob {
     uint32_t npix;       // width * height
     uint32_t width;
     uint32_t fb_off;     // first frame-buffer pixel of the job in the pool
-    uint32_t sample;     // sample index this pass renders (0 clears the job's pixels first)
+    uint32_t sample;     // first sample index this pass renders (0 clears the job's pixels first)
     uint32_t max_depth;
     uint32_t rr_start;
-    uint32_t pad;
+    uint32_t log_s;      // log2 of the samples it renders
     unsigned long long seed;
     float r2c[16];
     float c2w[16];
@@ -48,7 +48,16 @@ void engine_destroy(Engine* e);
 size_t engine_device_bytes(const Engine* e);
 // Scene table: device views into scene memory owned by the caller.
 int engine_set_scenes(Engine* e, const std::vector<SceneView>& views, hipStream_t st);
-// Stage the jobs (sum of npix <= capacity) and enqueue one pass on st.  fb is
+// Term lists of passes of more than one sample a job.  They grow on use, up to
+// the limit (0 bytes: never); engine_reserve_terms allocates them at once
+// instead.
+void engine_limit_terms(Engine* e, uint64_t bytes);
+int engine_reserve_terms(Engine* e, uint64_t bytes);
+// Gives every job as many samples as the pass has room for: jobs hold one
+// sample each (log_s 0) on entry, left[k] is how many job k has left (>= 1).
+// st is the stream of the passes.
+int engine_fill_pass(Engine* e, std::vector<EngineJob>& jobs, const std::vector<uint32_t>& left, hipStream_t st);
+// Stage the jobs (sum of npix << log_s <= capacity) and enqueue one pass on st.  fb is
 // the frame-buffer pool the jobs' fb_off index.
 int engine_run_pass(Engine* e, const EngineJob* jobs, uint32_t njobs, float4* fb, const TraceCfg& cfg,
                     hipStream_t st);

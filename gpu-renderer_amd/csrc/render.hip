@@ -72,12 +72,14 @@ struct Ctrl {
 struct PassJob {
     EngineJob j;
     uint32_t path_off;  // first path of the job in the pass
-    uint32_t pad[3];
+    uint32_t pix_off;   // its first pixel among the pass's pixels
+    uint32_t pad[2];
 };
 struct PassBuf {
     uint32_t npaths;
     uint32_t njobs;
-    uint32_t pad[62];
+    uint32_t npixels;
+    uint32_t pad[61];
     PassJob jobs[kMaxPassJobs];
 };
 
@@ -217,10 +219,17 @@ __global__ __launch_bounds__(256) void k_gen(RenderArgs a) {
             else hi = mid;
         }
         const EngineJob& jb = pb->jobs[lo].j;
-        const uint32_t lp = tid - pb->jobs[lo].path_off;
-        const uint32_t fbi = jb.fb_off + lp;
-        if (jb.sample == 0) a.fb[fbi] = make_float4(0.f, 0.f, 0.f, 0.f);
-        const uint64_t inc = pcg_inc(jb.sample, lp);
+        const uint32_t off = pb->jobs[lo].path_off;
+        const uint32_t lp = slot_pixel((tid - off) >> jb.log_s, jb.width, jb.npix);
+        const uint32_t sub = (tid - off) & ((1u << jb.log_s) - 1u);
+        uint32_t word = jb.fb_off + lp;
+        if (a.terms) {
+            word = off + (lp << jb.log_s | sub);
+            a.nterm[word] = 0;
+        } else if (jb.sample == 0) {
+            a.fb[word] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        const uint64_t inc = pcg_inc(jb.sample + sub, lp);
         uint64_t st = pcg_init(jb.seed, inc);
         const float jx = pcg_unit(st, inc);
         const float jy = pcg_unit(st, inc);
@@ -230,7 +239,7 @@ __global__ __launch_bounds__(256) void k_gen(RenderArgs a) {
         q.o_tmin[tid] = make_float4(o.x, o.y, o.z, 0.f);
         q.d_tmax[tid] = make_float4(d.x, d.y, d.z, 1e34f);
         q.w_pdf[tid] = make_float4(1.f, 1.f, 1.f, 0.f);
-        q.pix[tid] = fbi;
+        q.pix[tid] = word;
         q.job[tid] = (jb.scene << kJobBits) | lo;
     } else {
         const uint32_t W = a.sv.width;
@@ -563,8 +572,13 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
             // a job's paths stop at its own depth
             valid = bounce < pj.j.max_depth;
             rr_start = pj.j.rr_start;
+            const uint32_t word = qi.pix[i] & 0x7fffffffu;
+            lpix = word - pj.j.fb_off;
             sample = pj.j.sample;
-            lpix = (qi.pix[i] & 0x7fffffffu) - pj.j.fb_off;
+            if (a.terms) {
+                lpix = (word - pj.path_off) >> pj.j.log_s;
+                sample += (word - pj.path_off) & ((1u << pj.j.log_s) - 1u);
+            }
         }
     } else {
         sv = a.sv;
@@ -774,11 +788,31 @@ __global__ void k_finish(Ctrl* c, uint32_t samples) {
 
 // Adds the terms of a multi-sample pass to their pixels, in sample order and
 // within a sample in the order the path met them.
+template <bool MULTI>
 __global__ __launch_bounds__(256) void k_accum(RenderArgs a) {
     const uint32_t p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= (a.npix >> a.log_s)) return;
-    float4 x = a.fb[p];
-    for (uint32_t j = p << a.log_s; j < (p + 1) << a.log_s; ++j) {
+    uint32_t log_s = a.log_s, path = p << a.log_s, fbi = p;
+    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (MULTI) {
+        const PassBuf* pb = a.pass;
+        if (p >= pb->npixels) return;
+        uint32_t lo = 0, hi = pb->njobs;  // the job holding pixel p: last job whose pix_off <= p
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (pb->jobs[mid].pix_off <= p) lo = mid;
+            else hi = mid;
+        }
+        const EngineJob& jb = pb->jobs[lo].j;
+        const uint32_t lp = p - pb->jobs[lo].pix_off;
+        log_s = jb.log_s;
+        path = pb->jobs[lo].path_off + (lp << log_s);
+        fbi = jb.fb_off + lp;
+        if (jb.sample != 0) x = a.fb[fbi];
+    } else {
+        if (p >= (a.npix >> log_s)) return;
+        x = a.fb[fbi];
+    }
+    for (uint32_t j = path; j < path + (1u << log_s); ++j) {
         const uint32_t n = a.nterm[j];
         for (uint32_t k = 0; k < n; ++k) {
             const float4 v = a.terms[(uint64_t)k * a.tstride + j];
@@ -787,7 +821,7 @@ __global__ __launch_bounds__(256) void k_accum(RenderArgs a) {
             x.z = x.z + v.z;
         }
     }
-    a.fb[p] = x;
+    a.fb[fbi] = x;
 }
 
 __global__ void k_clear_fb(float4* fb, uint32_t n) {
@@ -805,6 +839,22 @@ __global__ void k_set_sample(Ctrl* c, uint32_t s) {
 inline uint32_t div_up(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
 }  // namespace
+
+// Multi-sample passes.  A small image (or the
+// late bounces of any image) leaves the chip idle and every launch pays the
+// latency of its longest ray, so a pass renders up to 2^kMaxLogS samples at
+// once.  Paths are pixel-major: the samples of a pixel sit in neighbouring
+// lanes, which keeps waves coherent.  16 samples of the 256x256 Cornell box
+// take 2.4 ms in one pass against 6.4 ms in 16; 4 samples of the 1920x1080
+// sphere grid 17.0 ms against 25.9, and passes of 2^20 / 2^21 / 2^22 / 2^23 /
+// 2^24 paths render 8 samples of an 803x451 textured scene in 12.7 / 7.8 / 5.7
+// / 5.7 / 5.7 ms and 4 of the sphere grid in 26.5 / 26.5 / 20.1 / 17.6 / 17.3.
+// The multi-job engine's passes do the same per job: a batch of 12 scenes at
+// 128^2 to 512^2, 16 samples, takes 69 ms instead of 92, a burst of 16 requests
+// of 4 to 64 samples to the server 231 instead of 430.
+constexpr uint32_t kMaxLogS = 6;
+constexpr uint64_t kPassPaths = 1ull << 23;   // paths of a multi-sample pass at most
+constexpr uint64_t kPassBytes = 6ull << 30;   // its queues and term lists at most
 
 // ---------------------------------------------------------- engine ----
 // Kernel set of one traversal configuration of the multi-job pass.
@@ -882,6 +932,8 @@ struct Engine {
     int device = 0;
     uint32_t capacity = 0, max_jobs = 0, ntiles = 0;
     DevBuf qmem[3], ctrl, status, spill, pass, scenes;
+    DevBuf terms, nterm;      // passes of several samples a job
+    uint64_t term_limit = 0;  // bytes the term lists may take
     QueueView q[3];
     int grid[kPassKernelCount] = {};
     hipStream_t cap_stream = nullptr;
@@ -895,8 +947,10 @@ struct Engine {
         uint32_t chunk;
         uint32_t size;  // launch size class: paths rounded up to a power of two
         float4* fb;
+        bool terms;     // several samples a job
         bool operator==(const GraphKey& o) const {
-            return depth == o.depth && kidx == o.kidx && chunk == o.chunk && size == o.size && fb == o.fb;
+            return depth == o.depth && kidx == o.kidx && chunk == o.chunk && size == o.size && fb == o.fb &&
+                   terms == o.terms;
         }
     };
     std::vector<std::pair<GraphKey, hipGraphExec_t>> graphs;
@@ -972,7 +1026,8 @@ int engine_set_scenes(Engine* e, const std::vector<SceneView>& views, hipStream_
 namespace {
 // Launch grids cover `size` paths (the pass's size class), not the capacity:
 // a small pass launches small grids.
-int record_pass(Engine* e, uint32_t depth, int kidx, uint32_t chunk, uint32_t size, float4* fb, hipStream_t st) {
+int record_pass(Engine* e, uint32_t depth, int kidx, uint32_t chunk, uint32_t size, float4* fb, bool terms,
+                hipStream_t st) {
     RenderArgs a{};
     a.scenes = e->scenes.as<SceneView>();
     a.pass = e->pass.as<PassBuf>();
@@ -985,6 +1040,11 @@ int record_pass(Engine* e, uint32_t depth, int kidx, uint32_t chunk, uint32_t si
     a.depth = depth;
     a.chunk = chunk;
     a.rng_mode = GPR_RNG_PCG;
+    if (terms) {
+        a.terms = e->terms.as<float4>();
+        a.nterm = e->nterm.as<uint8_t>();
+        a.tstride = size;
+    }
     const PassKernels& pk = pass_kernel_table(kidx);
     const dim3 tg(std::min<uint32_t>(e->grid[kidx], div_up(size, pk.nt))), tb(pk.nt);
     hipLaunchKernelGGL(k_gen<true>, dim3(div_up(size, 256)), dim3(256), 0, st, a);
@@ -994,8 +1054,18 @@ int record_pass(Engine* e, uint32_t depth, int kidx, uint32_t chunk, uint32_t si
         hipLaunchKernelGGL(pk.shadow, tg, tb, 0, st, a, b);
         hipLaunchKernelGGL(pk.ext_scatter, tg, tb, 0, st, a, b);
     }
+    if (terms) hipLaunchKernelGGL(k_accum<true>, dim3(div_up(size, 256)), dim3(256), 0, st, a);
     GPR_HIP(hipGetLastError());
     return GPR_OK;
+}
+}  // namespace
+
+namespace {
+// Launch size class of a pass: its paths rounded up to a power of two.
+uint32_t size_class(const Engine* e, uint64_t paths) {
+    uint64_t size = 1u << 16;
+    while (size < paths) size <<= 1;
+    return (uint32_t)std::min<uint64_t>(size, e->capacity);
 }
 }  // namespace
 
@@ -1010,35 +1080,40 @@ int engine_run_pass(Engine* e, const EngineJob* jobs, uint32_t njobs, float4* fb
     e->slot = (s + 1) % Engine::kStage;
     GPR_HIP(hipEventSynchronize(e->ev[s]));  // the staging slot's previous upload is done
     PassBuf* h = e->h_pass[s];
-    uint64_t off = 0;
+    uint64_t off = 0, pixels = 0;
     uint32_t depth = 0;
+    bool terms = false;
     for (uint32_t k = 0; k < njobs; ++k) {
         const EngineJob& j = jobs[k];
-        if (j.npix == 0 || j.width == 0 || j.max_depth > kMaxBounce)
+        if (j.npix == 0 || j.width == 0 || j.max_depth > kMaxBounce || j.log_s > kMaxLogS)
             return fail(GPR_ERR_INVALID, "engine: malformed job");
         h->jobs[k].j = j;
         h->jobs[k].path_off = (uint32_t)off;
-        off += j.npix;
+        h->jobs[k].pix_off = (uint32_t)pixels;
+        off += (uint64_t)j.npix << j.log_s;
+        pixels += j.npix;
+        terms = terms || j.log_s > 0;
         depth = std::max(depth, j.max_depth);
     }
     if (off > e->capacity) return fail(GPR_ERR_INVALID, "engine: pass exceeds the queue capacity");
     h->npaths = (uint32_t)off;
+    h->npixels = (uint32_t)pixels;
     h->njobs = njobs;
+    const uint32_t size = size_class(e, off);
+    if (depth == 0) depth = 1;
+    if (terms && (16ull * size * max_terms(depth) > e->terms.bytes || size > e->nterm.bytes))
+        return fail(GPR_ERR_INVALID, "engine: pass exceeds its term lists");
     const size_t bytes = offsetof(PassBuf, jobs) + sizeof(PassJob) * njobs;
     GPR_HIP(hipMemcpyAsync(e->pass.p, h, bytes, hipMemcpyHostToDevice, st));
     GPR_HIP(hipEventRecord(e->ev[s], st));
-    if (depth == 0) depth = 1;
-    uint32_t size = 1u << 16;
-    while (size < off) size <<= 1;
-    size = std::min(size, e->capacity);
-    const Engine::GraphKey key{depth, kidx, (uint32_t)cfg.chunk, size, fb};
+    const Engine::GraphKey key{depth, kidx, (uint32_t)cfg.chunk, size, fb, terms};
     hipGraphExec_t exec = nullptr;
     for (auto& g : e->graphs)
         if (g.first == key) exec = g.second;
     if (!exec) {
         hipGraph_t graph;
         GPR_HIP(hipStreamBeginCapture(e->cap_stream, hipStreamCaptureModeThreadLocal));
-        const int rc = record_pass(e, depth, kidx, (uint32_t)cfg.chunk, size, fb, e->cap_stream);
+        const int rc = record_pass(e, depth, kidx, (uint32_t)cfg.chunk, size, fb, terms, e->cap_stream);
         const hipError_t ec = hipStreamEndCapture(e->cap_stream, &graph);
         GPR_TRY(rc);
         if (ec != hipSuccess) return fail(GPR_ERR_HIP, std::string("pass capture: ") + hipGetErrorString(ec));
@@ -1048,6 +1123,74 @@ int engine_run_pass(Engine* e, const EngineJob* jobs, uint32_t njobs, float4* fb
         e->graphs.push_back({key, exec});
     }
     GPR_HIP(hipGraphLaunch(exec, st));
+    return GPR_OK;
+}
+
+void engine_limit_terms(Engine* e, uint64_t bytes) { e->term_limit = bytes; }
+
+int engine_reserve_terms(Engine* e, uint64_t bytes) {
+    const uint64_t paths = std::min<uint64_t>(e->capacity, kPassPaths);  // one term count (a byte) each
+    if (bytes <= 64 * paths) return GPR_OK;
+    if (e->nterm.alloc(paths) != GPR_OK || e->terms.alloc(bytes - paths) != GPR_OK) {
+        (void)hipGetLastError();  // the failed allocation
+        e->nterm.release();
+        return GPR_ERR_OOM;
+    }
+    e->term_limit = bytes - paths;
+    return GPR_OK;
+}
+
+namespace {
+// Term lists for a pass of `size` paths; false (and none larger from then on)
+// where the device has no room for them.
+int grow_terms(Engine* e, uint32_t size, uint32_t depth, hipStream_t st, bool* ok) {
+    const uint64_t need = 16ull * size * max_terms(depth);
+    *ok = true;
+    if (need <= e->terms.bytes && size <= e->nterm.bytes) return GPR_OK;
+    GPR_HIP(hipStreamSynchronize(st));  // passes in flight use the old lists
+    for (size_t g = e->graphs.size(); g-- > 0;)
+        if (e->graphs[g].first.terms) {
+            (void)hipGraphExecDestroy(e->graphs[g].second);
+            e->graphs.erase(e->graphs.begin() + g);
+        }
+    if (e->terms.alloc(need) != GPR_OK || e->nterm.alloc(size) != GPR_OK) {
+        (void)hipGetLastError();
+        e->terms.release();
+        e->nterm.release();
+        e->term_limit = 0;
+        *ok = false;
+    }
+    return GPR_OK;
+}
+}  // namespace
+
+int engine_fill_pass(Engine* e, std::vector<EngineJob>& jobs, const std::vector<uint32_t>& left, hipStream_t st) {
+    uint32_t depth = 1;
+    for (const EngineJob& j : jobs) depth = std::max(depth, j.max_depth);
+    const uint64_t most = std::min<uint64_t>(e->capacity, kPassPaths);
+    // the same power of two for every job that has as many samples left
+    const auto samples = [&](size_t i, uint32_t k) {
+        uint32_t s = 0;
+        while (s < k && (2u << s) <= left[i]) ++s;
+        return s;
+    };
+    uint32_t best = 0, size = 0;
+    for (uint32_t k = 1; k <= kMaxLogS; ++k) {
+        uint64_t paths = 0;
+        bool any = false;
+        for (size_t i = 0; i < jobs.size(); ++i) {
+            const uint32_t s = samples(i, k);
+            any = any || s == k;
+            paths += (uint64_t)jobs[i].npix << s;
+        }
+        if (!any || paths > most || 16ull * size_class(e, paths) * max_terms(depth) > e->term_limit) break;
+        best = k;
+        size = size_class(e, paths);
+    }
+    if (best == 0) return GPR_OK;
+    bool ok = false;
+    GPR_TRY(grow_terms(e, size, depth, st, &ok));
+    for (size_t i = 0; ok && i < jobs.size(); ++i) jobs[i].log_s = samples(i, best);
     return GPR_OK;
 }
 
@@ -1104,19 +1247,6 @@ int pack_shade(gpr_scene* s) {
 }  // namespace gpr
 
 using namespace gpr;
-
-// Multi-sample passes of the single-scene renderer.  A small image (or the
-// late bounces of any image) leaves the chip idle and every launch pays the
-// latency of its longest ray, so a pass renders up to 2^kMaxLogS samples at
-// once.  Paths are pixel-major: the samples of a pixel sit in neighbouring
-// lanes, which keeps waves coherent.  16 samples of the 256x256 Cornell box
-// take 2.4 ms in one pass against 6.4 ms in 16; 4 samples of the 1920x1080
-// sphere grid 17.0 ms against 25.9, and passes of 2^20 / 2^21 / 2^22 / 2^23 /
-// 2^24 paths render 8 samples of an 803x451 textured scene in 12.7 / 7.8 / 5.7
-// / 5.7 / 5.7 ms and 4 of the sphere grid in 26.5 / 26.5 / 20.1 / 17.6 / 17.3.
-constexpr uint32_t kMaxLogS = 6;
-constexpr uint64_t kPassPaths = 1ull << 23;   // paths of a multi-sample pass at most
-constexpr uint64_t kPassBytes = 6ull << 30;   // its queues and term lists at most
 
 // Buffers of multi-sample passes, shared by the renderers of one (device,
 // stream): gpr_render holds the lock until its passes have completed, so one
@@ -1231,7 +1361,7 @@ int launch_pass(gpr_renderer* r, uint32_t log_s, hipStream_t st) {
             hipLaunchKernelGGL((k_extend<false, false, false, NT, SL>), tg, tb, 0, st, a, b);
         }
     }
-    if (log_s) hipLaunchKernelGGL(k_accum, dim3(div_up(r->npix, 256)), dim3(256), 0, st, a);
+    if (log_s) hipLaunchKernelGGL(k_accum<false>, dim3(div_up(r->npix, 256)), dim3(256), 0, st, a);
     hipLaunchKernelGGL(k_finish, dim3(1), dim3(64), 0, st, a.ctrl, 1u << log_s);
     GPR_HIP(hipGetLastError());
     return GPR_OK;

@@ -99,6 +99,13 @@ int arena_add(Arena& A, const gpr_scene* s, hipStream_t st, uint32_t* id) {
     return GPR_OK;
 }
 
+// What a launch counts as in the statistics' passes of one sample a job.
+uint32_t pass_samples(const std::vector<EngineJob>& pass) {
+    uint32_t k = 0;
+    for (const EngineJob& j : pass) k = std::max(k, j.log_s);
+    return 1u << k;
+}
+
 int make_engine_job(const gpr_job& j, const std::vector<SceneView>& views, uint32_t capacity, EngineJob* out) {
     if (j.scene >= views.size()) return fail(GPR_ERR_INVALID, "job: unknown scene id");
     const uint64_t npix = (uint64_t)j.width * j.height;
@@ -202,20 +209,30 @@ int batch_prepare(gpr_batch* b) {
     return GPR_OK;
 }
 
+// Device bytes a batch's term lists may grow to (passes of several samples a
+// job, at most 2^23 paths: 2.3 GB at depth 8).
+constexpr uint64_t kBatchTermBytes = 4ull << 30;
+
 // Pack the next pass: jobs in order, each with samples left, while the
-// capacity holds.  Returns the number of jobs packed.
-uint32_t batch_pack(gpr_batch* b, std::vector<uint32_t>& issued, std::vector<EngineJob>& pass) {
+// capacity holds; with `fill`, as many samples of each as there is room for.
+int batch_pack(gpr_batch* b, std::vector<uint32_t>& issued, std::vector<EngineJob>& pass, bool fill) {
     pass.clear();
+    std::vector<uint32_t> left;
+    std::vector<size_t> which;
     uint64_t used = 0;
     for (size_t k = 0; k < b->jobs.size() && pass.size() < b->opts.max_jobs; ++k) {
         if (issued[k] >= b->spp[k]) continue;
         if (used + b->jobs[k].npix > b->opts.capacity) continue;
         EngineJob j = b->jobs[k];
-        j.sample = issued[k]++;
+        j.sample = issued[k];
         used += j.npix;
         pass.push_back(j);
+        left.push_back(b->spp[k] - issued[k]);
+        which.push_back(k);
     }
-    return (uint32_t)pass.size();
+    if (fill) GPR_TRY(engine_fill_pass(b->eng, pass, left, stream()));
+    for (size_t i = 0; i < pass.size(); ++i) issued[which[i]] += 1u << pass[i].log_s;
+    return GPR_OK;
 }
 }  // namespace
 
@@ -237,6 +254,7 @@ int gpr_batch_create(const gpr_batch_opts* o, gpr_batch** out) {
     GPR_HIP(hipSetDevice(b->device));
     GPR_TRY(b->arena.mem.alloc(std::max<uint64_t>(o->arena_bytes, 256)));
     GPR_TRY(engine_create(b->device, o->capacity, o->max_jobs, &b->eng));
+    engine_limit_terms(b->eng, kBatchTermBytes);
     *out = b.release();
     return GPR_OK;
 }
@@ -275,7 +293,7 @@ int gpr_batch_tune(gpr_batch* b, gpr_trace_cfg* out, uint32_t cap, uint32_t* n) 
     // real pass clears its pixels again, so the probes leave no trace)
     std::vector<uint32_t> issued(b->jobs.size(), 0);
     std::vector<EngineJob> pass;
-    batch_pack(b, issued, pass);
+    GPR_TRY(batch_pack(b, issued, pass, false));
     std::vector<gpr_trace_cfg> res;
     GPR_TRY(tune_engine(b->eng, pass, b->fb.as<float4>(), stream(), res));
     b->cfg = to_cfg(res[0]);
@@ -294,10 +312,12 @@ int gpr_batch_run(gpr_batch* b) {
     std::vector<uint32_t> issued(b->jobs.size(), 0);
     std::vector<EngineJob> pass;
     uint64_t passes = 0, paths = 0;
-    while (batch_pack(b, issued, pass) > 0) {
+    while (true) {
+        GPR_TRY(batch_pack(b, issued, pass, true));
+        if (pass.empty()) break;
         GPR_TRY(engine_run_pass(b->eng, pass.data(), (uint32_t)pass.size(), b->fb.as<float4>(), b->cfg, st));
-        ++passes;
-        for (auto& j : pass) paths += j.npix;
+        passes += pass_samples(pass);
+        for (auto& j : pass) paths += (uint64_t)j.npix << j.log_s;
     }
     uint32_t err = 0;
     GPR_TRY(engine_errors(b->eng, st, &err));
@@ -424,6 +444,9 @@ struct gpr_server {
 };
 
 namespace {
+// Device bytes a server sets aside for term lists at most (2^23 paths of depth 8).
+constexpr uint64_t kServerTermBytes = 2400ull << 20;
+
 struct Finishing {
     hipEvent_t ev;
     std::vector<Request*> reqs;
@@ -510,6 +533,8 @@ void server_loop(gpr_server* s) {
     std::vector<EngineJob> pass;
     std::vector<Request*> pass_reqs;
     std::vector<Request*> retire;
+    std::vector<uint32_t> left;
+    int fill_rc = GPR_OK;
     while (true) {
         TraceCfg cfg;
         {
@@ -541,19 +566,28 @@ void server_loop(gpr_server* s) {
                     retire.push_back(r);
                 }
             s->cancel_req = false;
-            // pack: active requests in admission order, one sample each
+            // pack: active requests in admission order, one sample each, more
+            // where the pass has room
             pass.clear();
             pass_reqs.clear();
+            left.clear();
             uint64_t used = 0;
             for (Request* r : s->active) {
                 if (r->issued >= r->job.spp || used + r->ej.npix > s->opts.capacity) continue;
                 EngineJob j = r->ej;
-                j.sample = r->issued++;
+                j.sample = r->issued;
                 used += j.npix;
                 pass.push_back(j);
                 pass_reqs.push_back(r);
+                left.push_back(r->job.spp - r->issued);
             }
+            fill_rc = engine_fill_pass(s->eng, pass, left, s->st);
+            for (size_t k = 0; k < pass.size(); ++k) pass_reqs[k]->issued += 1u << pass[k].log_s;
             s->in_pass = !pass.empty();
+        }
+        if (fill_rc != GPR_OK) {
+            loop_fail(s, "server: pass packing failed: " + std::string(gpr_last_error()));
+            return;
         }
         if (!pass.empty()) {
             const int prc = engine_run_pass(s->eng, pass.data(), (uint32_t)pass.size(), s->fb.as<float4>(), cfg, s->st);
@@ -571,8 +605,8 @@ void server_loop(gpr_server* s) {
                 if (r->issued == r->job.spp) f.reqs.push_back(r);
             {
                 std::lock_guard<std::mutex> g(s->mu);
-                s->passes++;
-                s->jobs_in_passes += pass.size();
+                s->passes += pass_samples(pass);
+                for (const EngineJob& j : pass) s->jobs_in_passes += 1u << j.log_s;
             }
             if (!f.reqs.empty()) {
                 if (hipEventCreateWithFlags(&f.ev, hipEventDisableTiming) != hipSuccess ||
@@ -623,7 +657,15 @@ int gpr_server_create(const gpr_server_opts* o, gpr_server** out) {
     const uint64_t fixed = o->arena_bytes + engine_device_bytes(s->eng);
     if (o->hbm_budget <= fixed + 16ull * o->capacity)
         return fail(GPR_ERR_BUDGET, "gpr_server_create: budget below arena + queues + one full frame buffer");
-    const uint64_t fb_pixels = std::min<uint64_t>((o->hbm_budget - fixed) / 16, (1ull << 31) - 1);
+    // Of what the budget leaves beyond four full passes of frame buffers, the
+    // term lists of passes of several samples a job come first.
+    uint64_t rest = o->hbm_budget - fixed;
+    const uint64_t frames = 64ull * o->capacity;
+    if (rest > frames) {
+        const uint64_t terms = std::min(rest - frames, kServerTermBytes);
+        if (engine_reserve_terms(s->eng, terms) == GPR_OK) rest -= terms;
+    }
+    const uint64_t fb_pixels = std::min<uint64_t>(rest / 16, (1ull << 31) - 1);
     GPR_TRY(s->arena.mem.alloc(std::max<uint64_t>(o->arena_bytes, 256)));
     GPR_TRY(s->fb.alloc(16 * fb_pixels));
     s->pool.init(fb_pixels);

@@ -385,8 +385,9 @@ int gpr_renderer_free(gpr_renderer* r);
 /* ------------------------------------------------- batched and served --- */
 /* Both forms render many jobs (scene, camera, resolution, spp) through one
  * multi-job wavefront: scenes are copied into one device arena, every pass
- * renders the next sample of each job it holds with all their paths in shared
- * ray queues, and the pass is replayed from a hipGraph.  They run in PCG mode
+ * renders the next sample of each job it holds (the next few, where few jobs
+ * leave room) with all their paths in shared ray queues, and the pass is
+ * replayed from a hipGraph.  They run in PCG mode
  * with BVH4 traversal, and a job's image is bit-identical to the single-scene
  * renderer's (gpr_renderer_create with GPR_RNG_PCG, GPR_TRAVERSAL_FAST, the
  * same seed / depth / roulette start, the same camera) whatever other jobs it
@@ -426,7 +427,7 @@ int gpr_batch_run(gpr_batch* b);
 /* Linear radiance sum of a job (width*height*3 floats) after gpr_batch_run. */
 int gpr_batch_read(gpr_batch* b, uint32_t job, float* rgb_sum);
 typedef struct {
-    uint64_t passes;
+    uint64_t passes;    /* of one sample a job: a launch with room for 2^k samples of its jobs counts as 2^k */
     uint64_t paths;     /* camera paths rendered */
     double ms;          /* wall time of the last gpr_batch_run */
 } gpr_batch_stats;
@@ -466,7 +467,7 @@ int gpr_server_tune(gpr_server* s, const gpr_job* jobs, uint32_t njobs, gpr_trac
 int gpr_server_set_cfg(gpr_server* s, const gpr_trace_cfg* cfg);
 typedef struct {
     uint64_t submitted, completed;
-    uint64_t passes;
+    uint64_t passes;       /* as gpr_batch_stats.passes */
     double renders_per_s;  /* completed / (last completion - first submit) */
     double p50_ms, p99_ms; /* latency percentiles of the completed requests */
     double mean_jobs_per_pass;

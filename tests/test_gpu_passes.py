@@ -89,3 +89,30 @@ def test_options_and_camera_change_between_passes():
         want = by_ones(s, 10, max_depth=depth, seed=3, rng_mode=mode)[0][0]
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (depth, mode)
     r.free()
+
+
+@pytest.mark.parametrize("capacity", [1500, 5000, 1 << 16, 1 << 20])
+def test_jobs_with_uneven_samples(capacity):
+    # jobs run out of samples at different passes; the capacity decides how many samples a pass holds
+    s = scene("spheres", 8, 8)
+    specs = [(37, 40, 1, 5), (9, 8, 64, 64), (33, 17, 5, 2), (1, 1, 130, 3), (20, 20, 16, 8)]
+    cams = [gpr.lookat((0, 0, 0), (1.0 + k, 6, 9)) for k in range(len(specs))]
+    b = gpr.Batch(gpr.arena_bytes(s), capacity=capacity, max_jobs=8)
+    srv = gpr.Server(gpr.arena_bytes(s) + (1 << 30), gpr.arena_bytes(s), capacity=capacity, max_jobs=8)
+    ib, isv = b.add_scene(s), srv.add_scene(s)
+    jobs = [(w, h, spp, c, 40, d, 3, 21 + w) for (w, h, spp, d), c in zip(specs, cams)]
+    for j in jobs:
+        b.add_job(gpr.job(ib, *j))
+    b.run()
+    tickets = [srv.submit(gpr.job(isv, *j)) for j in jobs]
+    served = [srv.wait(t)[0] for t in tickets]
+    for k, ((w, h, spp, d), c) in enumerate(zip(specs, cams)):
+        s.set_camera(c, 40, w, h)
+        want = by_ones(s, spp, max_depth=d, rr_start=3, seed=21 + w)[0][0]
+        assert np.array_equal(b.read(k).view(np.uint32), want.view(np.uint32)), k
+        assert np.array_equal(served[k].view(np.uint32), want.view(np.uint32)), k
+    b.run()  # again from the first sample
+    assert np.array_equal(b.read(0).view(np.uint32), served[0].view(np.uint32))
+    assert b.stats().paths == sum(w * h * spp for w, h, spp, _ in specs)
+    b.free()
+    srv.free()
