@@ -328,23 +328,6 @@ GPR_D float power_heur(float a, float b) {
     return a / (a + b);
 }
 
-// Claim `chunk` consecutive queue entries per wave from a cursor; calls
-// f(i) for every claimed entry below n.
-template <class F>
-GPR_D void for_each_claimed(uint32_t* cursor, uint32_t n, uint32_t chunk, F&& f) {
-    const int lane = threadIdx.x & 63;
-    while (true) {
-        uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(cursor, chunk);
-        base = __shfl(base, 0, 64);
-        if (base >= n) break;
-        for (uint32_t k = 0; k < chunk; k += 64) {
-            const uint32_t i = base + k + lane;
-            if (i < n) f(i);
-        }
-    }
-}
-
 // Per-lane ray refill over queue entries: a lane whose ray is done takes the
 // next entry from a wave-local pool of `chunk` entries (one atomic per chunk).
 // begin(i) sets entry i up and returns true if it finished at once; step()
@@ -481,7 +464,7 @@ __global__ __launch_bounds__(NT) void k_extend(RenderArgs a, uint32_t bounce) {
                 return true;
             });
     } else {
-        for_each_claimed(cur, n, a.chunk, [&](uint32_t i) {
+        for_each_claimed<NT, !MULTI>(cur, n, a.chunk, [&](uint32_t i) {
             const SceneView sv = scene_of<MULTI>(a, q, i);
             const Ray3 r = queue_ray(q, i);
             const gpr_hit h = trace_one<false, REF_ORDER>(a, sv, r, st);
@@ -523,7 +506,7 @@ __global__ __launch_bounds__(NT) void k_shadow(RenderArgs a, uint32_t bounce) {
                 return true;
             });
     } else {
-        for_each_claimed(cur, n, a.chunk, [&](uint32_t i) {
+        for_each_claimed<NT, !MULTI>(cur, n, a.chunk, [&](uint32_t i) {
             const SceneView sv = scene_of<MULTI>(a, q, i);
             const gpr_hit h = trace_one<true, REF_ORDER>(a, sv, queue_ray(q, i), st);
             shadow_finish(a, q, i, h);
@@ -1248,12 +1231,14 @@ int pack_shade(gpr_scene* s) {
 
 using namespace gpr;
 
-// Buffers of multi-sample passes, shared by the renderers of one (device,
-// stream): gpr_render holds the lock until its passes have completed, so one
-// call at a time uses them.  Freed with the last renderer that used them.
+// Stack overflow area of the traversals and buffers of multi-sample passes,
+// shared by the renderers of one (device, stream): gpr_render holds the lock
+// until its passes have completed, so one call at a time uses them.  Freed with
+// the last renderer that used them.
 struct PassWork {
     std::mutex mu;
-    DevBuf qmem[3], terms, nterm, status, spill;
+    DevBuf spill;  // kStackGlobal entries per resident lane, allocated once
+    DevBuf qmem[3], terms, nterm, status;
     QueueView q[3];
     uint32_t paths = 0, depth = 0, ntiles = 0;
     uint64_t gen = 0;  // of the buffers; graphs captured with older ones are dropped
@@ -1279,7 +1264,7 @@ struct gpr_renderer {
     gpr_render_opts opts{};
     uint32_t npix = 0, ntiles = 0;
     uint32_t spp_done = 0;
-    DevBuf fb, ctrl, status, spill;
+    DevBuf fb, ctrl, status;
     DevBuf qmem[3];
     DevBuf seeds[2];
     QueueView q[3];
@@ -1322,7 +1307,6 @@ RenderArgs make_args(gpr_renderer* r, uint32_t log_s) {
         const PassWork& w = *r->work;
         for (int k = 0; k < 3; ++k) a.q[k] = w.q[k];
         a.status = w.status.as<unsigned long long>();
-        a.spill = w.spill.as<int2>();
         a.ntiles = w.ntiles;
         a.terms = w.terms.as<float4>();
         a.nterm = w.nterm.as<uint8_t>();
@@ -1330,9 +1314,9 @@ RenderArgs make_args(gpr_renderer* r, uint32_t log_s) {
     } else {
         for (int k = 0; k < 3; ++k) a.q[k] = r->q[k];
         a.status = r->status.as<unsigned long long>();
-        a.spill = r->spill.as<int2>();
         a.ntiles = r->ntiles;
     }
+    a.spill = r->work->spill.as<int2>();
     a.chunk = 64;
     a.rng_mode = r->opts.rng_mode;
     a.rr_start = r->opts.rr_start;
@@ -1340,13 +1324,18 @@ RenderArgs make_args(gpr_renderer* r, uint32_t log_s) {
     return a;
 }
 
-constexpr int kRenderNT = 256, kRenderSL = 8;  // block size and LDS stack entries per lane of the single-scene renderer's traversal
+// Block size and LDS stack entries per lane of the single-scene renderer's
+// traversal.  12 entries keep the LDS of a closest-hit block at 24 KB, six
+// blocks to a CU as its registers allow; 8 / 12 / 16 entries: 8 samples of the
+// textured scene 5.03 / 4.85 / 4.88 ms, 4 of the sphere grid 16.7 / 16.7 / 17.1.
+constexpr int kRenderNT = 256, kRenderSL = 12;
 
 // One pass of 2^log_s samples: gen -> extend(primary) -> max_depth x {shade, shadow, extend} -> accum -> finish.
 int launch_pass(gpr_renderer* r, uint32_t log_s, hipStream_t st) {
     const RenderArgs a = make_args(r, log_s);
     const bool ref = r->opts.traversal == GPR_TRAVERSAL_REF;
-    const dim3 tg(std::min<uint32_t>(r->grid_trace, div_up(a.npix, kRenderNT))), tb(kRenderNT);
+    // the whole grid where the paths are few, too: they are spread thin over it
+    const dim3 tg(std::min<uint32_t>(r->grid_trace, a.npix)), tb(kRenderNT);
     constexpr int NT = kRenderNT, SL = kRenderSL;
     hipLaunchKernelGGL(k_gen<false>, dim3(div_up(a.npix, 256)), dim3(256), 0, st, a);
     if (ref) hipLaunchKernelGGL((k_extend<true, true, false, NT, SL>), tg, tb, 0, st, a, 0u);
@@ -1403,10 +1392,6 @@ int pass_graph(gpr_renderer* r, uint32_t log_s, hipGraphExec_t* out) {
 }  // namespace
 
 namespace {
-size_t spill_bytes(const gpr_renderer* r, uint32_t paths) {
-    return (size_t)std::min<uint32_t>(r->grid_trace, div_up(paths, kRenderNT)) * kRenderNT * kStackGlobal * sizeof(int2);
-}
-
 // Makes the stream's pass buffers hold `paths` paths of r's depth (w.mu held,
 // no pass in flight).
 int grow_work(gpr_renderer* r, PassWork& w, uint32_t paths) {
@@ -1415,22 +1400,19 @@ int grow_work(gpr_renderer* r, PassWork& w, uint32_t paths) {
     // a deeper render after a larger one: not both at once if that breaks the bound
     const bool both = n * path_bytes(depth) <= kPassBytes;
     const uint32_t np = both ? n : paths, nd = both ? depth : r->opts.max_depth;
-    if (w.paths >= paths && w.terms.bytes >= 16ull * paths * max_terms(r->opts.max_depth) &&
-        w.spill.bytes >= spill_bytes(r, paths))
-        return GPR_OK;
+    if (w.paths >= paths && w.terms.bytes >= 16ull * paths * max_terms(r->opts.max_depth)) return GPR_OK;
     w.paths = w.depth = 0;
     {
         std::lock_guard<std::mutex> lk(g_work_mu);
         w.gen = ++g_work_gen;
     }
     // given back first, so that the old and the new buffers never exist together
-    for (DevBuf* b : {&w.qmem[0], &w.qmem[1], &w.qmem[2], &w.terms, &w.nterm, &w.status, &w.spill}) b->release();
+    for (DevBuf* b : {&w.qmem[0], &w.qmem[1], &w.qmem[2], &w.terms, &w.nterm, &w.status}) b->release();
     w.ntiles = div_up(np, kShadeBlock);
     GPR_TRY(w.status.alloc(8ull * kMaxBounce * w.ntiles));
     for (int k = 0; k < 3; ++k) GPR_TRY(alloc_queue(w.qmem[k], w.q[k], np, false));
     GPR_TRY(w.terms.alloc(16ull * np * max_terms(nd)));
     GPR_TRY(w.nterm.alloc(np));
-    GPR_TRY(w.spill.alloc(spill_bytes(r, np)));
     w.paths = np;
     w.depth = nd;
     return GPR_OK;
@@ -1479,7 +1461,6 @@ int renderer_alloc(gpr_renderer* r) {
                                                      kRenderNT, 0) != hipSuccess)
         return fail(GPR_ERR_HIP, "occupancy query failed");
     r->grid_trace = std::max(1, cus * std::max(1, per_cu));
-    GPR_TRY(r->spill.alloc(spill_bytes(r, r->npix)));
     return GPR_OK;
 }
 }  // namespace
@@ -1617,17 +1598,14 @@ int gpr_render(gpr_renderer* r, uint32_t spp) {
     // (pathtracer.cu:177-200).
     if (r->spp_done > 0 && !same_view(r->scene->view(), r->accum)) GPR_TRY(gpr_renderer_reset(r));
     hipStream_t st = stream();
-    uint32_t log_s = 0;
-    std::unique_lock<std::mutex> lk;
-    if (spp > 1 && r->opts.rng_mode == GPR_RNG_PCG) {
-        std::shared_ptr<PassWork> w = pass_work(r->scene->device, st);
-        if (w != r->work) {
-            r->drop_graphs();
-            r->work = std::move(w);
-        }
-        lk = std::unique_lock<std::mutex>(r->work->mu);
-        log_s = plan_passes(r, *r->work, spp);
+    std::shared_ptr<PassWork> w = pass_work(r->scene->device, st);
+    if (w != r->work) {
+        r->drop_graphs();
+        r->work = std::move(w);
     }
+    std::lock_guard<std::mutex> lk(r->work->mu);
+    GPR_TRY(r->work->spill.alloc((size_t)r->grid_trace * kRenderNT * kStackGlobal * sizeof(int2)));
+    uint32_t log_s = spp > 1 ? plan_passes(r, *r->work, spp) : 0;
     for (uint32_t left = spp; left;) {
         while ((1u << log_s) > left) --log_s;
         hipGraphExec_t g = nullptr;

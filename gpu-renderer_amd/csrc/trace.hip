@@ -1,10 +1,10 @@
 // trace.hip -- ray-query kernels behind gpr_trace (trace / trace_shadow,
 // src/renderer/pathtracer_kernel.h:235-246, 310-321).
 //
-// k_trace_fast is persistent: every wave pulls 64 consecutive rays from a
-// global atomic cursor until the batch is drained, so the grid is sized to
-// the device (not to the batch) and the per-lane overflow stacks are indexed
-// by the persistent thread id.
+// The fast kernels are persistent: a wave takes its share of the batch and then
+// claims more from a global atomic cursor until the batch is drained, so the
+// grid is sized to the device (not to the batch) and the per-lane overflow
+// stacks are indexed by the persistent thread id.
 #include <algorithm>
 #include <map>
 #include <memory>
@@ -49,22 +49,11 @@ __global__ __launch_bounds__(NT) void k_trace_fast(SceneView sv, const gpr_ray* 
     Stack st;
     st.lds = lds + threadIdx.x;
     st.spill = reinterpret_cast<typename Stack::Entry*>(spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal);
-    const int lane = threadIdx.x & 63;
-    while (true) {
-        unsigned long long base = 0;
-        if (lane == 0) base = atomicAdd(cursor, (unsigned long long)chunk);
-        base = __shfl(base, 0, 64);
-        if (base >= n) break;
-        for (uint32_t k = 0; k < chunk; k += 64) {
-            const uint64_t i = base + k + lane;
-            if (i < n) {
-                const Ray3 r = load_ray(rays, i);
-                gpr_hit h;
-                if (!fast_trace<ANY>(sv, r, st, h)) atomicAdd(cursor + 1, 1ull);  // stack overflow count
-                store_hit(hits, i, h);
-            }
-        }
-    }
+    for_each_claimed<NT, false>(cursor, n, chunk, [&](uint64_t i) {
+        gpr_hit h;
+        if (!fast_trace<ANY>(sv, load_ray(rays, i), st, h)) atomicAdd(cursor + 1, 1ull);  // stack overflow count
+        store_hit(hits, i, h);
+    });
 }
 
 // Per-lane ray refill: the lanes of a wave step their rays one node at a
@@ -87,8 +76,15 @@ __global__ __launch_bounds__(NT) void k_trace_refill(SceneView sv, const gpr_ray
     st.lds = lds + threadIdx.x;
     st.spill = reinterpret_cast<typename Stack::Entry*>(spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal);
     const int lane = threadIdx.x & 63;
-    uint64_t pb = 0, pe = 0;  // wave-local pool [pb, pe) of ray indices (wave-uniform)
-    bool drained = false;     // the global cursor has passed n (wave-uniform)
+    // wave-local pool [pb, pe) of ray indices (wave-uniform); the first one is
+    // dealt out, thin where the batch is short, the others are claimed
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (NT / 64) + threadIdx.x / 64);
+    const uint32_t waves = gridDim.x * (NT / 64);
+    const uint32_t width = spread_width(n, waves);
+    const uint32_t first = width < 64 ? width : chunk;
+    const uint64_t claimed_from = (uint64_t)waves * first;
+    uint64_t pb = min((uint64_t)wave * first, n), pe = min(pb + first, n);
+    bool drained = claimed_from >= n;  // nothing is left to claim (wave-uniform)
     bool active = false;
     uint64_t ri = 0;
     // any hit walks with postponed leaves (leaf rounds once kLeafRound lanes have parked some)
@@ -104,7 +100,7 @@ __global__ __launch_bounds__(NT) void k_trace_refill(SceneView sv, const gpr_ray
             if (avail < cnt && !drained) {
                 unsigned long long b = 0;
                 if (lane == 0) b = atomicAdd(cursor, (unsigned long long)chunk);
-                b = __shfl(b, 0, 64);
+                b = claimed_from + __shfl(b, 0, 64);
                 nb = b < n ? b : n;
                 ne = b + chunk < n ? b + chunk : n;
                 if (b + chunk >= n) drained = true;
@@ -321,7 +317,7 @@ int launch_trace(const SceneView& sv, const gpr_ray* rays, gpr_hit* hits, uint64
     const TraceVariant& v = trace_variant_at(k);
     unsigned long long* cur = R.cursor.as<unsigned long long>();
     hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, cur, 4);
-    const uint64_t want = (n + v.nt - 1) / v.nt;  // more blocks than rays would only idle
+    const uint64_t want = n;  // a short batch is spread thin: a wave takes one ray at least
     const int kind = (refill ? 2 : 0) + (any ? 1 : 0);
     const TraceKernel ks[4] = {v.closest, v.any, v.closest_r, v.any_r};
     const dim3 grid((unsigned)std::min<uint64_t>(R.grid[k][kind], want));

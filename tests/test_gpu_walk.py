@@ -57,3 +57,21 @@ def test_ranges_behind_the_origin(tmin, tmax):
         h = s.trace(r)
         assert np.array_equal(h["id"], ref["id"]), shape
     s.free()
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 4095, 4097, 8193, 40960, 40961, 131072, 131073, 200001])
+def test_batch_sizes_around_the_spreading_of_short_batches(n):
+    # short batches use thin waves; every ray is traced once whatever the share of a wave
+    pos = gpr.gen_soup(5, 0, 3000, 0.03)
+    s = gpr.Scene.soup(pos).commit()
+    r = gpr.gen_rays(4, 1, n)
+    for any_hit in (False, True):
+        ref = s.trace(r, any_hit=any_hit, ref_order=True)
+        for shape in SHAPES + [(256, 8, 192, 0), (256, 8, 192, 1)]:
+            s.trace_set_cfg(*shape)
+            h = s.trace(r, any_hit=any_hit)
+            if any_hit:
+                assert np.array_equal(h["id"] >= 0, ref["id"] >= 0), shape
+            else:
+                assert np.array_equal(h["id"], ref["id"]), shape
+    s.free()
