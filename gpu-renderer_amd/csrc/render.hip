@@ -11,11 +11,12 @@
 //           MIS contribution (accumulate_BSDF_sampling_contribution) and, in
 //           reference RNG mode, its roulette (pathtracer_kernel.h:684-749)
 //   shade   shade_hit_with_MIS: emission, NEE shadow append, BSDF scatter
-//           append.  Appends are compacted in queue order: a wave ballot and
-//           mbcnt give lane offsets, LDS gives wave offsets, and a decoupled
-//           look-back over tiles (one 64-bit status word per tile, no other
-//           cross-XCD data) gives tile offsets -- so slot order equals the
-//           serial order of the reference's host loop.
+//           append.  Appends are compacted: a wave ballot and mbcnt give lane
+//           offsets, LDS gives wave offsets, and one atomic on the counter of
+//           the block's queue segment gives the block's place.  In reference
+//           RNG mode, where slot order must equal the serial order of the
+//           reference's host loop, a decoupled look-back over tiles (one 64-bit
+//           status word per tile) gives it instead.
 //   shadow  any-hit of the shadow queue + accumulate_light_sampling_contribution
 //
 // Per pixel the frame buffer receives emission, NEE and BSDF terms in the
@@ -41,6 +42,7 @@ namespace {
 
 constexpr int kShadeBlock = 256;
 constexpr uint32_t kMaxBounce = 64;
+constexpr uint32_t kMaxSegs = 4;  // a power of two
 constexpr uint32_t kLastSpread = 16;
 
 // Queue of path vertices / rays (SoA, capacity = paths per sample or pass).
@@ -59,14 +61,37 @@ struct QueueView {
 struct Ctrl {
     uint32_t sample;         // current sample index (single-scene; advanced by k_finish)
     uint32_t error;          // bit0: traversal stack overflow, bit1: look-back timeout
-    uint32_t shadow_size[kMaxBounce];
-    uint32_t scatter_size[kMaxBounce];
     uint32_t tile_counter[kMaxBounce];
     uint32_t ext_cursor[kMaxBounce + 1];  // [0] primary, [b+1] scatter queue of bounce b
     uint32_t sh_cursor[kMaxBounce];
-    // multi-sample passes: (shadow << 32 | scatter) entries of the last sample, spread over counters
-    unsigned long long last[kMaxBounce][kLastSpread];
 };
+
+// Segments of the shadow and scatter queues of an unordered pass: appends take
+// their place from one of several counters (shadow << 32 | scatter) on lines of
+// their own, since returning atomics on one address serialise.  Block b of
+// k_shade appends to segment (b / kSegGroup) % nseg, which holds at most cap
+// entries.  4 samples of the 1920x1080 sphere grid take 13.2 ms with four
+// segments, 14.5 with one, 13.2 with sixteen (15.2 with ordered appends: a
+// ticket, also one address, and a look-back per block).  A segment's slack is
+// memory: with `tight` (the engine, whose queues count against its caller's
+// budget) slack and counters stay below 2 bytes a path.
+struct Segs {
+    uint32_t nseg, cap;
+};
+constexpr uint32_t kSegGroup = 4;
+constexpr uint32_t shade_blocks(uint32_t paths, uint32_t nseg) {
+    return (paths + kShadeBlock - 1) / kShadeBlock + (nseg > 1 ? nseg : 0);  // a segment's last tile may be partial
+}
+Segs segs_for(uint32_t paths, bool tight) {
+    Segs s;
+    s.nseg = paths >= (tight ? 5u << 17 : 1u << 16) ? kMaxSegs : 1u;
+    const uint32_t groups = (shade_blocks(paths, s.nseg) + kSegGroup - 1) / kSegGroup;
+    s.cap = s.nseg == 1 ? paths : (groups + s.nseg - 1) / s.nseg * kSegGroup * kShadeBlock;
+    return s;
+}
+// 64-bit words between two segments' counters, and of all counters
+GPR_HD constexpr uint32_t seg_stride(uint32_t nseg) { return nseg > 1 ? 16u : 1u; }
+constexpr uint32_t seg_words(uint32_t nseg) { return kMaxBounce * nseg * seg_stride(nseg); }
 
 // Jobs of one multi-job pass (device copy of EngineJob[] plus the path offsets).
 struct PassJob {
@@ -94,8 +119,11 @@ struct RenderArgs {
     int2* spill;
     uint32_t npix;             // single-scene: paths per sample
     uint32_t ntiles;           // look-back words per bounce (capacity / kShadeBlock)
+    uint32_t nseg, seg_cap;    // segments of the shadow and scatter queues
+    unsigned long long* seg;   // [bounce][segment] entries appended: shadow << 32 | scatter
+    unsigned long long* last;  // multi-sample passes, [bounce][kLastSpread]: those of the last sample, spread
     uint32_t depth;            // bounces of the sample / pass
-    uint32_t chunk;            // entries a wave claims per atomic in extend / shadow
+    uint32_t chunk_log;        // log2 of the entries a wave takes a turn in extend / shadow
     uint32_t rng_mode;
     uint32_t rr_start;
     unsigned long long seed;
@@ -106,6 +134,9 @@ struct RenderArgs {
     uint32_t log_s;            // single-scene: log2 of the samples of the pass
 };
 
+GPR_D unsigned long long* seg_at(const RenderArgs& a, uint32_t bounce, uint32_t g) {
+    return a.seg + (bounce * a.nseg + g) * seg_stride(a.nseg);
+}
 template <bool MULTI>
 GPR_D uint32_t npaths_of(const RenderArgs& a) {
     if constexpr (MULTI) return a.pass->npaths;
@@ -193,20 +224,21 @@ __global__ __launch_bounds__(256) void k_gen(RenderArgs a) {
     // clear the per-sample counters, cursors and the look-back words this sample uses
     Ctrl* c = a.ctrl;
     for (uint32_t i = tid; i < kMaxBounce; i += gsz) {
-        c->shadow_size[i] = 0u;
-        c->scatter_size[i] = 0u;
         c->tile_counter[i] = 0u;
         c->ext_cursor[i + 1] = 0u;
         c->sh_cursor[i] = 0u;
     }
     if constexpr (!MULTI) {
         if (a.log_s)
-            for (uint32_t i = tid; i < kMaxBounce * kLastSpread; i += gsz) (&c->last[0][0])[i] = 0ull;
+            for (uint32_t i = tid; i < kMaxBounce * kLastSpread; i += gsz) a.last[i] = 0ull;
     }
+    for (uint32_t i = tid; i < kMaxBounce * a.nseg; i += gsz) a.seg[i * seg_stride(a.nseg)] = 0ull;
     if (tid == 0) c->ext_cursor[0] = 0u;
-    const uint32_t used_tiles = (npix + kShadeBlock - 1) / kShadeBlock;
-    const uint64_t nstat = (uint64_t)a.depth * used_tiles;
-    for (uint64_t i = tid; i < nstat; i += gsz) a.status[(i / used_tiles) * a.ntiles + i % used_tiles] = 0ull;
+    if (!MULTI && a.rng_mode == GPR_RNG_REFERENCE) {
+        const uint32_t used_tiles = (npix + kShadeBlock - 1) / kShadeBlock;
+        const uint64_t nstat = (uint64_t)a.depth * used_tiles;
+        for (uint64_t i = tid; i < nstat; i += gsz) a.status[(i / used_tiles) * a.ntiles + i % used_tiles] = 0ull;
+    }
     if (tid >= npix) return;
     const QueueView& q = a.q[0];
     if constexpr (MULTI) {
@@ -328,13 +360,74 @@ GPR_D float power_heur(float a, float b) {
     return a / (a + b);
 }
 
+// Walks a segmented queue in turns of 2^lg entries.  Lane l holds segment l's
+// entries and the turn it starts at; every lane of the wave calls range().
+struct SegWalk {
+    uint32_t n_l, first_l, turns, cap, lg;
+    GPR_D void init(uint32_t n, uint32_t nseg, uint32_t seg_cap, uint32_t log_turn) {
+        const uint32_t lane = threadIdx.x & 63;
+        n_l = lane < nseg ? n : 0u;
+        cap = seg_cap;
+        lg = log_turn;
+        const uint32_t k = (n_l + (1u << lg) - 1) >> lg;
+        uint32_t incl = k;
+#pragma unroll
+        for (uint32_t o = 1; o < kMaxSegs; o <<= 1) {
+            const uint32_t y = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += y;
+        }
+        turns = __builtin_amdgcn_readlane(incl, kMaxSegs - 1);
+        first_l = lane < nseg ? incl - k : 0xffffffffu;
+    }
+    GPR_D void range(uint32_t turn, uint32_t& begin, uint32_t& end) const {
+        // the last segment that starts at or before the turn (empty ones before it start there too)
+        const uint32_t g = (uint32_t)__popcll(__ballot(first_l <= turn)) - 1;
+        const uint32_t off = (turn - (uint32_t)__builtin_amdgcn_readlane(first_l, g)) << lg;
+        const uint32_t n = __builtin_amdgcn_readlane(n_l, g);
+        begin = g * cap + off;
+        end = g * cap + min(off + (1u << lg), n);
+    }
+};
+// Entries of lane l's segment: of the primary queue (one segment of all paths),
+// or of what bounce `bounce` appended.
+enum QueueKind { kPrimary, kScatter, kShadow };
+template <QueueKind KIND, bool MULTI>
+GPR_D uint32_t seg_count(const RenderArgs& a, uint32_t bounce) {
+    if constexpr (KIND == kPrimary) return npaths_of<MULTI>(a);
+    const unsigned long long v = *seg_at(a, bounce, threadIdx.x & (a.nseg - 1));  // nseg is a power of two
+    return KIND == kShadow ? (uint32_t)(v >> 32) : (uint32_t)v;
+}
+template <QueueKind KIND, bool MULTI>
+GPR_D SegWalk seg_walk(const RenderArgs& a, uint32_t bounce, uint32_t waves) {
+    const uint32_t n = seg_count<KIND, MULTI>(a, bounce), nseg = KIND == kPrimary ? 1u : a.nseg;
+    uint32_t total = (threadIdx.x & 63) < nseg ? n : 0u;
+#pragma unroll
+    for (uint32_t o = 1; o < kMaxSegs; o <<= 1) total += __shfl_xor(total, o, 64);
+    SegWalk w;
+    w.init(n, nseg, a.seg_cap, turn_log(__builtin_amdgcn_readfirstlane(total), waves, a.chunk_log));
+    return w;
+}
+// Calls f(i) for the entries of a queue, a turn's lanes together.
+template <QueueKind KIND, bool MULTI, int NT, class F>
+GPR_D void for_each_entry(const RenderArgs& a, uint32_t bounce, uint32_t* cursor, F&& f) {
+    const SegWalk w = seg_walk<KIND, MULTI>(a, bounce, gridDim.x * (NT / 64));
+    for_each_turn<NT, !MULTI>(cursor, w.turns, [&](uint32_t turn) {
+        uint32_t begin, end;
+        w.range(turn, begin, end);
+        for (uint32_t i = begin + (threadIdx.x & 63); i < end; i += 64) f(i);
+    });
+}
+
 // Per-lane ray refill over queue entries: a lane whose ray is done takes the
-// next entry from a wave-local pool of `chunk` entries (one atomic per chunk).
+// next entry from a wave-local pool of a turn's entries (one atomic a turn).
 // begin(i) sets entry i up and returns true if it finished at once; step()
 // advances the lane's ray one node and returns true when it is done.
-template <class Begin, class Step>
-GPR_D void refill_loop(uint32_t* cursor, uint32_t n, uint32_t chunk, Begin&& begin, Step&& step) {
+template <QueueKind KIND, bool MULTI, class Begin, class Step>
+GPR_D void refill_loop(const RenderArgs& a, uint32_t bounce, uint32_t* cursor, Begin&& begin, Step&& step) {
     const int lane = threadIdx.x & 63;
+    // whole turns only: a pool feeds all lanes of its wave
+    SegWalk w;
+    w.init(seg_count<KIND, MULTI>(a, bounce), KIND == kPrimary ? 1u : a.nseg, a.seg_cap, a.chunk_log);
     uint32_t pb = 0, pe = 0;  // wave-local pool of entries (wave-uniform)
     bool drained = false;
     bool active = false;
@@ -348,11 +441,10 @@ GPR_D void refill_loop(uint32_t* cursor, uint32_t n, uint32_t chunk, Begin&& beg
             uint32_t nb = pe, ne = pe;
             if (avail < cnt && !drained) {
                 uint32_t b = 0;
-                if (lane == 0) b = atomicAdd(cursor, chunk);
-                b = __shfl(b, 0, 64);
-                nb = b < n ? b : n;
-                ne = (uint64_t)b + chunk < n ? b + chunk : n;
-                if ((uint64_t)b + chunk >= n) drained = true;
+                if (lane == 0) b = atomicAdd(cursor, 1u);
+                b = __builtin_amdgcn_readfirstlane(b);
+                drained = b + 1 >= w.turns;
+                if (b < w.turns) w.range(b, nb, ne);
             }
             if (!active) {
                 const bool from_old = rank < avail;
@@ -440,14 +532,14 @@ __global__ __launch_bounds__(NT) void k_extend(RenderArgs a, uint32_t bounce) {
     st.spill = reinterpret_cast<typename Stack::Entry*>(a.spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal);
     // queue: primary = A; at bounce b the scatter queue is q[(b+1)&1]
     const QueueView& q = a.q[PRIMARY ? 0 : ((bounce + 1) & 1)];
-    const uint32_t n = PRIMARY ? npaths_of<MULTI>(a) : a.ctrl->scatter_size[bounce];
+    constexpr QueueKind kKind = PRIMARY ? kPrimary : kScatter;
     uint32_t* cur = &a.ctrl->ext_cursor[PRIMARY ? 0 : bounce + 1];
     if constexpr (REFILL && !REF_ORDER) {
         uint32_t ei = 0;
         SceneView sv;
         Trav t;
-        refill_loop(
-            cur, n, a.chunk,
+        refill_loop<kKind, MULTI>(
+            a, bounce, cur,
             [&](uint32_t i) {
                 ei = i;
                 sv = scene_of<MULTI>(a, q, i);
@@ -464,7 +556,7 @@ __global__ __launch_bounds__(NT) void k_extend(RenderArgs a, uint32_t bounce) {
                 return true;
             });
     } else {
-        for_each_claimed<NT, !MULTI>(cur, n, a.chunk, [&](uint32_t i) {
+        for_each_entry<kKind, MULTI, NT>(a, bounce, cur, [&](uint32_t i) {
             const SceneView sv = scene_of<MULTI>(a, q, i);
             const Ray3 r = queue_ray(q, i);
             const gpr_hit h = trace_one<false, REF_ORDER>(a, sv, r, st);
@@ -482,14 +574,13 @@ __global__ __launch_bounds__(NT) void k_shadow(RenderArgs a, uint32_t bounce) {
     st.lds = lds + threadIdx.x;
     st.spill = reinterpret_cast<typename Stack::Entry*>(a.spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal);
     const QueueView& q = a.q[2];
-    const uint32_t n = a.ctrl->shadow_size[bounce];
     uint32_t* cur = &a.ctrl->sh_cursor[bounce];
     if constexpr (REFILL && !REF_ORDER) {
         uint32_t ei = 0;
         SceneView sv;
         Trav t;
-        refill_loop(
-            cur, n, a.chunk,
+        refill_loop<kShadow, MULTI>(
+            a, bounce, cur,
             [&](uint32_t i) {
                 ei = i;
                 sv = scene_of<MULTI>(a, q, i);
@@ -506,7 +597,7 @@ __global__ __launch_bounds__(NT) void k_shadow(RenderArgs a, uint32_t bounce) {
                 return true;
             });
     } else {
-        for_each_claimed<NT, !MULTI>(cur, n, a.chunk, [&](uint32_t i) {
+        for_each_entry<kShadow, MULTI, NT>(a, bounce, cur, [&](uint32_t i) {
             const SceneView sv = scene_of<MULTI>(a, q, i);
             const gpr_hit h = trace_one<true, REF_ORDER>(a, sv, queue_ray(q, i), st);
             shadow_finish(a, q, i, h);
@@ -528,23 +619,40 @@ GPR_D unsigned long long pack_status(uint32_t flag, uint32_t sh, uint32_t sc) {
     return ((unsigned long long)flag << 62) | ((unsigned long long)sh << 31) | (unsigned long long)sc;
 }
 
-template <bool MULTI>
+// ORDERED: appends keep the queue order (reference RNG mode: seeds belong to
+// slots), by tickets and a decoupled look-back over one segment.  Otherwise a
+// block takes its place in its segment with one atomic.
+template <bool MULTI, bool ORDERED>
 __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bounce) {
     __shared__ uint32_t s_tile;
     __shared__ uint32_t s_wave[2][kShadeBlock / 64];
     __shared__ uint32_t s_base[2];
     __shared__ uint32_t s_last[kShadeBlock / 64];
-    const uint32_t n_in = bounce == 0 ? npaths_of<MULTI>(a) : a.ctrl->scatter_size[bounce - 1];
-    if (threadIdx.x == 0) s_tile = atomicAdd(&a.ctrl->tile_counter[bounce], 1u);
-    __syncthreads();
-    const uint32_t tile = s_tile;
-    const uint32_t ntiles_in = (n_in + kShadeBlock - 1) / kShadeBlock;
-    if (tile >= ntiles_in) return;
-    const uint32_t i = tile * kShadeBlock + threadIdx.x;
+    uint32_t tile, ntiles_in, i, n_end;
+    if constexpr (ORDERED) {
+        const uint32_t n_in = bounce == 0 ? npaths_of<MULTI>(a) : (uint32_t)*seg_at(a, bounce - 1, 0);
+        if (threadIdx.x == 0) s_tile = atomicAdd(&a.ctrl->tile_counter[bounce], 1u);
+        __syncthreads();
+        tile = s_tile;
+        ntiles_in = (n_in + kShadeBlock - 1) / kShadeBlock;
+        if (tile >= ntiles_in) return;
+        i = tile * kShadeBlock + threadIdx.x;
+        n_end = n_in;
+    } else {
+        constexpr uint32_t kLog = 8;
+        static_assert(kShadeBlock == 1 << kLog, "a turn is a block");
+        SegWalk w;
+        if (bounce == 0) w.init(npaths_of<MULTI>(a), 1, 0, kLog);
+        else w.init(seg_count<kScatter, MULTI>(a, bounce - 1), a.nseg, a.seg_cap, kLog);
+        tile = blockIdx.x;
+        if (tile >= w.turns) return;
+        w.range(tile, i, n_end);
+        i += threadIdx.x;
+    }
     const QueueView& qi = a.q[bounce & 1];
     const QueueView& qs = a.q[(bounce + 1) & 1];
     const QueueView& qsh = a.q[2];
-    bool valid = i < n_in;
+    bool valid = i < n_end;
     uint32_t job = 0, rr_start = a.rr_start, sample = 0, lpix = 0;
     SceneView sv;
     if constexpr (MULTI) {
@@ -583,7 +691,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
         const c3 w = C(wp.x, wp.y, wp.z);
         const int32_t hid = __float_as_int(hh.y);
         float smp[8];
-        if (!MULTI && a.rng_mode == GPR_RNG_REFERENCE) {
+        if constexpr (ORDERED) {
             uint32_t s = qi.seed[i];
 #pragma unroll
             for (int k = 0; k < 8; ++k) smp[k] = lcg_next(s);
@@ -649,7 +757,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
             {
                 const BSample bs = bsdf_sample(m, fr, wo, smp[5], smp[6], smp[4]);
                 c3 ow = bs.pdf == 0.f ? C(0.f) : w * bs.f / bs.pdf;
-                if ((MULTI || a.rng_mode != GPR_RNG_REFERENCE) && bounce >= rr_start && !black(ow)) {
+                if (!ORDERED && bounce >= rr_start && !black(ow)) {
                     const float qq = fmax_h(0.05f, 1 - cmax(ow));
                     if (smp[7] < qq) ow = C(0.f);
                     else ow = ow / (1 - qq);
@@ -683,7 +791,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
         s_wave[0][wave] = (uint32_t)__popcll(bsh);
         s_wave[1][wave] = (uint32_t)__popcll(bsc);
     }
-    if constexpr (!MULTI) {
+    if constexpr (!MULTI && !ORDERED) {
         if (a.log_s) {  // what gpr_renderer_queue_sizes reports of the last sample
             const uint32_t smask = (1u << a.log_s) - 1u;
             const unsigned long long mine = __ballot(valid && (pix & smask) == smask);
@@ -691,12 +799,12 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
         }
     }
     __syncthreads();
-    if constexpr (!MULTI) {
+    if constexpr (!MULTI && !ORDERED) {
         if (a.log_s && threadIdx.x == 0) {
             uint32_t l = 0;
 #pragma unroll
             for (int k = 0; k < kShadeBlock / 64; ++k) l += s_last[k];
-            if (l) atomicAdd(&a.ctrl->last[bounce][tile % kLastSpread], (unsigned long long)(l >> 16) << 32 | (l & 0xffffu));
+            if (l) atomicAdd(&a.last[bounce * kLastSpread + tile % kLastSpread], (unsigned long long)(l >> 16) << 32 | (l & 0xffffu));
         }
     }
     uint32_t wsh = 0, wsc = 0, tsh = 0, tsc = 0;
@@ -709,7 +817,15 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
         tsh += s_wave[0][k];
         tsc += s_wave[1][k];
     }
-    if (threadIdx.x == 0) {
+    if constexpr (!ORDERED) {
+        if (threadIdx.x == 0) {
+            const uint32_t g = blockIdx.x / kSegGroup % a.nseg;
+            unsigned long long at = 0;
+            if (tsh + tsc) at = atomicAdd(seg_at(a, bounce, g), (unsigned long long)tsh << 32 | tsc);
+            s_base[0] = g * a.seg_cap + (uint32_t)(at >> 32);
+            s_base[1] = g * a.seg_cap + (uint32_t)at;
+        }
+    } else if (threadIdx.x == 0) {
         unsigned long long* st = a.status + (uint64_t)bounce * a.ntiles;
         uint32_t psh = 0, psc = 0;
         if (tile == 0) {
@@ -740,10 +856,8 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
         }
         s_base[0] = psh;
         s_base[1] = psc;
-        if (tile == ntiles_in - 1) {
-            a.ctrl->shadow_size[bounce] = psh + tsh;
-            a.ctrl->scatter_size[bounce] = psc + tsc;
-        }
+        if (tile == ntiles_in - 1)
+            *seg_at(a, bounce, 0) = (unsigned long long)(psh + tsh) << 32 | (psc + tsc);
     }
     __syncthreads();
     if (has_sh) {
@@ -760,7 +874,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
         qs.d_tmax[s] = make_float4(osc.d.x, osc.d.y, osc.d.z, osc.tmax);
         qs.w_pdf[s] = make_float4(osc.w.r, osc.w.g, osc.w.b, osc.pdf);
         qs.pix[s] = pix | (osc.spec ? 0x80000000u : 0u);
-        qs.rng[s] = rng_out;
+        if constexpr (!ORDERED) qs.rng[s] = rng_out;
         if constexpr (MULTI) qs.job[s] = job;
     }
 }
@@ -889,6 +1003,11 @@ std::vector<TraceCfg> engine_tune_space() {
 }
 
 namespace {
+// Entries of a queue that holds `paths` paths or what a bounce of them appends.
+uint32_t queue_entries(uint32_t paths, bool tight) {
+    const Segs s = segs_for(paths, tight);
+    return std::max(paths, s.nseg * s.cap);
+}
 int alloc_queue(DevBuf& mem, QueueView& q, uint32_t n, bool with_job) {
     const size_t per = 16 * 4 + 4 + 8 + (with_job ? 4 : 0);
     GPR_TRY(mem.alloc((size_t)n * per + 8 * 256));
@@ -913,8 +1032,8 @@ int alloc_queue(DevBuf& mem, QueueView& q, uint32_t n, bool with_job) {
 
 struct Engine {
     int device = 0;
-    uint32_t capacity = 0, max_jobs = 0, ntiles = 0;
-    DevBuf qmem[3], ctrl, status, spill, pass, scenes;
+    uint32_t capacity = 0, max_jobs = 0;
+    DevBuf qmem[3], ctrl, seg, spill, pass, scenes;
     DevBuf terms, nterm;      // passes of several samples a job
     uint64_t term_limit = 0;  // bytes the term lists may take
     QueueView q[3];
@@ -957,11 +1076,10 @@ int engine_create(int device, uint32_t capacity, uint32_t max_jobs, Engine** out
     e->device = device;
     e->capacity = capacity;
     e->max_jobs = max_jobs;
-    e->ntiles = div_up(capacity, kShadeBlock);
-    for (int k = 0; k < 3; ++k) GPR_TRY(alloc_queue(e->qmem[k], e->q[k], capacity, true));
+    for (int k = 0; k < 3; ++k) GPR_TRY(alloc_queue(e->qmem[k], e->q[k], queue_entries(capacity, true), true));
     GPR_TRY(e->ctrl.alloc(sizeof(Ctrl)));
+    GPR_TRY(e->seg.alloc(8ull * seg_words(segs_for(capacity, true).nseg)));
     GPR_HIP(hipMemsetAsync(e->ctrl.p, 0, sizeof(Ctrl), stream()));
-    GPR_TRY(e->status.alloc(8ull * kMaxBounce * e->ntiles));
     GPR_TRY(e->pass.alloc(sizeof(PassBuf)));
     int cus = 0;
     GPR_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
@@ -988,8 +1106,7 @@ int engine_create(int device, uint32_t capacity, uint32_t max_jobs, Engine** out
 void engine_destroy(Engine* e) { delete e; }
 
 size_t engine_device_bytes(const Engine* e) {
-    return e->qmem[0].bytes + e->qmem[1].bytes + e->qmem[2].bytes + e->ctrl.bytes + e->status.bytes +
-           e->spill.bytes + e->pass.bytes + e->scenes.bytes;
+    return e->qmem[0].bytes + e->qmem[1].bytes + e->qmem[2].bytes + e->ctrl.bytes + e->seg.bytes + e->spill.bytes + e->pass.bytes + e->scenes.bytes;
 }
 
 int engine_set_scenes(Engine* e, const std::vector<SceneView>& views, hipStream_t st) {
@@ -1017,11 +1134,13 @@ int record_pass(Engine* e, uint32_t depth, int kidx, uint32_t chunk, uint32_t si
     for (int k = 0; k < 3; ++k) a.q[k] = e->q[k];
     a.fb = fb;
     a.ctrl = e->ctrl.as<Ctrl>();
-    a.status = e->status.as<unsigned long long>();
     a.spill = e->spill.as<int2>();
-    a.ntiles = e->ntiles;
+    const Segs sg = segs_for(size, true);
+    a.seg = e->seg.as<unsigned long long>();
+    a.nseg = sg.nseg;
+    a.seg_cap = sg.cap;
     a.depth = depth;
-    a.chunk = chunk;
+    a.chunk_log = 31u - (uint32_t)__builtin_clz(chunk);
     a.rng_mode = GPR_RNG_PCG;
     if (terms) {
         a.terms = e->terms.as<float4>();
@@ -1033,7 +1152,7 @@ int record_pass(Engine* e, uint32_t depth, int kidx, uint32_t chunk, uint32_t si
     hipLaunchKernelGGL(k_gen<true>, dim3(div_up(size, 256)), dim3(256), 0, st, a);
     hipLaunchKernelGGL(pk.ext_primary, tg, tb, 0, st, a, 0u);
     for (uint32_t b = 0; b < depth; ++b) {
-        hipLaunchKernelGGL(k_shade<true>, dim3(div_up(size, kShadeBlock)), dim3(kShadeBlock), 0, st, a, b);
+        hipLaunchKernelGGL((k_shade<true, false>), dim3(shade_blocks(size, sg.nseg)), dim3(kShadeBlock), 0, st, a, b);
         hipLaunchKernelGGL(pk.shadow, tg, tb, 0, st, a, b);
         hipLaunchKernelGGL(pk.ext_scatter, tg, tb, 0, st, a, b);
     }
@@ -1238,9 +1357,9 @@ using namespace gpr;
 struct PassWork {
     std::mutex mu;
     DevBuf spill;  // kStackGlobal entries per resident lane, allocated once
-    DevBuf qmem[3], terms, nterm, status;
+    DevBuf qmem[3], terms, nterm;
     QueueView q[3];
-    uint32_t paths = 0, depth = 0, ntiles = 0;
+    uint32_t paths = 0, depth = 0;
     uint64_t gen = 0;  // of the buffers; graphs captured with older ones are dropped
 };
 namespace {
@@ -1265,6 +1384,8 @@ struct gpr_renderer {
     uint32_t npix = 0, ntiles = 0;
     uint32_t spp_done = 0;
     DevBuf fb, ctrl, status;
+    DevBuf seg;              // queue segment counters, then those of the last sample
+    uint32_t last_nseg = 1;  // segments of the last pass
     DevBuf qmem[3];
     DevBuf seeds[2];
     QueueView q[3];
@@ -1306,8 +1427,6 @@ RenderArgs make_args(gpr_renderer* r, uint32_t log_s) {
     if (log_s) {
         const PassWork& w = *r->work;
         for (int k = 0; k < 3; ++k) a.q[k] = w.q[k];
-        a.status = w.status.as<unsigned long long>();
-        a.ntiles = w.ntiles;
         a.terms = w.terms.as<float4>();
         a.nterm = w.nterm.as<uint8_t>();
         a.tstride = a.npix;
@@ -1317,8 +1436,13 @@ RenderArgs make_args(gpr_renderer* r, uint32_t log_s) {
         a.ntiles = r->ntiles;
     }
     a.spill = r->work->spill.as<int2>();
-    a.chunk = 64;
+    a.seg = r->seg.as<unsigned long long>();
+    a.last = a.seg + seg_words(kMaxSegs);
     a.rng_mode = r->opts.rng_mode;
+    const Segs sg = a.rng_mode == GPR_RNG_REFERENCE ? Segs{1, a.npix} : segs_for(a.npix, false);
+    a.nseg = sg.nseg;
+    a.seg_cap = sg.cap;
+    a.chunk_log = 6;
     a.rr_start = r->opts.rr_start;
     a.seed = r->opts.seed;
     return a;
@@ -1341,7 +1465,10 @@ int launch_pass(gpr_renderer* r, uint32_t log_s, hipStream_t st) {
     if (ref) hipLaunchKernelGGL((k_extend<true, true, false, NT, SL>), tg, tb, 0, st, a, 0u);
     else hipLaunchKernelGGL((k_extend<true, false, false, NT, SL>), tg, tb, 0, st, a, 0u);
     for (uint32_t b = 0; b < r->opts.max_depth; ++b) {
-        hipLaunchKernelGGL(k_shade<false>, dim3(div_up(a.npix, kShadeBlock)), dim3(kShadeBlock), 0, st, a, b);
+        if (a.rng_mode == GPR_RNG_REFERENCE)
+            hipLaunchKernelGGL((k_shade<false, true>), dim3(div_up(a.npix, kShadeBlock)), dim3(kShadeBlock), 0, st, a, b);
+        else
+            hipLaunchKernelGGL((k_shade<false, false>), dim3(shade_blocks(a.npix, a.nseg)), dim3(kShadeBlock), 0, st, a, b);
         if (ref) {
             hipLaunchKernelGGL((k_shadow<true, false, NT, SL>), tg, tb, 0, st, a, b);
             hipLaunchKernelGGL((k_extend<false, true, false, NT, SL>), tg, tb, 0, st, a, b);
@@ -1407,10 +1534,8 @@ int grow_work(gpr_renderer* r, PassWork& w, uint32_t paths) {
         w.gen = ++g_work_gen;
     }
     // given back first, so that the old and the new buffers never exist together
-    for (DevBuf* b : {&w.qmem[0], &w.qmem[1], &w.qmem[2], &w.terms, &w.nterm, &w.status}) b->release();
-    w.ntiles = div_up(np, kShadeBlock);
-    GPR_TRY(w.status.alloc(8ull * kMaxBounce * w.ntiles));
-    for (int k = 0; k < 3; ++k) GPR_TRY(alloc_queue(w.qmem[k], w.q[k], np, false));
+    for (DevBuf* b : {&w.qmem[0], &w.qmem[1], &w.qmem[2], &w.terms, &w.nterm}) b->release();
+    for (int k = 0; k < 3; ++k) GPR_TRY(alloc_queue(w.qmem[k], w.q[k], queue_entries(np, false), false));
     GPR_TRY(w.terms.alloc(16ull * np * max_terms(nd)));
     GPR_TRY(w.nterm.alloc(np));
     w.paths = np;
@@ -1447,9 +1572,10 @@ int renderer_alloc(gpr_renderer* r) {
     GPR_HIP(hipSetDevice(s->device));
     GPR_TRY(r->fb.alloc(16ull * npix));
     GPR_TRY(r->ctrl.alloc(sizeof(Ctrl)));
+    GPR_TRY(r->seg.alloc(8ull * (seg_words(kMaxSegs) + kMaxBounce * kLastSpread)));
     r->ntiles = div_up(npix, kShadeBlock);
     GPR_TRY(r->status.alloc(8ull * kMaxBounce * r->ntiles));
-    for (int k = 0; k < 3; ++k) GPR_TRY(alloc_queue(r->qmem[k], r->q[k], r->npix, false));
+    for (int k = 0; k < 3; ++k) GPR_TRY(alloc_queue(r->qmem[k], r->q[k], queue_entries(r->npix, false), false));
     for (int k = 0; k < 2; ++k) {
         GPR_TRY(r->seeds[k].alloc(4ull * npix));
         GPR_HIP(hipMemsetAsync(r->seeds[k].p, 0, 4ull * npix, stream()));  // DEVICE_BUFFER allocations start zeroed (buffer.h:62)
@@ -1613,6 +1739,7 @@ int gpr_render(gpr_renderer* r, uint32_t spp) {
         GPR_HIP(hipGraphLaunch(g, st));
         left -= 1u << log_s;
         r->last_log_s = log_s;
+        r->last_nseg = make_args(r, log_s).nseg;
     }
     r->spp_done += spp;
     uint32_t err = 0;
@@ -1641,17 +1768,18 @@ int gpr_renderer_read(gpr_renderer* r, float* rgb, uint32_t* cnt) {
 
 int gpr_renderer_queue_sizes(gpr_renderer* r, uint32_t* shadow, uint32_t* scatter, uint32_t cap) {
     if (!r) return fail(GPR_ERR_INVALID, "gpr_renderer_queue_sizes: null renderer");
-    Ctrl c;
-    GPR_HIP(hipMemcpyAsync(&c, r->ctrl.p, sizeof(Ctrl), hipMemcpyDeviceToHost, stream()));
+    std::vector<unsigned long long> c(r->seg.bytes / 8);
+    GPR_HIP(hipMemcpyAsync(c.data(), r->seg.p, r->seg.bytes, hipMemcpyDeviceToHost, stream()));
     GPR_HIP(hipStreamSynchronize(stream()));
     for (uint32_t b = 0; b < cap && b < kMaxBounce; ++b) {
-        uint32_t sh = c.shadow_size[b], sc = c.scatter_size[b];
-        if (r->last_log_s) {  // the sizes of the last sample alone
-            sh = sc = 0;
-            for (uint32_t k = 0; k < kLastSpread; ++k) {
-                sh += (uint32_t)(c.last[b][k] >> 32);
-                sc += (uint32_t)c.last[b][k];
-            }
+        uint32_t sh = 0, sc = 0;
+        // of several samples the last one alone
+        const uint32_t parts = r->last_log_s ? kLastSpread : r->last_nseg;
+        for (uint32_t k = 0; k < parts; ++k) {
+            const unsigned long long n = r->last_log_s ? c[seg_words(kMaxSegs) + b * kLastSpread + k]
+                                                       : c[(b * r->last_nseg + k) * seg_stride(r->last_nseg)];
+            sh += (uint32_t)(n >> 32);
+            sc += (uint32_t)n;
         }
         if (shadow) shadow[b] = sh;
         if (scatter) scatter[b] = sc;

@@ -17,6 +17,9 @@
 namespace gpr {
 namespace {
 
+// chunks are used as powers of two (rounded down)
+uint32_t log2_floor(uint32_t v) { return 31u - (uint32_t)__builtin_clz(v); }
+
 __global__ void k_zero_u64(unsigned long long* p, int n) {
     if ((int)threadIdx.x < n) p[threadIdx.x] = 0ull;
 }
@@ -43,16 +46,21 @@ template <bool ANY, int NT, int SL>
 __global__ __launch_bounds__(NT) void k_trace_fast(SceneView sv, const gpr_ray* __restrict__ rays,
                                                    gpr_hit* __restrict__ hits, uint64_t n,
                                                    unsigned long long* __restrict__ cursor,
-                                                   int2* __restrict__ spill, uint32_t chunk) {
+                                                   int2* __restrict__ spill, uint32_t chunk_log) {
     using Stack = LaneStack<ANY, NT, SL>;
     __shared__ typename Stack::Entry lds[SL * NT];
     Stack st;
     st.lds = lds + threadIdx.x;
     st.spill = reinterpret_cast<typename Stack::Entry*>(spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal);
-    for_each_claimed<NT, false>(cursor, n, chunk, [&](uint64_t i) {
-        gpr_hit h;
-        if (!fast_trace<ANY>(sv, load_ray(rays, i), st, h)) atomicAdd(cursor + 1, 1ull);  // stack overflow count
-        store_hit(hits, i, h);
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t lg = turn_log(n, gridDim.x * (NT / 64), chunk_log);
+    for_each_turn<NT, false>(cursor, (n + (1ull << lg) - 1) >> lg, [&](uint64_t turn) {
+        const uint64_t end = min((turn + 1) << lg, n);
+        for (uint64_t i = (turn << lg) + lane; i < end; i += 64) {
+            gpr_hit h;
+            if (!fast_trace<ANY>(sv, load_ray(rays, i), st, h)) atomicAdd(cursor + 1, 1ull);  // stack overflow count
+            store_hit(hits, i, h);
+        }
     });
 }
 
@@ -69,7 +77,7 @@ template <bool ANY, int NT, int SL>
 __global__ __launch_bounds__(NT) void k_trace_refill(SceneView sv, const gpr_ray* __restrict__ rays,
                                                      gpr_hit* __restrict__ hits, uint64_t n,
                                                      unsigned long long* __restrict__ cursor,
-                                                     int2* __restrict__ spill, uint32_t chunk) {
+                                                     int2* __restrict__ spill, uint32_t chunk_log) {
     using Stack = LaneStack<ANY, NT, SL>;
     __shared__ typename Stack::Entry lds[SL * NT];
     Stack st;
@@ -80,8 +88,7 @@ __global__ __launch_bounds__(NT) void k_trace_refill(SceneView sv, const gpr_ray
     // dealt out, thin where the batch is short, the others are claimed
     const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (NT / 64) + threadIdx.x / 64);
     const uint32_t waves = gridDim.x * (NT / 64);
-    const uint32_t width = spread_width(n, waves);
-    const uint32_t first = width < 64 ? width : chunk;
+    const uint32_t first = 1u << turn_log(n, waves, chunk_log), chunk = 1u << chunk_log;
     const uint64_t claimed_from = (uint64_t)waves * first;
     uint64_t pb = min((uint64_t)wave * first, n), pe = min(pb + first, n);
     bool drained = claimed_from >= n;  // nothing is left to claim (wave-uniform)
@@ -322,7 +329,7 @@ int launch_trace(const SceneView& sv, const gpr_ray* rays, gpr_hit* hits, uint64
     const TraceKernel ks[4] = {v.closest, v.any, v.closest_r, v.any_r};
     const dim3 grid((unsigned)std::min<uint64_t>(R.grid[k][kind], want));
     hipLaunchKernelGGL(ks[kind], grid, dim3(v.nt), 0, st, sv, rays, hits, n, cur, R.spill.as<int2>(),
-                       (uint32_t)chunk);
+                       log2_floor((uint32_t)chunk));
     GPR_HIP(hipGetLastError());
     return GPR_OK;
 }

@@ -433,28 +433,28 @@ GPR_D bool fast_trace(const SceneView& sv, const Ray3& r, Stack& st, gpr_hit& hi
     return t.node == kTravDone;
 }
 
-// Lanes a wave uses for n rays: 64, or fewer when kSpreadWaves waves of 32 (or
-// the whole grid, if smaller) hold them all.
+// Rays a wave takes a turn: `chunk` (a power of two, at least 64) of them, or
+// fewer than a wave has lanes when kSpreadWaves waves of 32 lanes (or the whole
+// grid, if smaller) hold all n.  Log2.
 constexpr uint32_t kSpreadWaves = 4096;
 template <class I>
-GPR_D uint32_t spread_width(I n, uint32_t waves) {
+GPR_D uint32_t turn_log(I n, uint32_t waves, uint32_t chunk_log) {
     const uint32_t spread = waves < kSpreadWaves ? waves : kSpreadWaves;
-    if (n > (I)32 * spread) return 64;
-    uint32_t w = 1;
-    while ((I)w * spread < n) w <<= 1;
+    if (n > (I)32 * spread) return chunk_log;
+    uint32_t w = 0;
+    while (((I)spread << w) < n) ++w;
     return w;
 }
 
-// Hands the rays (queue entries) below n to the waves of the grid, `chunk`
-// consecutive ones a turn, and calls f(i) for each.
+// Hands turns 0 .. n-1 to the waves of the grid and calls f(turn) for each.
 //  - Half of the turns are dealt out in order, the rest is claimed from the
 //    cursor as waves come free: claims are atomics on one address, which
 //    serialise at ~12 ns each on this chip, so claiming every 64 rays bounded
 //    the renderer's big passes.
 //  - A short queue is spread thin over kSpreadWaves waves (four to a SIMD): a
 //    wave takes the union of its lanes' node steps and leaf tests, so thin
-//    waves finish sooner and the chip has room for them.
-// Against a claim per chunk: 4 samples of the 1920x1080 sphere grid 14.9 ms
+//    waves finish sooner and the chip has room for them (turn_log).
+// Against a claim per 64 rays: 4 samples of the 1920x1080 sphere grid 14.9 ms
 // instead of 16.7 (15.4 with only the first turn dealt out, 15.3 with three
 // quarters), one sample 5.0 instead of 6.5; one sample of an 803x451 textured
 // scene 1.48 ms instead of 2.60 (1.85 unspread, 1.60 / 1.51 / 1.48 over 1024 /
@@ -464,32 +464,21 @@ GPR_D uint32_t spread_width(I n, uint32_t waves) {
 // CU too large made 4M incoherent rays 24 % slower).  Without it only the first
 // turn is dealt out.
 template <int NT, bool DEAL_HALF, class I, class C, class F>
-GPR_D void for_each_claimed(C* cursor, I n, uint32_t chunk, F&& f) {
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (NT / 64) + threadIdx.x / 64);
+GPR_D void for_each_turn(C* cursor, I n, F&& f) {
     const uint32_t waves = gridDim.x * (NT / 64);
-    const uint32_t w = spread_width(n, waves);
-    if (w < 64) {
-        const uint32_t i = wave * w + lane;
-        if (lane < w && i < n) f((I)i);
-        return;
-    }
-    const I round = (I)waves * chunk;
-    uint32_t dealt = DEAL_HALF ? (uint32_t)(n / (2 * round)) : 1u;
-    const I claimed_from = (dealt > 1 ? dealt : 1) * round;
-    I base = (I)wave * chunk;
-    while (base < n) {
-        for (uint32_t k = 0; k < chunk; k += 64) {
-            const I i = base + k + lane;
-            if (i < n) f(i);
-        }
+    uint32_t dealt = DEAL_HALF ? (uint32_t)(n / (2 * (I)waves)) : 1u;
+    const I claimed_from = (I)(dealt > 1 ? dealt : 1) * waves;
+    I t = __builtin_amdgcn_readfirstlane(blockIdx.x * (NT / 64) + threadIdx.x / 64);
+    while (t < n) {
+        f(t);
         if (dealt > 1) {
             --dealt;
-            base += round;
+            t += waves;
         } else {
+            if (claimed_from >= n) break;
             C got = 0;
-            if (lane == 0) got = atomicAdd(cursor, (C)chunk);
-            base = claimed_from + (I)__shfl(got, 0, 64);
+            if ((threadIdx.x & 63) == 0) got = atomicAdd(cursor, (C)1);
+            t = claimed_from + (I)__shfl(got, 0, 64);
         }
     }
 }
