@@ -209,7 +209,7 @@ struct gpr_scene {
     bool committed = false;
     float r2c[16];
     uint64_t last_nv = 0, last_nt = 0;
-    int trace_nt = 256, trace_sl = 16, trace_chunk = 64, trace_refill = 0;  // BVH4 traversal launch configuration
+    int trace_nt = 0, trace_sl = 0, trace_chunk = 0, trace_refill = 0;  // BVH4 traversal launch configuration (nt 0: by batch)
     gpr::SceneView view() const;
 };
 
@@ -224,10 +224,10 @@ int sort_pairs(const uint32_t* keys, uint32_t* skeys, uint32_t* sidx, uint32_t n
 size_t sort_scratch_bytes(uint32_t n);
 int sort_prepare(void* scratch, size_t bytes, hipStream_t st);
 // trace.hip
-// nt / sl / chunk: block size, LDS stack entries, rays claimed per wave (the autotuner's space)
+// nt / sl / chunk: block size, LDS stack entries, rays claimed per wave (the autotuner's space); nt 0: chosen by the
+// size of the batch
 int launch_trace(const SceneView& sv, const gpr_ray* rays, gpr_hit* hits, uint64_t n, uint32_t flags,
-                 unsigned long long* stats, hipStream_t st, int nt = 256, int sl = 16, int chunk = 64,
-                 int refill = 0);
+                 unsigned long long* stats, hipStream_t st, int nt = 0, int sl = 0, int chunk = 0, int refill = 0);
 bool trace_cfg_valid(int nt, int sl, int chunk);
 int launch_trace_stats(const SceneView& sv, const gpr_ray* rays, uint64_t n, bool any, unsigned long long* stats,
                        hipStream_t st);

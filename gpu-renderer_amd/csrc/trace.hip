@@ -72,6 +72,11 @@ __global__ __launch_bounds__(NT) void k_trace_fast(SceneView sv, const gpr_ray* 
 // leaf children and tests them in wave-wide leaf rounds (TravD), before the
 // lane's next node: its hits are those of k_trace_fast too.
 constexpr int kLeafRound = 32;  // parked lanes of a wave that start an any-hit leaf round
+// Idle lanes that start a refill: taking rays up (a load from HBM and three
+// divisions) stops the whole wave, so a few lanes wait for each other.  4M rays
+// at 1M triangles, tuned, closest hit with 1 / 4 / 8 / 16 / 24 idle lanes 2.78 /
+// 2.69 / 2.63 / 2.63 / 2.63 ms; any hit with 16 / 24 / 32: 2.37 / 2.30 / 2.32 ms.
+constexpr int kRefillClosest = 16, kRefillAny = 24;
 
 template <bool ANY, int NT, int SL>
 __global__ __launch_bounds__(NT) void k_trace_refill(SceneView sv, const gpr_ray* __restrict__ rays,
@@ -98,7 +103,7 @@ __global__ __launch_bounds__(NT) void k_trace_refill(SceneView sv, const gpr_ray
     std::conditional_t<ANY, TravD, Trav> t;
     while (true) {
         const unsigned long long need = __ballot(!active);
-        if (need != 0ull && !(drained && pb == pe)) {
+        if (__popcll(need) >= (ANY ? kRefillAny : kRefillClosest) && !(drained && pb == pe)) {
             const uint32_t cnt = (uint32_t)__popcll(need);
             const uint32_t rank =
                 __builtin_amdgcn_mbcnt_hi((uint32_t)(need >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)need, 0u));
@@ -303,6 +308,30 @@ bool trace_cfg_valid(int nt, int sl, int chunk) {
     return trace_variant_index(nt, sl) >= 0 && chunk >= 64 && chunk % 64 == 0 && chunk <= 4096;
 }
 
+namespace {
+// Launch shape of a batch on a scene that was not tuned.  Refill pays once the
+// queue is long enough to keep its lanes fed; any-hit walks are shorter, so
+// later.  Measured (us, at 1M / 20K triangles):
+//   closest  512K rays  128x16  668 /  430   256x8  607 /  391   64x16 refill  697 /  448
+//            768K               832 /  553          823 /  546                 770 /  517
+//            2M                1787 / 1215         1734 / 1191                1485 /  987
+//   any hit  1M rays    128x16  849 /  627                       64x32 refill  976 /  688
+//            2M                1447 / 1122                                    1397 / 1014
+// and 256K closest-hit rays at 1M triangles 128x16 379, 256x8 408.
+void trace_default_cfg(uint64_t n, bool any, int& nt, int& sl, int& chunk, int& refill) {
+    chunk = 64;
+    refill = n >= (any ? 3u << 19 : 3u << 18) ? 1 : 0;
+    if (refill) {
+        nt = 64;
+        sl = any ? 32 : 16;
+    } else {
+        const bool mid = !any && n >= (3u << 17);
+        nt = mid ? 256 : 128;
+        sl = mid ? 8 : 16;
+    }
+}
+}  // namespace
+
 int launch_trace(const SceneView& sv, const gpr_ray* rays, gpr_hit* hits, uint64_t n, uint32_t flags,
                  unsigned long long* stats, hipStream_t st, int nt, int sl, int chunk, int refill) {
     if (n == 0) return GPR_OK;
@@ -316,6 +345,7 @@ int launch_trace(const SceneView& sv, const gpr_ray* rays, gpr_hit* hits, uint64
         GPR_HIP(hipGetLastError());
         return GPR_OK;
     }
+    if (nt == 0) trace_default_cfg(n, any, nt, sl, chunk, refill);
     const int k = trace_variant_index(nt, sl);
     if (k < 0 || !trace_cfg_valid(nt, sl, chunk)) return fail(GPR_ERR_INVALID, "trace: configuration outside the tuned set");
     TraceResources* rp = nullptr;
