@@ -166,6 +166,11 @@ struct BvhDev {
     Bvh4Node* bvh4 = nullptr;
     TriRec* tris = nullptr;
     float timing[5] = {0, 0, 0, 0, 0};
+    hipEvent_t ev[5] = {};  // stage boundaries, created by the first build
+    ~BvhDev() {
+        for (hipEvent_t e : ev)
+            if (e) (void)hipEventDestroy(e);
+    }
 };
 
 struct Mesh {
