@@ -2,14 +2,12 @@
 // src/renderer/pathtracer.cu:41-150, kernels of src/renderer/pathtracer_kernel.h).
 //
 // One sample of every pixel is a fixed launch sequence with no host round
-// trip:  gen -> extend(primary) -> max_depth x { shade -> shadow -> extend }
+// trip:  gen -> extend(primary) -> max_depth x { shade -> trace } -> flush
 // -> finish.  Queue sizes live on the device; each kernel reads the size it
 // consumes and early-exits, so the whole sample can be replayed as a hipGraph.
 //
 //   gen     primary rays (InitRandom/NextRandom jitter or PCG32), queue A
-//   extend  closest hit of a queue; for scattered rays also the BSDF-sampling
-//           MIS contribution (accumulate_BSDF_sampling_contribution) and, in
-//           reference RNG mode, its roulette (pathtracer_kernel.h:684-749)
+//   extend  closest hit of the primary queue
 //   shade   shade_hit_with_MIS: emission, NEE shadow append, BSDF scatter
 //           append.  Appends are compacted: a wave ballot and mbcnt give lane
 //           offsets, LDS gives wave offsets, and one atomic on the counter of
@@ -17,11 +15,16 @@
 //           RNG mode, where slot order must equal the serial order of the
 //           reference's host loop, a decoupled look-back over tiles (one 64-bit
 //           status word per tile) gives it instead.
-//   shadow  any-hit of the shadow queue + accumulate_light_sampling_contribution
+//   trace   any hit of the shadow queue + accumulate_light_sampling_contribution;
+//           closest hit of the scatter queue, its BSDF-sampling MIS term
+//           (accumulate_BSDF_sampling_contribution), left in the entry, and, in
+//           reference RNG mode, its roulette (pathtracer_kernel.h:684-749)
+//   flush   the MIS terms of the last bounce; those of the others are added by
+//           the next shade
 //
 // Per pixel the frame buffer receives emission, NEE and BSDF terms in the
-// same order as the reference kernels (one queue entry per pixel per kernel,
-// so the read-modify-write needs no atomics).
+// same order as the reference kernels (in every kernel one thread adds to a
+// path, so the read-modify-write needs no atomics).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -360,57 +363,63 @@ GPR_D float power_heur(float a, float b) {
     return a / (a + b);
 }
 
-// Walks a segmented queue in turns of 2^lg entries.  Lane l holds segment l's
-// entries and the turn it starts at; every lane of the wave calls range().
+// Walks a segmented queue in turns of 2^lg entries; every member is uniform.
 struct SegWalk {
-    uint32_t n_l, first_l, turns, cap, lg;
-    GPR_D void init(uint32_t n, uint32_t nseg, uint32_t seg_cap, uint32_t log_turn) {
-        const uint32_t lane = threadIdx.x & 63;
-        n_l = lane < nseg ? n : 0u;
+    uint32_t n[kMaxSegs], first[kMaxSegs];  // a segment's entries, and the turn it starts at
+    uint32_t turns, cap, lg;
+    GPR_D void init(uint32_t seg_cap, uint32_t log_turn) {
         cap = seg_cap;
         lg = log_turn;
-        const uint32_t k = (n_l + (1u << lg) - 1) >> lg;
-        uint32_t incl = k;
+        turns = 0;
 #pragma unroll
-        for (uint32_t o = 1; o < kMaxSegs; o <<= 1) {
-            const uint32_t y = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += y;
+        for (uint32_t g = 0; g < kMaxSegs; ++g) {
+            first[g] = turns;
+            turns += (n[g] + (1u << lg) - 1) >> lg;
         }
-        turns = __builtin_amdgcn_readlane(incl, kMaxSegs - 1);
-        first_l = lane < nseg ? incl - k : 0xffffffffu;
+    }
+    GPR_D uint32_t total() const {
+        uint32_t t = 0;
+#pragma unroll
+        for (uint32_t g = 0; g < kMaxSegs; ++g) t += n[g];
+        return t;
     }
     GPR_D void range(uint32_t turn, uint32_t& begin, uint32_t& end) const {
         // the last segment that starts at or before the turn (empty ones before it start there too)
-        const uint32_t g = (uint32_t)__popcll(__ballot(first_l <= turn)) - 1;
-        const uint32_t off = (turn - (uint32_t)__builtin_amdgcn_readlane(first_l, g)) << lg;
-        const uint32_t n = __builtin_amdgcn_readlane(n_l, g);
+        uint32_t g = 0, f = first[0], m = n[0];
+#pragma unroll
+        for (uint32_t k = 1; k < kMaxSegs; ++k) {
+            const bool later = first[k] <= turn;
+            g = later ? k : g;
+            f = later ? first[k] : f;
+            m = later ? n[k] : m;
+        }
+        const uint32_t off = (turn - f) << lg;
         begin = g * cap + off;
-        end = g * cap + min(off + (1u << lg), n);
+        end = g * cap + min(off + (1u << lg), m);
     }
 };
-// Entries of lane l's segment: of the primary queue (one segment of all paths),
-// or of what bounce `bounce` appended.
+// Entries of the primary queue (one segment of all paths), or of what bounce
+// `bounce` appended.
 enum QueueKind { kPrimary, kScatter, kShadow };
 template <QueueKind KIND, bool MULTI>
-GPR_D uint32_t seg_count(const RenderArgs& a, uint32_t bounce) {
-    if constexpr (KIND == kPrimary) return npaths_of<MULTI>(a);
-    const unsigned long long v = *seg_at(a, bounce, threadIdx.x & (a.nseg - 1));  // nseg is a power of two
-    return KIND == kShadow ? (uint32_t)(v >> 32) : (uint32_t)v;
-}
-template <QueueKind KIND, bool MULTI>
-GPR_D SegWalk seg_walk(const RenderArgs& a, uint32_t bounce, uint32_t waves) {
-    const uint32_t n = seg_count<KIND, MULTI>(a, bounce), nseg = KIND == kPrimary ? 1u : a.nseg;
-    uint32_t total = (threadIdx.x & 63) < nseg ? n : 0u;
+GPR_D void seg_counts(const RenderArgs& a, uint32_t bounce, SegWalk& w) {
 #pragma unroll
-    for (uint32_t o = 1; o < kMaxSegs; o <<= 1) total += __shfl_xor(total, o, 64);
-    SegWalk w;
-    w.init(n, nseg, a.seg_cap, turn_log(__builtin_amdgcn_readfirstlane(total), waves, a.chunk_log));
-    return w;
+    for (uint32_t g = 0; g < kMaxSegs; ++g) {
+        w.n[g] = 0;
+        if constexpr (KIND == kPrimary) {
+            if (g == 0) w.n[g] = npaths_of<MULTI>(a);
+        } else if (g < a.nseg) {
+            const unsigned long long v = *seg_at(a, bounce, g);
+            w.n[g] = __builtin_amdgcn_readfirstlane(KIND == kShadow ? (uint32_t)(v >> 32) : (uint32_t)v);
+        }
+    }
 }
 // Calls f(i) for the entries of a queue, a turn's lanes together.
 template <QueueKind KIND, bool MULTI, int NT, class F>
 GPR_D void for_each_entry(const RenderArgs& a, uint32_t bounce, uint32_t* cursor, F&& f) {
-    const SegWalk w = seg_walk<KIND, MULTI>(a, bounce, gridDim.x * (NT / 64));
+    SegWalk w;
+    seg_counts<KIND, MULTI>(a, bounce, w);
+    w.init(a.seg_cap, turn_log(w.total(), gridDim.x * (NT / 64), a.chunk_log));
     for_each_turn<NT, !MULTI>(cursor, w.turns, [&](uint32_t turn) {
         uint32_t begin, end;
         w.range(turn, begin, end);
@@ -427,7 +436,8 @@ GPR_D void refill_loop(const RenderArgs& a, uint32_t bounce, uint32_t* cursor, B
     const int lane = threadIdx.x & 63;
     // whole turns only: a pool feeds all lanes of its wave
     SegWalk w;
-    w.init(seg_count<KIND, MULTI>(a, bounce), KIND == kPrimary ? 1u : a.nseg, a.seg_cap, a.chunk_log);
+    seg_counts<KIND, MULTI>(a, bounce, w);
+    w.init(a.seg_cap, a.chunk_log);
     uint32_t pb = 0, pe = 0;  // wave-local pool of entries (wave-uniform)
     bool drained = false;
     bool active = false;
@@ -479,17 +489,28 @@ GPR_D Ray3 queue_ray(const QueueView& q, uint32_t i) {
 
 // After the closest hit of entry i: for scattered rays the BSDF-sampling MIS
 // term and, in reference RNG mode, its roulette (pathtracer_kernel.h:684-749).
+// The term waits in the entry for the next bounce's shading or k_flush
+// (tmin = kMisTerm marks it): the shadow rays of the same bounce add theirs
+// meanwhile, and a path's terms keep the order light sample, BSDF sample.  It
+// replaces the origin, which only a miss reads, or the t, u, v of a miss that
+// the roulette made of a hit.
+constexpr float kMisTerm = -1.f;
+GPR_D c3 mis_term(const float4& o_tmin, const float4& hit) {
+    return __float_as_int(hit.y) != -1 ? C(o_tmin.x, o_tmin.y, o_tmin.z) : C(hit.x, hit.z, hit.w);
+}
 template <bool PRIMARY, bool MULTI>
 GPR_D void extend_finish(const RenderArgs& a, const QueueView& q, uint32_t i, const SceneView& sv, const Ray3& r,
                          gpr_hit h, uint32_t bounce) {
     if (!PRIMARY) {
         const float4 wp = q.w_pdf[i];
-        const uint32_t pw = q.pix[i];
-        const uint32_t pix = pw & 0x7fffffffu;
-        const bool spec = (pw >> 31) != 0;
+        const bool spec = (q.pix[i] >> 31) != 0;
         const c3 w = C(wp.x, wp.y, wp.z);
-        float u_rr = 0.f;
-        if (!MULTI && a.rng_mode == GPR_RNG_REFERENCE) u_rr = lcg_next(q.seed[i]);
+        bool dropped = false;
+        if (!MULTI && a.rng_mode == GPR_RNG_REFERENCE) {
+            // roulette without reweighting; a terminated path is a miss (pathtracer_kernel.h:738-748)
+            const float u_rr = lcg_next(q.seed[i]);
+            dropped = cmax(w) < 1 && bounce > 3 && u_rr < fmax_h(0.05f, 1 - cmax(w));
+        }
         if (h.id != -1 && !spec) {
             const Shade ts = load_shade(sv, (uint32_t)h.id);
             const c3 le = emission_of(sv, ts);
@@ -501,14 +522,18 @@ GPR_D void extend_finish(const RenderArgs& a, const QueueView& q, uint32_t i, co
                 lpdf *= d * d / fabsf(dot3(r.d, lg.ns));
                 const c3 fl = dot3(-r.d, lg.ns) > 0 ? le : C(0.f);
                 const float wgt = power_heur(wp.w, lpdf);
-                add_term(a, pix, w * fl * wgt);
+                const c3 v = w * fl * wgt;
+                if (dropped) {
+                    h.t = v.r;
+                    h.u = v.g;
+                    h.v = v.b;
+                    q.o_tmin[i].w = kMisTerm;
+                } else {
+                    q.o_tmin[i] = make_float4(v.r, v.g, v.b, kMisTerm);
+                }
             }
         }
-        if (!MULTI && a.rng_mode == GPR_RNG_REFERENCE && cmax(w) < 1 && bounce > 3) {
-            // roulette without reweighting; a terminated path is a miss (pathtracer_kernel.h:738-748)
-            const float qq = fmax_h(0.05f, 1 - cmax(w));
-            if (u_rr < qq) h.id = -1;
-        }
+        if (dropped) h.id = -1;
     }
     q.hit[i] = make_float4(h.t, __int_as_float(h.id), h.u, h.v);
 }
@@ -525,11 +550,10 @@ GPR_D void shadow_finish(const RenderArgs& a, const QueueView& q, uint32_t i, co
 // REFILL: per-lane ray refill (BVH4 traversal only).
 template <bool PRIMARY, bool REF_ORDER, bool MULTI, int NT, int SL, bool REFILL = false>
 __global__ __launch_bounds__(NT) void k_extend(RenderArgs a, uint32_t bounce) {
-    using Stack = LaneStack<false, NT, SL>;
+    using Stack = LaneStack<false, SL>;
     __shared__ typename Stack::Entry lds[SL * NT];
     Stack st;
-    st.lds = lds + threadIdx.x;
-    st.spill = reinterpret_cast<typename Stack::Entry*>(a.spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal);
+    st.template place<NT>(lds, a.spill);
     // queue: primary = A; at bounce b the scatter queue is q[(b+1)&1]
     const QueueView& q = a.q[PRIMARY ? 0 : ((bounce + 1) & 1)];
     constexpr QueueKind kKind = PRIMARY ? kPrimary : kScatter;
@@ -565,43 +589,95 @@ __global__ __launch_bounds__(NT) void k_extend(RenderArgs a, uint32_t bounce) {
     }
 }
 
-// shadow: any hit + accumulate_light_sampling_contribution (pathtracer_kernel.h:642-664)
-template <bool REF_ORDER, bool MULTI, int NT, int SL, bool REFILL = false>
+// shadow: any hit + accumulate_light_sampling_contribution
+// (pathtracer_kernel.h:642-664), with per-lane ray refill.
+template <int NT, int SL>
 __global__ __launch_bounds__(NT) void k_shadow(RenderArgs a, uint32_t bounce) {
-    using Stack = LaneStack<true, NT, SL>;
+    using Stack = LaneStack<true, SL>;
     __shared__ typename Stack::Entry lds[SL * NT];
     Stack st;
-    st.lds = lds + threadIdx.x;
-    st.spill = reinterpret_cast<typename Stack::Entry*>(a.spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal);
+    st.template place<NT>(lds, a.spill);
     const QueueView& q = a.q[2];
-    uint32_t* cur = &a.ctrl->sh_cursor[bounce];
-    if constexpr (REFILL && !REF_ORDER) {
-        uint32_t ei = 0;
-        SceneView sv;
-        Trav t;
-        refill_loop<kShadow, MULTI>(
-            a, bounce, cur,
-            [&](uint32_t i) {
-                ei = i;
-                sv = scene_of<MULTI>(a, q, i);
-                trav_begin<true>(sv, queue_ray(q, i), st, t);
-                if (trav_live(sv, t)) return false;
-                shadow_finish(a, q, i, t.hit);
-                return true;
-            },
-            [&]() {
-                trav_step<true>(sv, st, t);
-                if (trav_live(sv, t)) return false;
-                if (t.node != kTravDone) atomicOr(&a.ctrl->error, 1u);
-                shadow_finish(a, q, ei, t.hit);
-                return true;
-            });
-    } else {
-        for_each_entry<kShadow, MULTI, NT>(a, bounce, cur, [&](uint32_t i) {
-            const SceneView sv = scene_of<MULTI>(a, q, i);
-            const gpr_hit h = trace_one<true, REF_ORDER>(a, sv, queue_ray(q, i), st);
-            shadow_finish(a, q, i, h);
+    uint32_t ei = 0;
+    SceneView sv;
+    Trav t;
+    refill_loop<kShadow, true>(
+        a, bounce, &a.ctrl->sh_cursor[bounce],
+        [&](uint32_t i) {
+            ei = i;
+            sv = scene_of<true>(a, q, i);
+            trav_begin<true>(sv, queue_ray(q, i), st, t);
+            if (trav_live(sv, t)) return false;
+            shadow_finish(a, q, i, t.hit);
+            return true;
+        },
+        [&]() {
+            trav_step<true>(sv, st, t);
+            if (trav_live(sv, t)) return false;
+            if (t.node != kTravDone) atomicOr(&a.ctrl->error, 1u);
+            shadow_finish(a, q, ei, t.hit);
+            return true;
         });
+}
+
+// The scattered rays of a bounce (closest hit) and its shadow rays (any hit) in
+// one launch: bound by the latency of the walks, and each launch ends in a tail
+// of a few long ones; here the tails overlap, and a bounce has one boundary
+// less.  Scattered rays come first, their walks are longer.  Two kernels
+// against one: a 1280x720 reference-RNG frame of depth 8 2332 -> 2082 us, 16
+// samples of the textured scene (362,000 pixels) 3.80 -> 3.55 ms, a 12-job batch
+// 55.6 -> 48.6 ms, 16 served jobs 177 -> 158 ms.
+template <bool REF_ORDER, bool MULTI, int NT, int SL>
+__global__ __launch_bounds__(NT) void k_trace(RenderArgs a, uint32_t bounce) {
+    __shared__ uint2 lds[SL * NT];
+    const QueueView& qx = a.q[(bounce + 1) & 1];
+    const QueueView& qs = a.q[2];
+    SegWalk wx, ws;
+    seg_counts<kScatter, MULTI>(a, bounce, wx);
+    seg_counts<kShadow, MULTI>(a, bounce, ws);
+    const uint32_t lg = turn_log(wx.total() + ws.total(), gridDim.x * (NT / 64), a.chunk_log);
+    wx.init(a.seg_cap, lg);
+    ws.init(a.seg_cap, lg);
+    for_each_turn<NT, !MULTI>(&a.ctrl->ext_cursor[bounce + 1], wx.turns + ws.turns, [&](uint32_t turn) {
+        uint32_t begin, end;
+        if (turn < wx.turns) {
+            LaneStack<false, SL> st;
+            st.template place<NT>(lds, a.spill);
+            wx.range(turn, begin, end);
+            for (uint32_t i = begin + (threadIdx.x & 63); i < end; i += 64) {
+                const SceneView sv = scene_of<MULTI>(a, qx, i);
+                const Ray3 r = queue_ray(qx, i);
+                const gpr_hit h = trace_one<false, REF_ORDER>(a, sv, r, st);
+                extend_finish<false, MULTI>(a, qx, i, sv, r, h, bounce);
+            }
+        } else {
+            LaneStack<true, 2 * SL> st;  // half the entry, twice the entries
+            st.template place<NT>(lds, a.spill);
+            ws.range(turn - wx.turns, begin, end);
+            for (uint32_t i = begin + (threadIdx.x & 63); i < end; i += 64) {
+                const SceneView sv = scene_of<MULTI>(a, qs, i);
+                const gpr_hit h = trace_one<true, REF_ORDER>(a, sv, queue_ray(qs, i), st);
+                shadow_finish(a, qs, i, h);
+            }
+        }
+    });
+}
+
+// Adds the BSDF-sampling terms that the last bounce's scattered rays left.
+template <bool MULTI>
+__global__ __launch_bounds__(256) void k_flush(RenderArgs a) {
+    const uint32_t bounce = a.depth - 1;
+    const QueueView& q = a.q[a.depth & 1];
+    SegWalk w;
+    seg_counts<kScatter, MULTI>(a, bounce, w);
+    w.init(a.seg_cap, 8);
+    for (uint32_t turn = blockIdx.x; turn < w.turns; turn += gridDim.x) {
+        uint32_t begin, end;
+        w.range(turn, begin, end);
+        const uint32_t i = begin + threadIdx.x;
+        if (i >= end) continue;
+        const float4 o = q.o_tmin[i];
+        if (o.w == kMisTerm) add_term(a, q.pix[i] & 0x7fffffffu, mis_term(o, q.hit[i]));
     }
 }
 
@@ -642,8 +718,9 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
         constexpr uint32_t kLog = 8;
         static_assert(kShadeBlock == 1 << kLog, "a turn is a block");
         SegWalk w;
-        if (bounce == 0) w.init(npaths_of<MULTI>(a), 1, 0, kLog);
-        else w.init(seg_count<kScatter, MULTI>(a, bounce - 1), a.nseg, a.seg_cap, kLog);
+        if (bounce == 0) seg_counts<kPrimary, MULTI>(a, 0, w);
+        else seg_counts<kScatter, MULTI>(a, bounce - 1, w);
+        w.init(a.seg_cap, kLog);
         tile = blockIdx.x;
         if (tile >= w.turns) return;
         w.range(tile, i, n_end);
@@ -662,6 +739,10 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
             sv = ldg(a.scenes + (job >> kJobBits));
             // a job's paths stop at its own depth
             valid = bounce < pj.j.max_depth;
+            if (!valid) {
+                const float4 o = qi.o_tmin[i];
+                if (o.w == kMisTerm) add_term(a, qi.pix[i] & 0x7fffffffu, C(o.x, o.y, o.z));
+            }
             rr_start = pj.j.rr_start;
             const uint32_t word = qi.pix[i] & 0x7fffffffu;
             lpix = word - pj.j.fb_off;
@@ -703,6 +784,12 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
             for (int k = 0; k < 8; ++k) smp[k] = pcg_unit(s, inc);
             rng_out = s;
         }
+        if constexpr (ORDERED) {
+            if (bounce != 0) {
+                const float4 o = qi.o_tmin[i];
+                if (o.w == kMisTerm) add_term(a, pix, mis_term(o, hh));
+            }
+        }
         if (hid != -1) {
             const uint32_t t = (uint32_t)hid;
             const Shade ts = load_shade(sv, t);
@@ -717,6 +804,10 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
                     const c3 fl = dot3(wo, g.ns) > 0 ? le : C(0.f);
                     add_term(a, pix, w * fl);
                 }
+            } else if (!ORDERED && !black(loadc(m.emission))) {
+                // a light met by a non-specular scattered ray: k_trace left its MIS term
+                const float4 o = qi.o_tmin[i];
+                add_term(a, pix, C(o.x, o.y, o.z));
             }
             if (!bsdf_is_delta(m) && sv.nlights > 0) {
                 // sample_lights (pathtracer_kernel.h:323-336): uniform by count, uniform on the triangle
@@ -958,14 +1049,16 @@ constexpr uint64_t kPassBytes = 6ull << 30;   // its queues and term lists at mo
 namespace {
 struct PassKernels {
     void (*ext_primary)(RenderArgs, uint32_t);
-    void (*ext_scatter)(RenderArgs, uint32_t);
+    void (*trace)(RenderArgs, uint32_t);   // scattered and shadow rays, or the scattered ones where shadow is not null
     void (*shadow)(RenderArgs, uint32_t);
     int nt, sl, layout;
 };
 template <int NT, int SL, bool R>
 PassKernels pass_kernels() {
-    return {k_extend<true, false, true, NT, SL, R>, k_extend<false, false, true, NT, SL, R>,
-            k_shadow<false, true, NT, SL, R>, NT, SL, 0};
+    if constexpr (R)
+        return {k_extend<true, false, true, NT, SL, true>, k_extend<false, false, true, NT, SL, true>,
+                k_shadow<NT, SL>, NT, SL, 0};
+    else return {k_extend<true, false, true, NT, SL>, k_trace<false, true, NT, SL>, nullptr, NT, SL, 0};
 }
 const PassKernels& pass_kernel_table(int idx) {
     static const PassKernels t[] = {
@@ -977,8 +1070,7 @@ const PassKernels& pass_kernel_table(int idx) {
         pass_kernels<128, 8, true>(),   pass_kernels<128, 16, true>(),  pass_kernels<128, 32, true>(),
         pass_kernels<256, 8, true>(),   pass_kernels<256, 16, true>(),  pass_kernels<256, 32, true>(),
         pass_kernels<512, 8, true>(),   pass_kernels<512, 16, true>(),  pass_kernels<512, 32, true>(),
-        {k_extend<true, true, true, 256, 16>, k_extend<false, true, true, 256, 16>, k_shadow<true, true, 256, 16>,
-         256, 16, 1},
+        {k_extend<true, true, true, 256, 16>, k_trace<true, true, 256, 16>, nullptr, 256, 16, 1},
     };
     return t[idx];
 }
@@ -1087,7 +1179,7 @@ int engine_create(int device, uint32_t capacity, uint32_t max_jobs, Engine** out
     for (int k = 0; k < kPassKernelCount; ++k) {
         const PassKernels& pk = pass_kernel_table(k);
         int per_cu = 0;
-        GPR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pk.ext_scatter, pk.nt, 0));
+        GPR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pk.trace, pk.nt, 0));
         // more persistent threads than queue entries would only idle
         e->grid[k] = std::max(1, std::min<int>(cus * std::max(1, per_cu), (int)div_up(capacity, pk.nt)));
         threads = std::max(threads, (size_t)e->grid[k] * pk.nt);
@@ -1153,9 +1245,10 @@ int record_pass(Engine* e, uint32_t depth, int kidx, uint32_t chunk, uint32_t si
     hipLaunchKernelGGL(pk.ext_primary, tg, tb, 0, st, a, 0u);
     for (uint32_t b = 0; b < depth; ++b) {
         hipLaunchKernelGGL((k_shade<true, false>), dim3(shade_blocks(size, sg.nseg)), dim3(kShadeBlock), 0, st, a, b);
-        hipLaunchKernelGGL(pk.shadow, tg, tb, 0, st, a, b);
-        hipLaunchKernelGGL(pk.ext_scatter, tg, tb, 0, st, a, b);
+        if (pk.shadow) hipLaunchKernelGGL(pk.shadow, tg, tb, 0, st, a, b);
+        hipLaunchKernelGGL(pk.trace, tg, tb, 0, st, a, b);
     }
+    hipLaunchKernelGGL(k_flush<true>, dim3(std::min(1024u, div_up(size, 256))), dim3(256), 0, st, a);
     if (terms) hipLaunchKernelGGL(k_accum<true>, dim3(div_up(size, 256)), dim3(256), 0, st, a);
     GPR_HIP(hipGetLastError());
     return GPR_OK;
@@ -1454,7 +1547,7 @@ RenderArgs make_args(gpr_renderer* r, uint32_t log_s) {
 // textured scene 5.03 / 4.85 / 4.88 ms, 4 of the sphere grid 16.7 / 16.7 / 17.1.
 constexpr int kRenderNT = 256, kRenderSL = 12;
 
-// One pass of 2^log_s samples: gen -> extend(primary) -> max_depth x {shade, shadow, extend} -> accum -> finish.
+// One pass of 2^log_s samples: gen -> extend(primary) -> max_depth x {shade, trace} -> flush -> accum -> finish.
 int launch_pass(gpr_renderer* r, uint32_t log_s, hipStream_t st) {
     const RenderArgs a = make_args(r, log_s);
     const bool ref = r->opts.traversal == GPR_TRAVERSAL_REF;
@@ -1469,14 +1562,10 @@ int launch_pass(gpr_renderer* r, uint32_t log_s, hipStream_t st) {
             hipLaunchKernelGGL((k_shade<false, true>), dim3(div_up(a.npix, kShadeBlock)), dim3(kShadeBlock), 0, st, a, b);
         else
             hipLaunchKernelGGL((k_shade<false, false>), dim3(shade_blocks(a.npix, a.nseg)), dim3(kShadeBlock), 0, st, a, b);
-        if (ref) {
-            hipLaunchKernelGGL((k_shadow<true, false, NT, SL>), tg, tb, 0, st, a, b);
-            hipLaunchKernelGGL((k_extend<false, true, false, NT, SL>), tg, tb, 0, st, a, b);
-        } else {
-            hipLaunchKernelGGL((k_shadow<false, false, NT, SL>), tg, tb, 0, st, a, b);
-            hipLaunchKernelGGL((k_extend<false, false, false, NT, SL>), tg, tb, 0, st, a, b);
-        }
+        if (ref) hipLaunchKernelGGL((k_trace<true, false, NT, SL>), tg, tb, 0, st, a, b);
+        else hipLaunchKernelGGL((k_trace<false, false, NT, SL>), tg, tb, 0, st, a, b);
     }
+    if (a.depth) hipLaunchKernelGGL(k_flush<false>, dim3(std::min(1024u, div_up(a.npix, 256))), dim3(256), 0, st, a);
     if (log_s) hipLaunchKernelGGL(k_accum<false>, dim3(div_up(r->npix, 256)), dim3(256), 0, st, a);
     hipLaunchKernelGGL(k_finish, dim3(1), dim3(64), 0, st, a.ctrl, 1u << log_s);
     GPR_HIP(hipGetLastError());
@@ -1583,7 +1672,7 @@ int renderer_alloc(gpr_renderer* r) {
     }
     int cus = 0, per_cu = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->device) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_extend<false, false, false, kRenderNT, kRenderSL>,
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_trace<false, false, kRenderNT, kRenderSL>,
                                                      kRenderNT, 0) != hipSuccess)
         return fail(GPR_ERR_HIP, "occupancy query failed");
     r->grid_trace = std::max(1, cus * std::max(1, per_cu));

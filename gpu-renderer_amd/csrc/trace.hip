@@ -47,11 +47,10 @@ __global__ __launch_bounds__(NT) void k_trace_fast(SceneView sv, const gpr_ray* 
                                                    gpr_hit* __restrict__ hits, uint64_t n,
                                                    unsigned long long* __restrict__ cursor,
                                                    int2* __restrict__ spill, uint32_t chunk_log) {
-    using Stack = LaneStack<ANY, NT, SL>;
+    using Stack = LaneStack<ANY, SL>;
     __shared__ typename Stack::Entry lds[SL * NT];
     Stack st;
-    st.lds = lds + threadIdx.x;
-    st.spill = reinterpret_cast<typename Stack::Entry*>(spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal);
+    st.template place<NT>(lds, spill);
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t lg = turn_log(n, gridDim.x * (NT / 64), chunk_log);
     for_each_turn<NT, false>(cursor, (n + (1ull << lg) - 1) >> lg, [&](uint64_t turn) {
@@ -83,11 +82,10 @@ __global__ __launch_bounds__(NT) void k_trace_refill(SceneView sv, const gpr_ray
                                                      gpr_hit* __restrict__ hits, uint64_t n,
                                                      unsigned long long* __restrict__ cursor,
                                                      int2* __restrict__ spill, uint32_t chunk_log) {
-    using Stack = LaneStack<ANY, NT, SL>;
+    using Stack = LaneStack<ANY, SL>;
     __shared__ typename Stack::Entry lds[SL * NT];
     Stack st;
-    st.lds = lds + threadIdx.x;
-    st.spill = reinterpret_cast<typename Stack::Entry*>(spill + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal);
+    st.template place<NT>(lds, spill);
     const int lane = threadIdx.x & 63;
     // wave-local pool [pb, pe) of ray indices (wave-uniform); the first one is
     // dealt out, thin where the batch is short, the others are claimed
@@ -199,11 +197,10 @@ template <bool ANY>
 __global__ __launch_bounds__(256) void k_trace_stats(SceneView sv, const gpr_ray* __restrict__ rays, uint64_t n,
                                                      unsigned long long* __restrict__ stats,
                                                      int2* __restrict__ spill) {
-    using Stack = LaneStack<ANY, 256, 16>;
+    using Stack = LaneStack<ANY, 16>;
     __shared__ typename Stack::Entry lds[16 * 256];
     Stack st;
-    st.lds = lds + threadIdx.x;
-    st.spill = reinterpret_cast<typename Stack::Entry*>(spill + (uint64_t)(blockIdx.x * 256 + threadIdx.x) * kStackGlobal);
+    st.template place<256>(lds, spill);
     unsigned long long nf = 0, nt = 0, ov = 0;
     for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) {
         Trav t;

@@ -117,31 +117,37 @@ GPR_D gpr_hit ref_trace(const SceneView& sv, Ray3 r, uint32_t* nvisit, uint32_t*
 }
 
 // ------------------------------------------------------ BVH4 traversal ---
-// Per-lane traversal stack: the oldest SL entries in an LDS column of a block
-// of NT lanes (entry k at lds[k * NT]), the rest in a per-lane global slab of
-// kStackGlobal entries (walks rarely reach it).  Entry 0 is a sentinel that
+// Per-lane traversal stack: the oldest SL entries in an LDS column of the wave's
+// own part of the block's LDS (entry k at lds[k * 64]), the rest in a per-lane
+// global slab of kStackGlobal entries (walks rarely reach it).  Entry 0 is a sentinel that
 // every pop accepts and that ends the walk, so popping needs no empty test.
 // Closest hit keeps 8 bytes per entry (the order key and the child), any hit
 // only the child.
-template <class E, int NT, int SL>
+template <class E, int SL>
 struct LaneStackT {
-    static constexpr int kNT = NT, kSL = SL;
     using Entry = E;
+    static constexpr int kStride = 64;
     E* lds;    // this lane's column
     E* spill;  // this lane's overflow area (kStackGlobal entries)
     int sp;
+    // block_lds: SL entries a lane; overflow: kStackGlobal int2 a lane of the grid
+    template <int NT>
+    GPR_D void place(void* block_lds, int2* overflow) {
+        lds = static_cast<E*>(block_lds) + (threadIdx.x / 64) * (SL * 64) + (threadIdx.x & 63);
+        spill = reinterpret_cast<E*>(overflow + (uint64_t)(blockIdx.x * NT + threadIdx.x) * kStackGlobal);
+    }
     GPR_D void reset(E sentinel) {
         lds[0] = sentinel;
         sp = 1;
     }
     GPR_D void put(int at, E e) {
-        if (at < SL) lds[at * NT] = e;
+        if (at < SL) lds[at * kStride] = e;
         else spill[at - SL] = e;
     }
     GPR_D E pop() {
         --sp;
         if (sp >= SL) return spill[sp - SL];
-        return lds[sp * NT];
+        return lds[sp * kStride];
     }
     // true when no active lane of the wave could leave the LDS part by pushing k entries
     GPR_D bool roomy(int k) const { return __ballot(sp + k > SL) == 0ull; }
@@ -157,8 +163,8 @@ template <>
 struct StackEntry<true> {
     using type = int32_t;
 };
-template <bool ANY, int NT, int SL>
-using LaneStack = LaneStackT<typename StackEntry<ANY>::type, NT, SL>;
+template <bool ANY, int SL>
+using LaneStack = LaneStackT<typename StackEntry<ANY>::type, SL>;
 
 GPR_D void tri_rec_hit(const TriRec* tris, uint32_t ntri, int32_t leaf, const Ray3& r, float& tmax,
                        gpr_hit& hit, bool& found) {
@@ -318,7 +324,7 @@ GPR_D void trav_descend(Stack& st, Trav& t, const NodeHits& h) {
         // overwritten by the next entry (or left above the top)
 #pragma unroll
         for (int k = 3; k >= 1; --k) {
-            st.lds[st.sp * Stack::kNT] = entry(e[k]);
+            st.lds[st.sp * Stack::kStride] = entry(e[k]);
             st.sp += key_of(e[k]) != kKeyNone ? 1 : 0;
         }
     } else {
@@ -352,7 +358,7 @@ GPR_D void trav_descend_any(Stack& st, Trav& t, const NodeHits& h) {
     if (st.roomy(3)) {
 #pragma unroll
         for (int c = 3; c >= 0; --c) {
-            if (c < 3) st.lds[st.sp * Stack::kNT] = next;
+            if (c < 3) st.lds[st.sp * Stack::kStride] = next;
             st.sp += (c < 3 && h.hitc[c] && next >= 0) ? 1 : 0;
             next = h.hitc[c] ? h.ch[c] : next;
         }
@@ -478,7 +484,8 @@ GPR_D void for_each_turn(C* cursor, I n, F&& f) {
             if (claimed_from >= n) break;
             C got = 0;
             if ((threadIdx.x & 63) == 0) got = atomicAdd(cursor, (C)1);
-            t = claimed_from + (I)__shfl(got, 0, 64);
+            if constexpr (sizeof(I) == 4) t = claimed_from + __builtin_amdgcn_readfirstlane(got);
+            else t = claimed_from + (I)__shfl(got, 0, 64);
         }
     }
 }

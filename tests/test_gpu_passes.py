@@ -116,3 +116,26 @@ def test_jobs_with_uneven_samples(capacity):
     assert b.stats().paths == sum(w * h * spp for w, h, spp, _ in specs)
     b.free()
     srv.free()
+
+
+@pytest.mark.parametrize("rng_mode", [gpr.RNG_REFERENCE, gpr.RNG_PCG])
+@pytest.mark.parametrize("depth", [4, 5, 6, 12])
+def test_terms_of_paths_that_end_at_a_light(rng_mode, depth):
+    # a grey floor under a grey light the size of the floor, and a sky: scattered rays meet the light at every bounce,
+    # the last one included, and in reference RNG mode the roulette turns some of those hits into misses of the sky
+    from test_gpu_render import gpu_render, oracle_render
+    s = gpr.Scene()
+    for y, e in ((-1.0, 0.0), (1.0, 2.0)):
+        p, uv, c = G._quad([(-3, y, -3), (3, y, -3), (3, y, 3), (-3, y, 3)], [(0, 0), (1, 0), (1, 1), (0, 1)])
+        s.add_mesh(p if y < 0 else p[::-1].copy(), corners=c, uv=uv,
+                   mat=gpr.material(gpr.MAT_DIFFUSE, color=(0.6, 0.5, 0.7), emission=(e, e, e)))
+    s.set_env_map(s.add_texture(np.random.default_rng(1).random((8, 16, 3))), np.eye(4, dtype=np.float32))
+    s.set_camera_lookat((0, 0, 0), (0.5, 0.2, 4.0), (0, 1, 0), 60, 37, 19)
+    s.commit()
+    print(f"[passes] light terms depth {depth} rng {rng_mode}", flush=True)
+    for traversal in (gpr.TRAVERSAL_REF, gpr.TRAVERSAL_FAST):
+        got, cnt, _, _ = gpu_render(s, 5, depth, rng_mode, 3, traversal)
+        want, wcnt = oracle_render(s, 5, depth, rng_mode, 3)
+        assert np.array_equal(cnt, wcnt)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    s.free()
