@@ -8,6 +8,7 @@
 // in the single-scene renderer.
 #pragma once
 
+#include <mutex>
 #include <vector>
 
 #include "gpr_internal.h"
@@ -64,5 +65,12 @@ int engine_run_pass(Engine* e, const EngineJob* jobs, uint32_t njobs, float4* fb
 // Error flags accumulated by the passes so far (bit0 stack overflow, bit1
 // look-back timeout); synchronises st.
 int engine_errors(Engine* e, hipStream_t st, uint32_t* flags);
+
+// Copies frame-buffer pixels of `device` to the host as 12-byte colours, one call at a time.
+struct PixelReader {
+    std::mutex mu;
+    DevBuf scratch;  // packed pixels, 12 MB at most, kept for the next call
+    int read(int device, const float4* fb, uint64_t n, float* rgb, hipStream_t st);
+};
 
 }  // namespace gpr

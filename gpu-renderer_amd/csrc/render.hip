@@ -1024,9 +1024,55 @@ __global__ void k_set_sample(Ctrl* c, uint32_t s) {
     }
 }
 
+constexpr uint64_t kReadPixels = 1ull << 20;  // pixels packed for the host at once
+
+// The three channels of n frame-buffer pixels.
+__global__ __launch_bounds__(256) void k_pack_rgb(const float4* __restrict__ fb, uint32_t n, float* __restrict__ out) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const float4 x = fb[i];
+    out[3ull * i] = x.x;
+    out[3ull * i + 1] = x.y;
+    out[3ull * i + 2] = x.z;
+}
+
 inline uint32_t div_up(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
 }  // namespace
+
+// The pixels are packed on the device and land in the caller's buffer.  Bound by
+// the host's first touch of that buffer: copied as 16-byte pixels to a buffer of
+// their own and repacked by the host, a 1920x1080 image took 10.2 ms, now 3.5
+// (of a render of 4 samples 20.7 -> 14.0 ms in all, 803x451 and 8 samples 3.50
+// -> 3.20).
+int PixelReader::read(int device, const float4* fb, uint64_t n, float* rgb, hipStream_t st) {
+    std::lock_guard<std::mutex> lk(mu);
+    const uint64_t most = std::min<uint64_t>(n, kReadPixels);
+    int now = -1;
+    GPR_HIP(hipGetDevice(&now));
+    if (now != device || scratch.alloc(12 * most) != GPR_OK) {
+        // a thread of another device may not launch on these pixels; or no room for the scratch
+        (void)hipGetLastError();
+        std::vector<float4> tmp(n);
+        GPR_HIP(hipMemcpyAsync(tmp.data(), fb, 16 * n, hipMemcpyDeviceToHost, st));
+        GPR_HIP(hipStreamSynchronize(st));
+        for (uint64_t i = 0; i < n; ++i) {
+            rgb[3 * i] = tmp[i].x;
+            rgb[3 * i + 1] = tmp[i].y;
+            rgb[3 * i + 2] = tmp[i].z;
+        }
+        return GPR_OK;
+    }
+    float* d = scratch.as<float>();
+    for (uint64_t at = 0; at < n; at += most) {
+        const uint32_t m = (uint32_t)std::min<uint64_t>(most, n - at);
+        hipLaunchKernelGGL(k_pack_rgb, dim3(div_up(m, 256)), dim3(256), 0, st, fb + at, m, d);
+        GPR_HIP(hipGetLastError());
+        GPR_HIP(hipMemcpyAsync(rgb + 3 * at, d, 12ull * m, hipMemcpyDeviceToHost, st));
+    }
+    GPR_HIP(hipStreamSynchronize(st));
+    return GPR_OK;
+}
 
 // Multi-sample passes.  A small image (or the
 // late bounces of any image) leaves the chip idle and every launch pays the
@@ -1477,6 +1523,7 @@ struct gpr_renderer {
     uint32_t npix = 0, ntiles = 0;
     uint32_t spp_done = 0;
     DevBuf fb, ctrl, status;
+    PixelReader reader;
     DevBuf seg;              // queue segment counters, then those of the last sample
     uint32_t last_nseg = 1;  // segments of the last pass
     DevBuf qmem[3];
@@ -1841,18 +1888,12 @@ int gpr_render(gpr_renderer* r, uint32_t spp) {
 
 int gpr_renderer_read(gpr_renderer* r, float* rgb, uint32_t* cnt) {
     if (!r) return fail(GPR_ERR_INVALID, "gpr_renderer_read: null renderer");
-    std::vector<float> tmp(4ull * r->npix);
-    GPR_HIP(hipMemcpyAsync(tmp.data(), r->fb.p, 16ull * r->npix, hipMemcpyDeviceToHost, stream()));
-    GPR_HIP(hipStreamSynchronize(stream()));
-    for (uint64_t i = 0; i < r->npix; ++i) {
-        if (rgb) {
-            rgb[3 * i + 0] = tmp[4 * i + 0];
-            rgb[3 * i + 1] = tmp[4 * i + 1];
-            rgb[3 * i + 2] = tmp[4 * i + 2];
-        }
-        if (cnt) cnt[i] = r->spp_done;
+    if (cnt) std::fill_n(cnt, r->npix, r->spp_done);
+    if (!rgb) {
+        GPR_HIP(hipStreamSynchronize(stream()));
+        return GPR_OK;
     }
-    return GPR_OK;
+    return r->reader.read(r->scene->device, r->fb.as<float4>(), r->npix, rgb, stream());
 }
 
 int gpr_renderer_queue_sizes(gpr_renderer* r, uint32_t* shadow, uint32_t* scatter, uint32_t cap) {

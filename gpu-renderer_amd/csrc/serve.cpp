@@ -182,6 +182,7 @@ struct gpr_batch {
     std::vector<EngineJob> jobs;
     std::vector<uint32_t> spp;
     DevBuf fb;
+    PixelReader reader;
     uint64_t fb_pixels = 0;
     bool fb_ready = false;
     TraceCfg cfg{256, 16, 64, 0, 0};
@@ -331,15 +332,7 @@ int gpr_batch_run(gpr_batch* b) {
 int gpr_batch_read(gpr_batch* b, uint32_t job, float* rgb) {
     if (!b || !rgb || job >= b->jobs.size() || !b->fb_ready) return fail(GPR_ERR_INVALID, "gpr_batch_read: bad argument");
     const EngineJob& j = b->jobs[job];
-    std::vector<float> tmp(4ull * j.npix);
-    GPR_HIP(hipMemcpyAsync(tmp.data(), b->fb.as<float4>() + j.fb_off, 16ull * j.npix, hipMemcpyDeviceToHost, stream()));
-    GPR_HIP(hipStreamSynchronize(stream()));
-    for (uint64_t i = 0; i < j.npix; ++i) {
-        rgb[3 * i + 0] = tmp[4 * i + 0];
-        rgb[3 * i + 1] = tmp[4 * i + 1];
-        rgb[3 * i + 2] = tmp[4 * i + 2];
-    }
-    return GPR_OK;
+    return b->reader.read(b->device, b->fb.as<float4>() + j.fb_off, j.npix, rgb, stream());
 }
 
 int gpr_batch_get_stats(const gpr_batch* b, gpr_batch_stats* out) {
