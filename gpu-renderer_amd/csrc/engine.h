@@ -54,6 +54,11 @@ int engine_set_scenes(Engine* e, const std::vector<SceneView>& views, hipStream_
 // instead.
 void engine_limit_terms(Engine* e, uint64_t bytes);
 int engine_reserve_terms(Engine* e, uint64_t bytes);
+// Large passes run as two parts side by side; the second one's traversal stacks
+// overflow to an area of their own.  engine_limit_terms lets it be allocated on
+// use; engine_reserve_side allocates it (engine_side_bytes) at once.
+uint64_t engine_side_bytes(const Engine* e);
+int engine_reserve_side(Engine* e);
 // Gives every job as many samples as the pass has room for: jobs hold one
 // sample each (log_s 0) on entry, left[k] is how many job k has left (>= 1).
 // st is the stream of the passes.

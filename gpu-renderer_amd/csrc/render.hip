@@ -92,6 +92,18 @@ Segs segs_for(uint32_t paths, bool tight) {
     s.cap = s.nseg == 1 ? paths : (groups + s.nseg - 1) / s.nseg * kSegGroup * kShadeBlock;
     return s;
 }
+// A large pass runs as two parts, each a chain of launches of its own over half
+// of the paths, side by side.  The traversal kernels hold the whole chip until
+// their queue is dealt out and then wait for their longest walks (CUs were busy
+// 79 % of a launch); the other part's next kernel takes the blocks that come
+// free.  One part against two: a batch of 12 scenes 45.6 -> 41.9 ms, 16 server
+// requests 154 -> 137 ms (passes of 2^22 paths); 4 samples of the 1920x1080
+// sphere grid 13.9 -> 13.5 ms in all, 8 of the textured scene (2.9M paths) 3.29
+// -> 3.20.  A pass of 2^20 paths is too short: 16 samples of the 256x256 Cornell
+// box 1.39 -> 1.43 ms.  In the engine (`tight`) parts also take queue slack of
+// their own, below 2 bytes a path from the size given.
+constexpr uint32_t kMaxParts = 2;
+constexpr uint32_t parts_for(uint32_t paths, bool tight) { return paths >= (tight ? 5u << 18 : 1u << 21) ? kMaxParts : 1u; }
 // 64-bit words between two segments' counters, and of all counters
 GPR_HD constexpr uint32_t seg_stride(uint32_t nseg) { return nseg > 1 ? 16u : 1u; }
 constexpr uint32_t seg_words(uint32_t nseg) { return kMaxBounce * nseg * seg_stride(nseg); }
@@ -117,10 +129,12 @@ struct RenderArgs {
     const PassBuf* pass;       // multi-job passes: jobs of this pass
     QueueView q[3];            // A, B (in/scatter alternate), S (shadow)
     float4* fb;
-    Ctrl* ctrl;
+    Ctrl* ctrl;                // cursors of this part of the pass
+    Ctrl* base;                // sample and error flags of the pass
     unsigned long long* status;  // [kMaxBounce][ntiles] look-back words
     int2* spill;
-    uint32_t npix;             // single-scene: paths per sample
+    uint32_t paths;            // single-scene: paths of the pass
+    uint32_t parts, part;      // the pass runs as one chain of launches or as two, this is one of them
     uint32_t ntiles;           // look-back words per bounce (capacity / kShadeBlock)
     uint32_t nseg, seg_cap;    // segments of the shadow and scatter queues
     unsigned long long* seg;   // [bounce][segment] entries appended: shadow << 32 | scatter
@@ -140,10 +154,23 @@ struct RenderArgs {
 GPR_D unsigned long long* seg_at(const RenderArgs& a, uint32_t bounce, uint32_t g) {
     return a.seg + (bounce * a.nseg + g) * seg_stride(a.nseg);
 }
+// Paths of a pass before part `part` of `parts`.
+GPR_HD constexpr uint32_t part_begin(uint32_t n, uint32_t parts, uint32_t part) {
+    if (part == 0) return 0;
+    const uint32_t half = ((n + 1) / 2 + kShadeBlock - 1) / kShadeBlock * kShadeBlock;  // no later part is larger
+    return part < parts && half < n ? half : n;
+}
+template <bool MULTI>
+GPR_D uint32_t first_path_of(const RenderArgs& a) {
+    if constexpr (MULTI) return part_begin(a.pass->npaths, a.parts, a.part);
+    else return part_begin(a.paths, a.parts, a.part);
+}
 template <bool MULTI>
 GPR_D uint32_t npaths_of(const RenderArgs& a) {
-    if constexpr (MULTI) return a.pass->npaths;
-    else return a.npix;
+    uint32_t n;
+    if constexpr (MULTI) n = a.pass->npaths;
+    else n = a.paths;
+    return part_begin(n, a.parts, a.part + 1) - part_begin(n, a.parts, a.part);
 }
 // Multi-job queue entries carry scene << kJobBits | pass job, so the kernels
 // that only need the scene (traversal) index the scene table directly.
@@ -223,7 +250,8 @@ template <bool MULTI>
 __global__ __launch_bounds__(256) void k_gen(RenderArgs a) {
     const uint32_t tid = blockIdx.x * 256 + threadIdx.x;
     const uint32_t gsz = gridDim.x * 256;
-    const uint32_t npix = npaths_of<MULTI>(a);
+    const uint32_t n = npaths_of<MULTI>(a);
+    const uint32_t path = first_path_of<MULTI>(a) + tid;  // in the slot order of the pass
     // clear the per-sample counters, cursors and the look-back words this sample uses
     Ctrl* c = a.ctrl;
     for (uint32_t i = tid; i < kMaxBounce; i += gsz) {
@@ -238,25 +266,25 @@ __global__ __launch_bounds__(256) void k_gen(RenderArgs a) {
     for (uint32_t i = tid; i < kMaxBounce * a.nseg; i += gsz) a.seg[i * seg_stride(a.nseg)] = 0ull;
     if (tid == 0) c->ext_cursor[0] = 0u;
     if (!MULTI && a.rng_mode == GPR_RNG_REFERENCE) {
-        const uint32_t used_tiles = (npix + kShadeBlock - 1) / kShadeBlock;
+        const uint32_t used_tiles = (n + kShadeBlock - 1) / kShadeBlock;
         const uint64_t nstat = (uint64_t)a.depth * used_tiles;
         for (uint64_t i = tid; i < nstat; i += gsz) a.status[(i / used_tiles) * a.ntiles + i % used_tiles] = 0ull;
     }
-    if (tid >= npix) return;
+    if (tid >= n) return;
     const QueueView& q = a.q[0];
     if constexpr (MULTI) {
-        // the job holding path tid: last job whose path_off <= tid
+        // the job holding the path: last job whose path_off <= path
         const PassBuf* pb = a.pass;
         uint32_t lo = 0, hi = pb->njobs;
         while (hi - lo > 1) {
             const uint32_t mid = (lo + hi) >> 1;
-            if (pb->jobs[mid].path_off <= tid) lo = mid;
+            if (pb->jobs[mid].path_off <= path) lo = mid;
             else hi = mid;
         }
         const EngineJob& jb = pb->jobs[lo].j;
         const uint32_t off = pb->jobs[lo].path_off;
-        const uint32_t lp = slot_pixel((tid - off) >> jb.log_s, jb.width, jb.npix);
-        const uint32_t sub = (tid - off) & ((1u << jb.log_s) - 1u);
+        const uint32_t lp = slot_pixel((path - off) >> jb.log_s, jb.width, jb.npix);
+        const uint32_t sub = (path - off) & ((1u << jb.log_s) - 1u);
         uint32_t word = jb.fb_off + lp;
         if (a.terms) {
             word = off + (lp << jb.log_s | sub);
@@ -279,9 +307,9 @@ __global__ __launch_bounds__(256) void k_gen(RenderArgs a) {
     } else {
         const uint32_t W = a.sv.width;
         // reference RNG mode indexes its seeds by slot: slot order = pixel order
-        const uint32_t lpix = a.rng_mode == GPR_RNG_REFERENCE ? tid : slot_pixel(tid >> a.log_s, W, npix >> a.log_s);
-        const uint32_t sub = tid & ((1u << a.log_s) - 1u);
-        const uint32_t sample = c->sample + sub;
+        const uint32_t lpix = a.rng_mode == GPR_RNG_REFERENCE ? tid : slot_pixel(path >> a.log_s, W, a.paths >> a.log_s);
+        const uint32_t sub = path & ((1u << a.log_s) - 1u);
+        const uint32_t sample = a.base->sample + sub;
         const uint32_t x = lpix % W, y = lpix / W;
         float jx, jy;
         if (a.rng_mode == GPR_RNG_REFERENCE) {
@@ -302,9 +330,9 @@ __global__ __launch_bounds__(256) void k_gen(RenderArgs a) {
         q.o_tmin[tid] = make_float4(o.x, o.y, o.z, 0.f);
         q.d_tmax[tid] = make_float4(d.x, d.y, d.z, 1e34f);
         q.w_pdf[tid] = make_float4(1.f, 1.f, 1.f, 0.f);
-        const uint32_t path = (lpix << a.log_s) | sub;
-        q.pix[tid] = path;
-        if (a.terms) a.nterm[path] = 0;
+        const uint32_t word = (lpix << a.log_s) | sub;
+        q.pix[tid] = word;
+        if (a.terms) a.nterm[word] = 0;
     }
 }
 
@@ -315,7 +343,7 @@ GPR_D gpr_hit trace_one(const RenderArgs& a, const SceneView& sv, const Ray3& r,
         uint32_t nv = 0, nt = 0;
         h = ref_trace<ANY>(sv, r, &nv, &nt);
     } else {
-        if (!fast_trace<ANY>(sv, r, st, h)) atomicOr(&a.ctrl->error, 1u);
+        if (!fast_trace<ANY>(sv, r, st, h)) atomicOr(&a.base->error, 1u);
     }
     return h;
 }
@@ -575,7 +603,7 @@ __global__ __launch_bounds__(NT) void k_extend(RenderArgs a, uint32_t bounce) {
             [&]() {
                 trav_step<false>(sv, st, t);
                 if (trav_live(sv, t)) return false;
-                if (t.node != kTravDone) atomicOr(&a.ctrl->error, 1u);
+                if (t.node != kTravDone) atomicOr(&a.base->error, 1u);
                 extend_finish<PRIMARY, MULTI>(a, q, ei, sv, t.r, t.hit, bounce);
                 return true;
             });
@@ -614,7 +642,7 @@ __global__ __launch_bounds__(NT) void k_shadow(RenderArgs a, uint32_t bounce) {
         [&]() {
             trav_step<true>(sv, st, t);
             if (trav_live(sv, t)) return false;
-            if (t.node != kTravDone) atomicOr(&a.ctrl->error, 1u);
+            if (t.node != kTravDone) atomicOr(&a.base->error, 1u);
             shadow_finish(a, q, ei, t.hit);
             return true;
         });
@@ -765,7 +793,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
         pix = pw & 0x7fffffffu;
         if constexpr (!MULTI) {
             lpix = pix >> a.log_s;
-            sample = a.ctrl->sample + (pix & ((1u << a.log_s) - 1u));
+            sample = a.base->sample + (pix & ((1u << a.log_s) - 1u));
         }
         const bool spec = (pw >> 31) != 0;
         const v3 rd = V(dt.x, dt.y, dt.z);
@@ -931,7 +959,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
                 if (f == 0) {
                     // predecessor tiles took their ids earlier and are resident: this wait ends
                     if (++spins > (1u << 26)) {
-                        atomicOr(&a.ctrl->error, 2u);
+                        atomicOr(&a.base->error, 2u);
                         break;
                     }
                     __builtin_amdgcn_s_sleep(1);
@@ -997,7 +1025,7 @@ __global__ __launch_bounds__(256) void k_accum(RenderArgs a) {
         fbi = jb.fb_off + lp;
         if (jb.sample != 0) x = a.fb[fbi];
     } else {
-        if (p >= (a.npix >> log_s)) return;
+        if (p >= (a.paths >> log_s)) return;
         x = a.fb[fbi];
     }
     for (uint32_t j = path; j < path + (1u << log_s); ++j) {
@@ -1146,6 +1174,69 @@ uint32_t queue_entries(uint32_t paths, bool tight) {
     const Segs s = segs_for(paths, tight);
     return std::max(paths, s.nseg * s.cap);
 }
+// Entries of the queues of passes of up to `paths` paths, in one part or two.
+uint32_t pass_entries(uint32_t paths, bool tight) {
+    constexpr uint32_t kSlack = 5120;  // segments hold at most that much beyond their paths
+    if (parts_for(paths, tight) == 1) return queue_entries(paths, tight);
+    return paths + kMaxParts * (kSlack + kShadeBlock);
+}
+QueueView queue_from(QueueView q, uint32_t at) {
+    q.o_tmin += at;
+    q.d_tmax += at;
+    q.hit += at;
+    q.w_pdf += at;
+    q.pix += at;
+    q.rng += at;
+    if (q.job) q.job += at;
+    return q;
+}
+// Sets a pass's arguments up for one of its parts: its share of the queues,
+// counters and cursors, and the stack overflow area `side` of the second one.
+// `paths` is what the launches cover.  Returns what those of a part cover.
+uint32_t set_part(RenderArgs& a, uint32_t paths, uint32_t parts, uint32_t part, bool tight, int2* side) {
+    const uint32_t n = parts == 1 ? paths : part_begin(paths, parts, 1);
+    const Segs sg = a.rng_mode == GPR_RNG_REFERENCE ? Segs{1, n} : segs_for(n, tight);
+    a.parts = parts;
+    a.part = part;
+    a.nseg = sg.nseg;
+    a.seg_cap = sg.cap;
+    if (part) {
+        for (QueueView& q : a.q) q = queue_from(q, queue_entries(n, tight));
+        a.ctrl += 1;
+        a.seg += seg_words(kMaxSegs);
+        if (a.last) a.last += kMaxBounce * kLastSpread;
+        a.spill = side;
+    }
+    return n;
+}
+// The second chain of a pass while it is captured: work on st between fork and
+// join runs beside what is launched on the stream `fork` returns.
+struct SideStream {
+    hipStream_t s = nullptr;
+    hipEvent_t forked = nullptr, joined = nullptr;
+    int make() {
+        if (s) return GPR_OK;
+        if (!forked) GPR_HIP(hipEventCreateWithFlags(&forked, hipEventDisableTiming));
+        if (!joined) GPR_HIP(hipEventCreateWithFlags(&joined, hipEventDisableTiming));
+        GPR_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+        return GPR_OK;
+    }
+    int fork(hipStream_t st) {
+        GPR_HIP(hipEventRecord(forked, st));
+        GPR_HIP(hipStreamWaitEvent(s, forked, 0));
+        return GPR_OK;
+    }
+    int join(hipStream_t st) {
+        GPR_HIP(hipEventRecord(joined, s));
+        GPR_HIP(hipStreamWaitEvent(st, joined, 0));
+        return GPR_OK;
+    }
+    ~SideStream() {
+        if (s) (void)hipStreamDestroy(s);
+        if (forked) (void)hipEventDestroy(forked);
+        if (joined) (void)hipEventDestroy(joined);
+    }
+};
 int alloc_queue(DevBuf& mem, QueueView& q, uint32_t n, bool with_job) {
     const size_t per = 16 * 4 + 4 + 8 + (with_job ? 4 : 0);
     GPR_TRY(mem.alloc((size_t)n * per + 8 * 256));
@@ -1174,6 +1265,9 @@ struct Engine {
     DevBuf qmem[3], ctrl, seg, spill, pass, scenes;
     DevBuf terms, nterm;      // passes of several samples a job
     uint64_t term_limit = 0;  // bytes the term lists may take
+    DevBuf side_spill;        // stack overflow area of a pass's second part
+    bool side_grows = false;  // it is allocated on use
+    SideStream side;
     QueueView q[3];
     int grid[kPassKernelCount] = {};
     hipStream_t cap_stream = nullptr;
@@ -1188,9 +1282,10 @@ struct Engine {
         uint32_t size;  // launch size class: paths rounded up to a power of two
         float4* fb;
         bool terms;     // several samples a job
+        uint32_t parts;
         bool operator==(const GraphKey& o) const {
             return depth == o.depth && kidx == o.kidx && chunk == o.chunk && size == o.size && fb == o.fb &&
-                   terms == o.terms;
+                   terms == o.terms && parts == o.parts;
         }
     };
     std::vector<std::pair<GraphKey, hipGraphExec_t>> graphs;
@@ -1214,10 +1309,11 @@ int engine_create(int device, uint32_t capacity, uint32_t max_jobs, Engine** out
     e->device = device;
     e->capacity = capacity;
     e->max_jobs = max_jobs;
-    for (int k = 0; k < 3; ++k) GPR_TRY(alloc_queue(e->qmem[k], e->q[k], queue_entries(capacity, true), true));
-    GPR_TRY(e->ctrl.alloc(sizeof(Ctrl)));
-    GPR_TRY(e->seg.alloc(8ull * seg_words(segs_for(capacity, true).nseg)));
-    GPR_HIP(hipMemsetAsync(e->ctrl.p, 0, sizeof(Ctrl), stream()));
+    for (int k = 0; k < 3; ++k) GPR_TRY(alloc_queue(e->qmem[k], e->q[k], pass_entries(capacity, true), true));
+    GPR_TRY(e->ctrl.alloc(kMaxParts * sizeof(Ctrl)));
+    GPR_TRY(e->seg.alloc(parts_for(capacity, true) > 1 ? 8ull * kMaxParts * seg_words(kMaxSegs)
+                                                       : 8ull * seg_words(segs_for(capacity, true).nseg)));
+    GPR_HIP(hipMemsetAsync(e->ctrl.p, 0, kMaxParts * sizeof(Ctrl), stream()));
     GPR_TRY(e->pass.alloc(sizeof(PassBuf)));
     int cus = 0;
     GPR_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
@@ -1265,43 +1361,60 @@ namespace {
 // Launch grids cover `size` paths (the pass's size class), not the capacity:
 // a small pass launches small grids.
 int record_pass(Engine* e, uint32_t depth, int kidx, uint32_t chunk, uint32_t size, float4* fb, bool terms,
-                hipStream_t st) {
-    RenderArgs a{};
-    a.scenes = e->scenes.as<SceneView>();
-    a.pass = e->pass.as<PassBuf>();
-    for (int k = 0; k < 3; ++k) a.q[k] = e->q[k];
-    a.fb = fb;
-    a.ctrl = e->ctrl.as<Ctrl>();
-    a.spill = e->spill.as<int2>();
-    const Segs sg = segs_for(size, true);
-    a.seg = e->seg.as<unsigned long long>();
-    a.nseg = sg.nseg;
-    a.seg_cap = sg.cap;
-    a.depth = depth;
-    a.chunk_log = 31u - (uint32_t)__builtin_clz(chunk);
-    a.rng_mode = GPR_RNG_PCG;
+                uint32_t parts, hipStream_t st) {
+    RenderArgs pass{};
+    pass.scenes = e->scenes.as<SceneView>();
+    pass.pass = e->pass.as<PassBuf>();
+    for (int k = 0; k < 3; ++k) pass.q[k] = e->q[k];
+    pass.fb = fb;
+    pass.ctrl = pass.base = e->ctrl.as<Ctrl>();
+    pass.spill = e->spill.as<int2>();
+    pass.seg = e->seg.as<unsigned long long>();
+    pass.depth = depth;
+    pass.chunk_log = 31u - (uint32_t)__builtin_clz(chunk);
+    pass.rng_mode = GPR_RNG_PCG;
     if (terms) {
-        a.terms = e->terms.as<float4>();
-        a.nterm = e->nterm.as<uint8_t>();
-        a.tstride = size;
+        pass.terms = e->terms.as<float4>();
+        pass.nterm = e->nterm.as<uint8_t>();
+        pass.tstride = size;
     }
     const PassKernels& pk = pass_kernel_table(kidx);
-    const dim3 tg(std::min<uint32_t>(e->grid[kidx], div_up(size, pk.nt))), tb(pk.nt);
-    hipLaunchKernelGGL(k_gen<true>, dim3(div_up(size, 256)), dim3(256), 0, st, a);
-    hipLaunchKernelGGL(pk.ext_primary, tg, tb, 0, st, a, 0u);
-    for (uint32_t b = 0; b < depth; ++b) {
-        hipLaunchKernelGGL((k_shade<true, false>), dim3(shade_blocks(size, sg.nseg)), dim3(kShadeBlock), 0, st, a, b);
-        if (pk.shadow) hipLaunchKernelGGL(pk.shadow, tg, tb, 0, st, a, b);
-        hipLaunchKernelGGL(pk.trace, tg, tb, 0, st, a, b);
+    if (parts > 1) GPR_TRY(e->side.fork(st));
+    for (uint32_t part = 0; part < parts; ++part) {
+        RenderArgs a = pass;
+        const uint32_t n = set_part(a, size, parts, part, true, e->side_spill.as<int2>());
+        const hipStream_t ps = part ? e->side.s : st;
+        const dim3 tg(std::min<uint32_t>(e->grid[kidx], div_up(n, pk.nt))), tb(pk.nt);
+        hipLaunchKernelGGL(k_gen<true>, dim3(div_up(n, 256)), dim3(256), 0, ps, a);
+        hipLaunchKernelGGL(pk.ext_primary, tg, tb, 0, ps, a, 0u);
+        for (uint32_t b = 0; b < depth; ++b) {
+            hipLaunchKernelGGL((k_shade<true, false>), dim3(shade_blocks(n, a.nseg)), dim3(kShadeBlock), 0, ps, a, b);
+            if (pk.shadow) hipLaunchKernelGGL(pk.shadow, tg, tb, 0, ps, a, b);
+            hipLaunchKernelGGL(pk.trace, tg, tb, 0, ps, a, b);
+        }
+        hipLaunchKernelGGL(k_flush<true>, dim3(std::min(1024u, div_up(n, 256))), dim3(256), 0, ps, a);
     }
-    hipLaunchKernelGGL(k_flush<true>, dim3(std::min(1024u, div_up(size, 256))), dim3(256), 0, st, a);
-    if (terms) hipLaunchKernelGGL(k_accum<true>, dim3(div_up(size, 256)), dim3(256), 0, st, a);
+    if (parts > 1) GPR_TRY(e->side.join(st));
+    if (terms) hipLaunchKernelGGL(k_accum<true>, dim3(div_up(size, 256)), dim3(256), 0, st, pass);
     GPR_HIP(hipGetLastError());
     return GPR_OK;
 }
 }  // namespace
 
 namespace {
+// Stack overflow area of the second part's walks.
+uint64_t side_bytes(const Engine* e, int kidx) {
+    return (uint64_t)e->grid[kidx] * pass_kernel_table(kidx).nt * kStackGlobal * sizeof(int2);
+}
+// Whether a pass can run as two parts: the second one's area is there, or can
+// be allocated (once, at its largest, as captured passes hold its address).
+bool side_ready(Engine* e, int kidx) {
+    if (e->side_grows && !e->side_spill.p) {
+        e->side_grows = false;
+        if (e->side_spill.alloc(e->spill.bytes) != GPR_OK) (void)hipGetLastError();  // the failed allocation
+    }
+    return e->side_spill.bytes >= side_bytes(e, kidx) && e->side.make() == GPR_OK;
+}
 // Launch size class of a pass: its paths rounded up to a power of two.
 uint32_t size_class(const Engine* e, uint64_t paths) {
     uint64_t size = 1u << 16;
@@ -1347,14 +1460,16 @@ int engine_run_pass(Engine* e, const EngineJob* jobs, uint32_t njobs, float4* fb
     const size_t bytes = offsetof(PassBuf, jobs) + sizeof(PassJob) * njobs;
     GPR_HIP(hipMemcpyAsync(e->pass.p, h, bytes, hipMemcpyHostToDevice, st));
     GPR_HIP(hipEventRecord(e->ev[s], st));
-    const Engine::GraphKey key{depth, kidx, (uint32_t)cfg.chunk, size, fb, terms};
+    uint32_t parts = parts_for(size, true);
+    if (parts > 1 && !side_ready(e, kidx)) parts = 1;
+    const Engine::GraphKey key{depth, kidx, (uint32_t)cfg.chunk, size, fb, terms, parts};
     hipGraphExec_t exec = nullptr;
     for (auto& g : e->graphs)
         if (g.first == key) exec = g.second;
     if (!exec) {
         hipGraph_t graph;
         GPR_HIP(hipStreamBeginCapture(e->cap_stream, hipStreamCaptureModeThreadLocal));
-        const int rc = record_pass(e, depth, kidx, (uint32_t)cfg.chunk, size, fb, terms, e->cap_stream);
+        const int rc = record_pass(e, depth, kidx, (uint32_t)cfg.chunk, size, fb, terms, parts, e->cap_stream);
         const hipError_t ec = hipStreamEndCapture(e->cap_stream, &graph);
         GPR_TRY(rc);
         if (ec != hipSuccess) return fail(GPR_ERR_HIP, std::string("pass capture: ") + hipGetErrorString(ec));
@@ -1367,7 +1482,20 @@ int engine_run_pass(Engine* e, const EngineJob* jobs, uint32_t njobs, float4* fb
     return GPR_OK;
 }
 
-void engine_limit_terms(Engine* e, uint64_t bytes) { e->term_limit = bytes; }
+void engine_limit_terms(Engine* e, uint64_t bytes) {
+    e->term_limit = bytes;
+    e->side_grows = true;
+}
+
+uint64_t engine_side_bytes(const Engine* e) {
+    if (parts_for(e->capacity, true) == 1) return 0;
+    return side_bytes(e, pass_kernel_index(TraceCfg{256, 16, 64, 0, 0}));
+}
+int engine_reserve_side(Engine* e) {
+    if (e->side_spill.alloc(engine_side_bytes(e)) == GPR_OK) return GPR_OK;
+    (void)hipGetLastError();  // the failed allocation
+    return GPR_ERR_OOM;
+}
 
 int engine_reserve_terms(Engine* e, uint64_t bytes) {
     const uint64_t paths = std::min<uint64_t>(e->capacity, kPassPaths);  // one term count (a byte) each
@@ -1495,7 +1623,9 @@ using namespace gpr;
 // the last renderer that used them.
 struct PassWork {
     std::mutex mu;
-    DevBuf spill;  // kStackGlobal entries per resident lane, allocated once
+    DevBuf spill;       // kStackGlobal entries per resident lane, allocated once
+    DevBuf side_spill;  // those of a pass's second part
+    bool side_failed = false;
     DevBuf qmem[3], terms, nterm;
     QueueView q[3];
     uint32_t paths = 0, depth = 0;
@@ -1525,7 +1655,8 @@ struct gpr_renderer {
     DevBuf fb, ctrl, status;
     PixelReader reader;
     DevBuf seg;              // queue segment counters, then those of the last sample
-    uint32_t last_nseg = 1;  // segments of the last pass
+    uint32_t last_nseg = 1, last_parts = 1;  // segments and parts of the last pass
+    SideStream side;
     DevBuf qmem[3];
     DevBuf seeds[2];
     QueueView q[3];
@@ -1560,8 +1691,8 @@ RenderArgs make_args(gpr_renderer* r, uint32_t log_s) {
     RenderArgs a{};
     a.sv = r->scene->view();
     a.fb = r->fb.as<float4>();
-    a.ctrl = r->ctrl.as<Ctrl>();
-    a.npix = r->npix << log_s;
+    a.ctrl = a.base = r->ctrl.as<Ctrl>();
+    a.paths = r->npix << log_s;
     a.depth = r->opts.max_depth;
     a.log_s = log_s;
     if (log_s) {
@@ -1569,7 +1700,7 @@ RenderArgs make_args(gpr_renderer* r, uint32_t log_s) {
         for (int k = 0; k < 3; ++k) a.q[k] = w.q[k];
         a.terms = w.terms.as<float4>();
         a.nterm = w.nterm.as<uint8_t>();
-        a.tstride = a.npix;
+        a.tstride = a.paths;
     } else {
         for (int k = 0; k < 3; ++k) a.q[k] = r->q[k];
         a.status = r->status.as<unsigned long long>();
@@ -1577,11 +1708,8 @@ RenderArgs make_args(gpr_renderer* r, uint32_t log_s) {
     }
     a.spill = r->work->spill.as<int2>();
     a.seg = r->seg.as<unsigned long long>();
-    a.last = a.seg + seg_words(kMaxSegs);
+    a.last = a.seg + kMaxParts * seg_words(kMaxSegs);
     a.rng_mode = r->opts.rng_mode;
-    const Segs sg = a.rng_mode == GPR_RNG_REFERENCE ? Segs{1, a.npix} : segs_for(a.npix, false);
-    a.nseg = sg.nseg;
-    a.seg_cap = sg.cap;
     a.chunk_log = 6;
     a.rr_start = r->opts.rr_start;
     a.seed = r->opts.seed;
@@ -1594,27 +1722,46 @@ RenderArgs make_args(gpr_renderer* r, uint32_t log_s) {
 // textured scene 5.03 / 4.85 / 4.88 ms, 4 of the sphere grid 16.7 / 16.7 / 17.1.
 constexpr int kRenderNT = 256, kRenderSL = 12;
 
-// One pass of 2^log_s samples: gen -> extend(primary) -> max_depth x {shade, trace} -> flush -> accum -> finish.
-int launch_pass(gpr_renderer* r, uint32_t log_s, hipStream_t st) {
-    const RenderArgs a = make_args(r, log_s);
-    const bool ref = r->opts.traversal == GPR_TRAVERSAL_REF;
-    // the whole grid where the paths are few, too: they are spread thin over it
-    const dim3 tg(std::min<uint32_t>(r->grid_trace, a.npix)), tb(kRenderNT);
-    constexpr int NT = kRenderNT, SL = kRenderSL;
-    hipLaunchKernelGGL(k_gen<false>, dim3(div_up(a.npix, 256)), dim3(256), 0, st, a);
-    if (ref) hipLaunchKernelGGL((k_extend<true, true, false, NT, SL>), tg, tb, 0, st, a, 0u);
-    else hipLaunchKernelGGL((k_extend<true, false, false, NT, SL>), tg, tb, 0, st, a, 0u);
-    for (uint32_t b = 0; b < r->opts.max_depth; ++b) {
-        if (a.rng_mode == GPR_RNG_REFERENCE)
-            hipLaunchKernelGGL((k_shade<false, true>), dim3(div_up(a.npix, kShadeBlock)), dim3(kShadeBlock), 0, st, a, b);
-        else
-            hipLaunchKernelGGL((k_shade<false, false>), dim3(shade_blocks(a.npix, a.nseg)), dim3(kShadeBlock), 0, st, a, b);
-        if (ref) hipLaunchKernelGGL((k_trace<true, false, NT, SL>), tg, tb, 0, st, a, b);
-        else hipLaunchKernelGGL((k_trace<false, false, NT, SL>), tg, tb, 0, st, a, b);
+// Parts of a pass of 2^log_s samples.  Reference RNG mode orders its queues by
+// pixel: one part.
+uint32_t pass_parts(gpr_renderer* r, uint32_t log_s) {
+    if (r->opts.rng_mode != GPR_RNG_PCG || parts_for(r->npix << log_s, false) == 1) return 1;
+    PassWork& w = *r->work;
+    if (!w.side_spill.p && !w.side_failed && w.side_spill.alloc(w.spill.bytes) != GPR_OK) {
+        (void)hipGetLastError();  // the failed allocation
+        w.side_failed = true;
     }
-    if (a.depth) hipLaunchKernelGGL(k_flush<false>, dim3(std::min(1024u, div_up(a.npix, 256))), dim3(256), 0, st, a);
-    if (log_s) hipLaunchKernelGGL(k_accum<false>, dim3(div_up(r->npix, 256)), dim3(256), 0, st, a);
-    hipLaunchKernelGGL(k_finish, dim3(1), dim3(64), 0, st, a.ctrl, 1u << log_s);
+    return w.side_spill.p && r->side.make() == GPR_OK ? kMaxParts : 1;
+}
+
+// One pass of 2^log_s samples: gen -> extend(primary) -> max_depth x {shade, trace} -> flush -> accum -> finish.
+int launch_pass(gpr_renderer* r, uint32_t log_s, uint32_t parts, hipStream_t st) {
+    const RenderArgs pass = make_args(r, log_s);
+    const bool ref = r->opts.traversal == GPR_TRAVERSAL_REF;
+    constexpr int NT = kRenderNT, SL = kRenderSL;
+    if (parts > 1) GPR_TRY(r->side.fork(st));
+    for (uint32_t part = 0; part < parts; ++part) {
+        RenderArgs a = pass;
+        const uint32_t n = set_part(a, a.paths, parts, part, false, r->work->side_spill.as<int2>());
+        const hipStream_t ps = part ? r->side.s : st;
+        // the whole grid where the paths are few, too: they are spread thin over it
+        const dim3 tg(std::min<uint32_t>(r->grid_trace, n)), tb(kRenderNT);
+        hipLaunchKernelGGL(k_gen<false>, dim3(div_up(n, 256)), dim3(256), 0, ps, a);
+        if (ref) hipLaunchKernelGGL((k_extend<true, true, false, NT, SL>), tg, tb, 0, ps, a, 0u);
+        else hipLaunchKernelGGL((k_extend<true, false, false, NT, SL>), tg, tb, 0, ps, a, 0u);
+        for (uint32_t b = 0; b < r->opts.max_depth; ++b) {
+            if (a.rng_mode == GPR_RNG_REFERENCE)
+                hipLaunchKernelGGL((k_shade<false, true>), dim3(div_up(n, kShadeBlock)), dim3(kShadeBlock), 0, ps, a, b);
+            else
+                hipLaunchKernelGGL((k_shade<false, false>), dim3(shade_blocks(n, a.nseg)), dim3(kShadeBlock), 0, ps, a, b);
+            if (ref) hipLaunchKernelGGL((k_trace<true, false, NT, SL>), tg, tb, 0, ps, a, b);
+            else hipLaunchKernelGGL((k_trace<false, false, NT, SL>), tg, tb, 0, ps, a, b);
+        }
+        if (a.depth) hipLaunchKernelGGL(k_flush<false>, dim3(std::min(1024u, div_up(n, 256))), dim3(256), 0, ps, a);
+    }
+    if (parts > 1) GPR_TRY(r->side.join(st));
+    if (log_s) hipLaunchKernelGGL(k_accum<false>, dim3(div_up(r->npix, 256)), dim3(256), 0, st, pass);
+    hipLaunchKernelGGL(k_finish, dim3(1), dim3(64), 0, st, pass.base, 1u << log_s);
     GPR_HIP(hipGetLastError());
     return GPR_OK;
 }
@@ -1626,7 +1773,7 @@ int launch_pass(gpr_renderer* r, uint32_t log_s, hipStream_t st) {
 // zero and a byte comparison covers all of them.
 bool same_view(const SceneView& a, const SceneView& b) { return std::memcmp(&a, &b, sizeof(SceneView)) == 0; }
 
-int pass_graph(gpr_renderer* r, uint32_t log_s, hipGraphExec_t* out) {
+int pass_graph(gpr_renderer* r, uint32_t log_s, uint32_t parts, hipGraphExec_t* out) {
     const SceneView now = r->scene->view();
     if (r->has_graph() && !same_view(now, r->baked)) {
         GPR_HIP(hipStreamSynchronize(stream()));
@@ -1638,7 +1785,7 @@ int pass_graph(gpr_renderer* r, uint32_t log_s, hipGraphExec_t* out) {
         if (!r->cap_stream) GPR_HIP(hipStreamCreateWithFlags(&r->cap_stream, hipStreamNonBlocking));
         hipGraph_t g;
         GPR_HIP(hipStreamBeginCapture(r->cap_stream, hipStreamCaptureModeThreadLocal));
-        const int rc = launch_pass(r, log_s, r->cap_stream);
+        const int rc = launch_pass(r, log_s, parts, r->cap_stream);
         const hipError_t ec = hipStreamEndCapture(r->cap_stream, &g);
         GPR_TRY(rc);
         if (ec != hipSuccess) return fail(GPR_ERR_HIP, std::string("sample capture: ") + hipGetErrorString(ec));
@@ -1671,7 +1818,7 @@ int grow_work(gpr_renderer* r, PassWork& w, uint32_t paths) {
     }
     // given back first, so that the old and the new buffers never exist together
     for (DevBuf* b : {&w.qmem[0], &w.qmem[1], &w.qmem[2], &w.terms, &w.nterm}) b->release();
-    for (int k = 0; k < 3; ++k) GPR_TRY(alloc_queue(w.qmem[k], w.q[k], queue_entries(np, false), false));
+    for (int k = 0; k < 3; ++k) GPR_TRY(alloc_queue(w.qmem[k], w.q[k], pass_entries(np, false), false));
     GPR_TRY(w.terms.alloc(16ull * np * max_terms(nd)));
     GPR_TRY(w.nterm.alloc(np));
     w.paths = np;
@@ -1707,11 +1854,11 @@ int renderer_alloc(gpr_renderer* r) {
     r->npix = (uint32_t)npix;
     GPR_HIP(hipSetDevice(s->device));
     GPR_TRY(r->fb.alloc(16ull * npix));
-    GPR_TRY(r->ctrl.alloc(sizeof(Ctrl)));
-    GPR_TRY(r->seg.alloc(8ull * (seg_words(kMaxSegs) + kMaxBounce * kLastSpread)));
+    GPR_TRY(r->ctrl.alloc(kMaxParts * sizeof(Ctrl)));
+    GPR_TRY(r->seg.alloc(8ull * kMaxParts * (seg_words(kMaxSegs) + kMaxBounce * kLastSpread)));
     r->ntiles = div_up(npix, kShadeBlock);
     GPR_TRY(r->status.alloc(8ull * kMaxBounce * r->ntiles));
-    for (int k = 0; k < 3; ++k) GPR_TRY(alloc_queue(r->qmem[k], r->q[k], queue_entries(r->npix, false), false));
+    for (int k = 0; k < 3; ++k) GPR_TRY(alloc_queue(r->qmem[k], r->q[k], pass_entries(r->npix, false), false));
     for (int k = 0; k < 2; ++k) {
         GPR_TRY(r->seeds[k].alloc(4ull * npix));
         GPR_HIP(hipMemsetAsync(r->seeds[k].p, 0, 4ull * npix, stream()));  // DEVICE_BUFFER allocations start zeroed (buffer.h:62)
@@ -1871,11 +2018,15 @@ int gpr_render(gpr_renderer* r, uint32_t spp) {
     for (uint32_t left = spp; left;) {
         while ((1u << log_s) > left) --log_s;
         hipGraphExec_t g = nullptr;
-        GPR_TRY(pass_graph(r, log_s, &g));
+        const uint32_t parts = pass_parts(r, log_s);
+        GPR_TRY(pass_graph(r, log_s, parts, &g));
         GPR_HIP(hipGraphLaunch(g, st));
         left -= 1u << log_s;
+        RenderArgs a = make_args(r, log_s);
+        set_part(a, a.paths, parts, 0, false, nullptr);
         r->last_log_s = log_s;
-        r->last_nseg = make_args(r, log_s).nseg;
+        r->last_parts = parts;
+        r->last_nseg = a.nseg;
     }
     r->spp_done += spp;
     uint32_t err = 0;
@@ -1904,13 +2055,15 @@ int gpr_renderer_queue_sizes(gpr_renderer* r, uint32_t* shadow, uint32_t* scatte
     for (uint32_t b = 0; b < cap && b < kMaxBounce; ++b) {
         uint32_t sh = 0, sc = 0;
         // of several samples the last one alone
-        const uint32_t parts = r->last_log_s ? kLastSpread : r->last_nseg;
-        for (uint32_t k = 0; k < parts; ++k) {
-            const unsigned long long n = r->last_log_s ? c[seg_words(kMaxSegs) + b * kLastSpread + k]
-                                                       : c[(b * r->last_nseg + k) * seg_stride(r->last_nseg)];
-            sh += (uint32_t)(n >> 32);
-            sc += (uint32_t)n;
-        }
+        const uint32_t words = r->last_log_s ? kLastSpread : r->last_nseg;
+        for (uint32_t p = 0; p < r->last_parts; ++p)
+            for (uint32_t k = 0; k < words; ++k) {
+                const unsigned long long n =
+                    r->last_log_s ? c[kMaxParts * seg_words(kMaxSegs) + (p * kMaxBounce + b) * kLastSpread + k]
+                                  : c[p * seg_words(kMaxSegs) + (b * r->last_nseg + k) * seg_stride(r->last_nseg)];
+                sh += (uint32_t)(n >> 32);
+                sc += (uint32_t)n;
+            }
         if (shadow) shadow[b] = sh;
         if (scatter) scatter[b] = sc;
     }

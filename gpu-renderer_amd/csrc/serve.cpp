@@ -439,6 +439,7 @@ struct gpr_server {
 namespace {
 // Device bytes a server sets aside for term lists at most (2^23 paths of depth 8).
 constexpr uint64_t kServerTermBytes = 2400ull << 20;
+constexpr uint64_t kTermBytesPerPath = 16 * 17 + 1;  // at depth 8
 
 struct Finishing {
     hipEvent_t ev;
@@ -651,9 +652,14 @@ int gpr_server_create(const gpr_server_opts* o, gpr_server** out) {
     if (o->hbm_budget <= fixed + 16ull * o->capacity)
         return fail(GPR_ERR_BUDGET, "gpr_server_create: budget below arena + queues + one full frame buffer");
     // Of what the budget leaves beyond four full passes of frame buffers, the
-    // term lists of passes of several samples a job come first.
+    // term lists of passes of several samples a job come first, and before them
+    // what a pass in two parts needs, if lists for a full pass still fit.
     uint64_t rest = o->hbm_budget - fixed;
     const uint64_t frames = 64ull * o->capacity;
+    const uint64_t side = engine_side_bytes(s->eng);
+    if (side > 0 && rest > frames + side && rest - frames - side >= kTermBytesPerPath * o->capacity &&
+        engine_reserve_side(s->eng) == GPR_OK)
+        rest -= side;
     if (rest > frames) {
         const uint64_t terms = std::min(rest - frames, kServerTermBytes);
         if (engine_reserve_terms(s->eng, terms) == GPR_OK) rest -= terms;
