@@ -166,6 +166,35 @@ __global__ __launch_bounds__(NT) void k_trace_refill(SceneView sv, const gpr_ray
     }
 }
 
+// Short batches: four lanes to a ray (quad_trace), at most 16 rays to a wave.
+// Blocks of 64 / 128 / 256 threads and stacks of 16 / 32 entries measured within
+// noise of each other.
+constexpr int kQuadNT = 128, kQuadSL = 32;
+template <bool ANY>
+__global__ __launch_bounds__(kQuadNT) void k_trace_quad(SceneView sv, const gpr_ray* __restrict__ rays,
+                                                        gpr_hit* __restrict__ hits, uint64_t n,
+                                                        unsigned long long* __restrict__ cursor,
+                                                        int2* __restrict__ spill, uint32_t chunk_log) {
+    using Stack = QuadStack<typename StackEntry<ANY>::type, kQuadSL>;
+    __shared__ typename StackEntry<ANY>::type lds[kQuadSL * kQuadNT / 4];
+    Stack st;
+    st.template place<kQuadNT>(lds, spill);
+    const uint32_t quad = (threadIdx.x & 63) / 4;
+    const uint32_t lg = min(turn_log(n, gridDim.x * (kQuadNT / 64), chunk_log), 4u);
+    for_each_turn<kQuadNT, false>(cursor, (n + (1ull << lg) - 1) >> lg, [&](uint64_t turn) {
+        const uint64_t i = (turn << lg) + quad;
+        if (quad < (1u << lg) && i < n) {
+            gpr_hit h;
+            uint32_t own;
+            const bool ok = quad_trace<ANY>(sv, load_ray(rays, i), st, h, own);
+            if ((threadIdx.x & 3) == own) {
+                if (!ok) atomicAdd(cursor + 1, 1ull);  // stack overflow count
+                store_hit(hits, i, h);
+            }
+        }
+    });
+}
+
 template <bool ANY>
 __global__ __launch_bounds__(256) void k_trace_ref(SceneView sv, const gpr_ray* __restrict__ rays,
                                                    gpr_hit* __restrict__ hits, uint64_t n,
@@ -253,6 +282,7 @@ struct TraceResources {
     DevBuf spill;
     DevBuf cursor;
     int grid[kTraceVariants][4] = {};  // [variant][closest, any, closest refill, any refill]
+    int grid_quad[2] = {};             // closest, any
     int dev = -1;
 };
 // Work buffers of the fast traces, one set per (device, stream): launches on
@@ -284,6 +314,12 @@ int ensure_resources(TraceResources& R) {
             threads = std::max(threads, (size_t)R.grid[k][a] * v.nt);
         }
     }
+    for (int a = 0; a < 2; ++a) {
+        int per_cu = 0;
+        GPR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, a ? k_trace_quad<true> : k_trace_quad<false>, kQuadNT, 0));
+        R.grid_quad[a] = cus * std::max(1, per_cu);
+        threads = std::max(threads, (size_t)R.grid_quad[a] * kQuadNT / 4);  // a stack for every four lanes
+    }
     GPR_TRY(R.spill.alloc(threads * kStackGlobal * sizeof(int2)));
     GPR_TRY(R.cursor.alloc(4 * sizeof(unsigned long long)));
     R.dev = dev;
@@ -306,6 +342,13 @@ bool trace_cfg_valid(int nt, int sl, int chunk) {
 }
 
 namespace {
+// Four lanes take a ray up to this many rays, about what the chip holds at once
+// in that form.  Measured (us a call), 128x16 against it, at 1M / 20K triangles:
+//   closest   4096 rays  164 / 101   108 /  67      any hit  4096  125 / 104   111 /  82
+//            32768       232 / 151   171 / 105              32768  215 / 130   178 / 109
+//           131072       325 / 203   265 / 187             131072  354 / 183   328 / 179
+//           262144       379 / 242   383 / 290             262144  369 / 204   397 / 289
+constexpr uint64_t kQuadRays = 1u << 17;
 // Launch shape of a batch on a scene that was not tuned.  Refill pays once the
 // queue is long enough to keep its lanes fed; any-hit walks are shorter, so
 // later.  Measured (us, at 1M / 20K triangles):
@@ -339,6 +382,17 @@ int launch_trace(const SceneView& sv, const gpr_ray* rays, gpr_hit* hits, uint64
         const dim3 grid((unsigned)((n + 255) / 256));
         if (any) hipLaunchKernelGGL(k_trace_ref<true>, grid, dim3(256), 0, st, sv, rays, hits, n, stats);
         else hipLaunchKernelGGL(k_trace_ref<false>, grid, dim3(256), 0, st, sv, rays, hits, n, stats);
+        GPR_HIP(hipGetLastError());
+        return GPR_OK;
+    }
+    if (nt == 0 && n <= kQuadRays) {
+        TraceResources* rp = nullptr;
+        GPR_TRY(resources_for(st, &rp));
+        unsigned long long* cur = rp->cursor.as<unsigned long long>();
+        hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, cur, 4);
+        const dim3 grid((unsigned)std::min<uint64_t>(rp->grid_quad[any ? 1 : 0], n));
+        const auto kernel = any ? k_trace_quad<true> : k_trace_quad<false>;
+        hipLaunchKernelGGL(kernel, grid, dim3(kQuadNT), 0, st, sv, rays, hits, n, cur, rp->spill.as<int2>(), 4u);
         GPR_HIP(hipGetLastError());
         return GPR_OK;
     }

@@ -28,8 +28,8 @@ struct Ray3 {
 
 // triangle_intersect (pathtracer_kernel.h:119-152): float dots widened to
 // double, double 1/det; rejects det==0, u<0|u>1, v<0|u+v>1, t<tmin|t>tmax.
-GPR_D bool tri_hit_ref(v3 p0, v3 p1, v3 p2, v3 o, v3 d, float tmin, float tmax, float& th,
-                       float& uh, float& vh) {
+GPR_D bool tri_hit_wide(v3 p0, v3 p1, v3 p2, v3 o, v3 d, float tmin, float tmax, double& th,
+                        float& uh, float& vh) {
     const v3 e1 = p1 - p0;
     const v3 e2 = p2 - p0;
     const v3 P = cross3(d, e2);
@@ -44,9 +44,16 @@ GPR_D bool tri_hit_ref(v3 p0, v3 p1, v3 p2, v3 o, v3 d, float tmin, float tmax, 
     if (v < 0.0 || u + v > 1.0) return false;
     const double t = (double)dot3(Q, e2) * inv_det;
     if (t < (double)tmin || t > (double)tmax) return false;
-    th = (float)t;
+    th = t;
     uh = (float)u;
     vh = (float)v;
+    return true;
+}
+GPR_D bool tri_hit_ref(v3 p0, v3 p1, v3 p2, v3 o, v3 d, float tmin, float tmax, float& th,
+                       float& uh, float& vh) {
+    double t;
+    if (!tri_hit_wide(p0, p1, p2, o, d, tmin, tmax, t, uh, vh)) return false;
+    th = (float)t;
     return true;
 }
 
@@ -437,6 +444,169 @@ GPR_D bool fast_trace(const SceneView& sv, const Ray3& r, Stack& st, gpr_hit& hi
     while (trav_live(sv, t)) trav_step<ANY>(sv, st, t);
     hit = t.hit;
     return t.node == kTravDone;
+}
+
+// ------------------------------------------- four lanes to a ray (BVH4) ---
+// A short batch leaves most lanes of the chip idle, and its time is that of one
+// long walk: a chain of node loads and of the ~190 instructions a lane runs
+// between two of them.  Here four lanes walk one ray: each tests one child's
+// box, or its triangle if the child is a leaf, the children order by comparing
+// keys across the four lanes, and each pushed child is stored by its own lane,
+// about half the instructions.  Boxes, keys, stack entries and the order of the
+// triangle tests are those of trav_step, so hits are bit-identical.
+template <int CTRL>
+GPR_D uint32_t quad_dpp(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, CTRL, 0xf, 0xf, true);
+}
+enum : int { kQuadRot1 = 0x39, kQuadRot2 = 0x4e, kQuadRot3 = 0x93 };  // lane i reads lane i + 1, 2, 3 of its four
+template <int FROM>
+GPR_D double quad_from(double x) {
+    constexpr int ctrl = FROM * 0x55;
+    return __hiloint2double((int)quad_dpp<ctrl>((uint32_t)__double2hiint(x)),
+                            (int)quad_dpp<ctrl>((uint32_t)__double2loint(x)));
+}
+GPR_D uint32_t quad_or(uint32_t x) {
+    x |= quad_dpp<kQuadRot2>(x);
+    return x | quad_dpp<kQuadRot1>(x);
+}
+// the four lanes' bits, slot 0 lowest
+GPR_D uint32_t quad_mask(bool b) { return quad_or(b ? 1u << (threadIdx.x & 3) : 0u); }
+
+// A ray's stack, shared by its four lanes: SL entries in LDS, the rest in the overflow area.
+template <class E, int SL>
+struct QuadStack {
+    static constexpr int kStride = 16;
+    E* lds;
+    E* spill;
+    int sp;
+    template <int NT>
+    GPR_D void place(void* block_lds, int2* overflow) {
+        const uint32_t wave = threadIdx.x / 64, quad = (threadIdx.x & 63) / 4;
+        lds = static_cast<E*>(block_lds) + wave * (SL * 16) + quad;
+        spill = reinterpret_cast<E*>(overflow + ((uint64_t)(blockIdx.x * (NT / 64) + wave) * 16 + quad) * kStackGlobal);
+    }
+    GPR_D void put(int at, E e) {
+        if (at < SL) lds[at * kStride] = e;
+        else spill[at - SL] = e;
+    }
+    GPR_D E get(int at) const { return at < SL ? lds[at * kStride] : spill[at - SL]; }
+    GPR_D bool full(int k) const { return sp + k > SL + kStackGlobal; }
+    // entries that one lane wrote are read by the others
+    GPR_D void publish() const {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+};
+
+// The walk of fast_trace<ANY>.  All four lanes hold the ray, tmax, node and
+// stack height; lane c of the four holds child c, and `hit` belongs to the lane
+// that `own` names (the first one for a miss).  Returns false where fast_trace does.
+template <bool ANY, class Stack>
+GPR_D bool quad_trace(const SceneView& sv, const Ray3& r, Stack& st, gpr_hit& hit, uint32_t& own) {
+    using E = typename StackEntry<ANY>::type;
+    const uint32_t c = threadIdx.x & 3;
+    float tmax = r.tmax;
+    hit = gpr_hit{INFINITY, -1, 0.f, 0.f};
+    own = 0;
+    if (sv.root4 < 0) {  // single-triangle scene
+        bool found = false;
+        tri_rec_hit(sv.tris, sv.ntri, ~sv.root4, r, tmax, hit, found);
+        return true;
+    }
+    if constexpr (ANY) st.put(0, kTravDone);
+    else st.put(0, make_uint2((uint32_t)kTravDone << 2, 0xff800000u));
+    st.sp = 1;
+    const v3 inv = V(1 / r.d.x, 1 / r.d.y, 1 / r.d.z);
+    const uint32_t nxo = (__builtin_signbit(inv.x) ? 16u : 0u) + 4 * c, fxo = nxo ^ 16u;
+    const uint32_t nyo = (__builtin_signbit(inv.y) ? 48u : 32u) + 4 * c, fyo = nyo ^ 16u;
+    const uint32_t nzo = (__builtin_signbit(inv.z) ? 80u : 64u) + 4 * c, fzo = nzo ^ 16u;
+    int32_t node = sv.root4;
+    uint32_t fetched = 0;
+    while ((uint32_t)node < sv.nbvh4 && fetched <= sv.nbvh4) {
+        const char* np = reinterpret_cast<const char*>(sv.bvh4) + ((uint64_t)(uint32_t)node << 7);
+        const auto plane = [&](uint32_t off) { return ldg(reinterpret_cast<const float*>(np + off)); };
+        const float nx = plane(nxo), fx = plane(fxo), ny = plane(nyo), fy = plane(fyo), nz = plane(nzo), fz = plane(fzo);
+        const int32_t ch = ldg(reinterpret_cast<const int32_t*>(np + 96 + 4 * c));
+        const float x0 = (nx - r.o.x) * inv.x, x1 = (fx - r.o.x) * inv.x;
+        const float y0 = (ny - r.o.y) * inv.y, y1 = (fy - r.o.y) * inv.y;
+        const float z0 = (nz - r.o.z) * inv.z, z1 = (fz - r.o.z) * inv.z;
+        const float tn = fmaxf(fmaxf(x0, y0), fmaxf(z0, r.tmin));
+        const float tf = fminf(fminf(x1, y1), fminf(z1, tmax));
+        const bool in = tn <= tf * kSlabCons;
+        ++fetched;
+        // leaf children, all at once
+        bool ok = false;
+        double td = 0.0;
+        gpr_hit h{};
+        if (in && (uint32_t)ch > (uint32_t)kEmptyChild && (uint32_t)~ch < sv.ntri) {
+            const TriRec* t = sv.tris + (uint32_t)~ch;
+            const float4 a = ldg(&t->a), b = ldg(&t->b), e = ldg(&t->c);
+            ok = tri_hit_wide(V(a.x, a.y, a.z), V(a.w, b.x, b.y), V(b.z, b.w, e.x), r.o, r.d, r.tmin, tmax, td, h.u, h.v);
+            h.t = (float)td;
+            h.id = (int32_t)__float_as_uint(e.y);
+        }
+        if (__ballot(ok) != 0ull) {
+            const uint32_t m = quad_mask(ok);
+            if constexpr (ANY) {
+                if (m) {  // the first in slot order ends the walk
+                    own = __builtin_ctz(m);
+                    if (c == own) hit = h;
+                    return true;
+                }
+            } else {
+                // in slot order, each against what the ones before it left of the ray
+                uint32_t best = 4;
+                const auto take = [&](uint32_t s, double t) {
+                    const bool nearer = (m >> s & 1u) && !(t > (double)tmax);
+                    tmax = nearer ? (float)t : tmax;
+                    best = nearer ? s : best;
+                };
+                take(0, quad_from<0>(td));
+                take(1, quad_from<1>(td));
+                take(2, quad_from<2>(td));
+                take(3, quad_from<3>(td));
+                if (best != 4) own = best;
+                if (c == best) hit = h;
+            }
+        }
+        // inner children: the first one next, the others pushed
+        bool go = in && ch >= 0;
+        uint32_t key, payload;
+        E e;
+        if constexpr (ANY) {
+            key = go ? c : kKeyNone;
+            payload = (uint32_t)ch;
+            e = ch;
+        } else {
+            go = go && tn <= tmax * kSlabCons;
+            key = go ? ((__float_as_uint(fmaxf(tn, 0.f)) & ~3u) | c) : kKeyNone;
+            payload = ((uint32_t)ch << 2) | (__float_as_uint(tn) & 3u);
+            e = make_uint2(payload, key);
+        }
+        const uint32_t before = (quad_dpp<kQuadRot1>(key) < key ? 1u : 0u) + (quad_dpp<kQuadRot2>(key) < key ? 1u : 0u) +
+                                (quad_dpp<kQuadRot3>(key) < key ? 1u : 0u);
+        const int n = __popc(quad_mask(go));
+        if (n == 0) {
+            if constexpr (ANY) {
+                node = st.get(--st.sp);
+            } else {
+                const float plim = fmaxf(tmax * kSlabCons, __uint_as_float(4u));
+                E p;
+                do {
+                    p = st.get(--st.sp);
+                } while (__uint_as_float((p.y & ~3u) | (p.x & 3u)) > plim);
+                node = (int32_t)(p.x >> 2);
+            }
+        } else {
+            if (st.full(3)) return false;
+            if (go && before > 0) st.put(st.sp + n - 1 - (int)before, e);
+            st.sp += n - 1;
+            const uint32_t next = quad_or(go && before == 0 ? payload : 0u);
+            node = ANY ? (int32_t)next : (int32_t)(next >> 2);
+        }
+        st.publish();
+    }
+    return node == kTravDone;
 }
 
 // Rays a wave takes a turn: `chunk` (a power of two, at least 64) of them, or
