@@ -48,3 +48,36 @@ def test_four_lanes_to_a_ray(ntri, n, any_hit):
     want = s.trace(r, any_hit=any_hit)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
     s.free()
+
+
+@pytest.mark.parametrize("name,w,h,spp", [("spheres", 256, 256, 4), ("textured", 257, 255, 3), ("spheres", 91, 90, 8)])
+def test_short_queues_of_a_render(name, w, h, spp):
+    # one sample a pass keeps the queues at or below 2^16 entries (four lanes to an entry), all of them in one exceed it
+    import gpu_scenes as G
+    s = gpr.Scene.sphere_grid(w, h, 6) if name == "spheres" else G.textured(w, h).commit()
+    o = dict(max_depth=8, rr_start=3, seed=3)
+    print(f"[quads] {name} {w}x{h} spp {spp}", flush=True)
+    one, many = gpr.Renderer(s, **o), gpr.Renderer(s, **o)
+    for _ in range(spp):
+        one.render(1)
+    many.render(spp)
+    assert np.array_equal(one.read()[0].view(np.uint32), many.read()[0].view(np.uint32))
+    one.free()
+    many.free()
+
+
+def test_short_queues_of_the_engine_against_refilled_walks():
+    s = gpr.Scene.sphere_grid(8, 8, 6)
+    b = gpr.Batch(gpr.arena_bytes(s), capacity=1 << 18, max_jobs=2)
+    i = b.add_scene(s)
+    for w, h in ((201, 77), (64, 33)):
+        b.add_job(gpr.job(i, w, h, 3, gpr.lookat((0, 0, 0), (1.0, 6, 9)), 40, 6, 3, w))
+    out = []
+    for cfg in ((256, 16, 64, 0, 0), (64, 8, 64, 0, 0), (512, 8, 128, 0, 0), (128, 16, 64, 0, 1)):
+        print(f"[quads] engine cfg {cfg}", flush=True)
+        b.set_cfg(*cfg)
+        b.run()
+        out.append([b.read(0), b.read(1)])
+    for o in out:
+        assert all(np.array_equal(x.view(np.uint32), y.view(np.uint32)) for x, y in zip(o, out[-1]))
+    b.free()
