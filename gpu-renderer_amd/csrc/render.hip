@@ -794,24 +794,66 @@ GPR_D unsigned long long pack_status(uint32_t flag, uint32_t sh, uint32_t sc) {
     return ((unsigned long long)flag << 62) | ((unsigned long long)sh << 31) | (unsigned long long)sc;
 }
 
+// Publishes a tile's counts and returns the sum of those before it (without the
+// flag), by the 64 lanes of one wave: a step back reads 64 tiles.
+GPR_D unsigned long long look_back(unsigned long long* st, uint32_t tile, unsigned long long mine, uint32_t* error) {
+    const uint32_t lane = threadIdx.x & 63;
+    constexpr unsigned long long kCounts = (1ull << 62) - 1;
+    unsigned long long sum = 0;
+    if (tile > 0) {
+        if (lane == 0) __hip_atomic_store(st + tile, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        uint32_t spins = 0;
+        for (uint32_t end = tile;;) {  // tiles from end on are summed
+            unsigned long long v = 2ull << 62;  // nothing before the first tile
+            if (lane < end) v = __hip_atomic_load(st + (end - 1 - lane), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned long long open = __ballot((v >> 62) == 0), whole = __ballot((v >> 62) == 2);
+            const int stop = whole ? __builtin_ctzll(whole) : 63;  // the lane whose tile ends the step
+            if (open & (2ull << stop) - 1) {
+                // predecessor tiles took their ids earlier and are resident: this wait ends
+                if (++spins > (1u << 26)) {
+                    if (lane == 0) atomicOr(error, 2u);
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(1);
+                continue;
+            }
+            v = (int)lane <= stop ? v & kCounts : 0ull;
+            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+            sum += v;
+            if (whole) break;
+            end -= 64;
+        }
+    }
+    if (lane == 0)
+        __hip_atomic_store(st + tile, (2ull << 62) | (sum + (mine & kCounts)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return sum;
+}
+
 // ORDERED: appends keep the queue order (reference RNG mode: seeds belong to
 // slots), by tickets and a decoupled look-back over one segment.  Otherwise a
 // block takes its place in its segment with one atomic.
+// Ordered tiles take a ticket each, an atomic on one address (~12 ns, one after
+// the other), so they are larger: 4 samples of the 640x360 Cornell box in reference
+// RNG mode 2093 / 1942 / 1799 / 1719 us with 256 entries and a look-back by one
+// thread, and 256 / 512 / 1024 entries with a look-back by a wave; a 1600x900
+// textured frame 2124 / 2119 / 2046 / 2049, a 300x200 frame 618 / 609 / 617 / 700.
+constexpr int kOrderedBlock = 512;
 template <bool MULTI, bool ORDERED>
-__global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bounce) {
+__global__ __launch_bounds__(ORDERED ? kOrderedBlock : kShadeBlock) void k_shade(RenderArgs a, uint32_t bounce) {
+    constexpr int NB = ORDERED ? kOrderedBlock : kShadeBlock;
     __shared__ uint32_t s_tile;
-    __shared__ uint32_t s_wave[2][kShadeBlock / 64];
+    __shared__ uint32_t s_wave[2][NB / 64];
     __shared__ uint32_t s_base[2];
-    __shared__ uint32_t s_last[kShadeBlock / 64];
+    __shared__ uint32_t s_last[NB / 64];
     uint32_t tile, ntiles_in, i, n_end;
     if constexpr (ORDERED) {
         const uint32_t n_in = bounce == 0 ? npaths_of<MULTI>(a) : (uint32_t)*seg_at(a, bounce - 1, 0);
         if (threadIdx.x == 0) s_tile = atomicAdd(&a.ctrl->tile_counter[bounce], 1u);
         __syncthreads();
         tile = s_tile;
-        ntiles_in = (n_in + kShadeBlock - 1) / kShadeBlock;
+        ntiles_in = (n_in + NB - 1) / NB;
         if (tile >= ntiles_in) return;
-        i = tile * kShadeBlock + threadIdx.x;
+        i = tile * NB + threadIdx.x;
         n_end = n_in;
     } else {
         constexpr uint32_t kLog = 8;
@@ -999,7 +1041,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
     }
     uint32_t wsh = 0, wsc = 0, tsh = 0, tsc = 0;
 #pragma unroll
-    for (int k = 0; k < kShadeBlock / 64; ++k) {
+    for (int k = 0; k < NB / 64; ++k) {
         if (k < wave) {
             wsh += s_wave[0][k];
             wsc += s_wave[1][k];
@@ -1015,39 +1057,16 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(RenderArgs a, uint32_t bo
             s_base[0] = g * a.seg_cap + (uint32_t)(at >> 32);
             s_base[1] = g * a.seg_cap + (uint32_t)at;
         }
-    } else if (threadIdx.x == 0) {
+    } else if (wave == 0) {
         unsigned long long* st = a.status + (uint64_t)bounce * a.ntiles;
-        uint32_t psh = 0, psc = 0;
-        if (tile == 0) {
-            __hip_atomic_store(st, pack_status(2, tsh, tsc), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            __hip_atomic_store(st + tile, pack_status(1, tsh, tsc), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            int j = (int)tile - 1;
-            uint32_t spins = 0;
-            while (j >= 0) {
-                const unsigned long long v = __hip_atomic_load(st + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const uint32_t f = (uint32_t)(v >> 62);
-                if (f == 0) {
-                    // predecessor tiles took their ids earlier and are resident: this wait ends
-                    if (++spins > (1u << 26)) {
-                        atomicOr(&a.base->error, 2u);
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(1);
-                    continue;
-                }
-                psh += (uint32_t)((v >> 31) & 0x7fffffffu);
-                psc += (uint32_t)(v & 0x7fffffffu);
-                if (f == 2) break;
-                --j;
-            }
-            __hip_atomic_store(st + tile, pack_status(2, psh + tsh, psc + tsc), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned long long before = look_back(st, tile, pack_status(1, tsh, tsc), &a.base->error);
+        if (lane == 0) {
+            const uint32_t psh = (uint32_t)(before >> 31), psc = (uint32_t)(before & 0x7fffffffu);
+            s_base[0] = psh;
+            s_base[1] = psc;
+            if (tile == ntiles_in - 1)
+                *seg_at(a, bounce, 0) = (unsigned long long)(psh + tsh) << 32 | (psc + tsc);
         }
-        s_base[0] = psh;
-        s_base[1] = psc;
-        if (tile == ntiles_in - 1)
-            *seg_at(a, bounce, 0) = (unsigned long long)(psh + tsh) << 32 | (psc + tsc);
     }
     __syncthreads();
     if (has_sh) {
@@ -1822,7 +1841,7 @@ int launch_pass(gpr_renderer* r, uint32_t log_s, uint32_t parts, hipStream_t st)
         else hipLaunchKernelGGL((k_extend<true, false, false, NT, SL>), tg, tb, 0, ps, a, 0u);
         for (uint32_t b = 0; b < r->opts.max_depth; ++b) {
             if (a.rng_mode == GPR_RNG_REFERENCE)
-                hipLaunchKernelGGL((k_shade<false, true>), dim3(div_up(n, kShadeBlock)), dim3(kShadeBlock), 0, ps, a, b);
+                hipLaunchKernelGGL((k_shade<false, true>), dim3(div_up(n, kOrderedBlock)), dim3(kOrderedBlock), 0, ps, a, b);
             else
                 hipLaunchKernelGGL((k_shade<false, false>), dim3(shade_blocks(n, a.nseg)), dim3(kShadeBlock), 0, ps, a, b);
             if (ref) hipLaunchKernelGGL((k_trace<true, false, NT, SL>), tg, tb, 0, ps, a, b);
