@@ -60,13 +60,15 @@ struct QueueView {
     uint32_t* job;    // multi-job passes: the entry's scene << kJobBits | pass job
 };
 
+constexpr uint32_t kClaimWords = kClaimSets * claim_stride<uint32_t>();
+
 // Per-sample control block (counters cleared by k_gen).
-struct Ctrl {
+struct alignas(kClaimLine) Ctrl {
     uint32_t sample;         // current sample index (single-scene; advanced by k_finish)
     uint32_t error;          // bit0: traversal stack overflow, bit1: look-back timeout
     uint32_t tile_counter[kMaxBounce];
-    uint32_t ext_cursor[kMaxBounce + 1];  // [0] primary, [b+1] scatter queue of bounce b
     uint32_t sh_cursor[kMaxBounce];
+    alignas(kClaimLine) uint32_t claims[kMaxBounce + 1][kClaimWords];  // turns: [0] primary queue, [b+1] queues of bounce b
 };
 
 // Segments of the shadow and scatter queues of an unordered pass: appends take
@@ -256,7 +258,6 @@ __global__ __launch_bounds__(256) void k_gen(RenderArgs a) {
     Ctrl* c = a.ctrl;
     for (uint32_t i = tid; i < kMaxBounce; i += gsz) {
         c->tile_counter[i] = 0u;
-        c->ext_cursor[i + 1] = 0u;
         c->sh_cursor[i] = 0u;
     }
     if constexpr (!MULTI) {
@@ -264,7 +265,8 @@ __global__ __launch_bounds__(256) void k_gen(RenderArgs a) {
             for (uint32_t i = tid; i < kMaxBounce * kLastSpread; i += gsz) a.last[i] = 0ull;
     }
     for (uint32_t i = tid; i < kMaxBounce * a.nseg; i += gsz) a.seg[i * seg_stride(a.nseg)] = 0ull;
-    if (tid == 0) c->ext_cursor[0] = 0u;
+    for (uint32_t i = tid; i < (kMaxBounce + 1) * kClaimSets; i += gsz)
+        (&c->claims[0][0])[i * claim_stride<uint32_t>()] = 0u;
     if (!MULTI && a.rng_mode == GPR_RNG_REFERENCE) {
         const uint32_t used_tiles = (n + kShadeBlock - 1) / kShadeBlock;
         const uint64_t nstat = (uint64_t)a.depth * used_tiles;
@@ -448,7 +450,7 @@ GPR_D void for_each_entry(const RenderArgs& a, uint32_t bounce, uint32_t* cursor
     SegWalk w;
     seg_counts<KIND, MULTI>(a, bounce, w);
     w.init(a.seg_cap, turn_log(w.total(), gridDim.x * (NT / 64), a.chunk_log));
-    for_each_turn<NT, !MULTI>(cursor, w.turns, [&](uint32_t turn) {
+    for_each_turn<NT>(cursor, w.turns, [&](uint32_t turn) {
         uint32_t begin, end;
         w.range(turn, begin, end);
         for (uint32_t i = begin + (threadIdx.x & 63); i < end; i += 64) f(i);
@@ -610,7 +612,7 @@ __global__ __launch_bounds__(NT) void k_extend(RenderArgs a, uint32_t bounce) {
     // queue: primary = A; at bounce b the scatter queue is q[(b+1)&1]
     const QueueView& q = a.q[PRIMARY ? 0 : ((bounce + 1) & 1)];
     constexpr QueueKind kKind = PRIMARY ? kPrimary : kScatter;
-    uint32_t* cur = &a.ctrl->ext_cursor[PRIMARY ? 0 : bounce + 1];
+    uint32_t* cur = a.ctrl->claims[PRIMARY ? 0 : bounce + 1];
     if constexpr (REFILL && !REF_ORDER) {
         uint32_t ei = 0;
         SceneView sv;
@@ -639,7 +641,7 @@ __global__ __launch_bounds__(NT) void k_extend(RenderArgs a, uint32_t bounce) {
             const uint32_t total = w.total();
             if (total <= kQuadEntries) {
                 w.init(a.seg_cap, entries_log(total, gridDim.x * (NT / 64), a.chunk_log, true));
-                for_each_turn<NT, !MULTI>(cur, w.turns, [&](uint32_t turn) {
+                for_each_turn<NT>(cur, w.turns, [&](uint32_t turn) {
                     uint32_t begin, end;
                     w.range(turn, begin, end);
                     const uint32_t i = begin + (threadIdx.x & 63) / 4;
@@ -713,7 +715,7 @@ __global__ __launch_bounds__(NT) void k_trace(RenderArgs a, uint32_t bounce) {
     wx.init(a.seg_cap, lg);
     ws.init(a.seg_cap, lg);
     if (!REF_ORDER && total <= kQuadEntries) {
-        for_each_turn<NT, !MULTI>(&a.ctrl->ext_cursor[bounce + 1], wx.turns + ws.turns, [&](uint32_t turn) {
+        for_each_turn<NT>(a.ctrl->claims[bounce + 1], wx.turns + ws.turns, [&](uint32_t turn) {
             const uint32_t quad = (threadIdx.x & 63) / 4;
             uint32_t begin, end;
             if (turn < wx.turns) {
@@ -737,7 +739,7 @@ __global__ __launch_bounds__(NT) void k_trace(RenderArgs a, uint32_t bounce) {
         });
         return;
     }
-    for_each_turn<NT, !MULTI>(&a.ctrl->ext_cursor[bounce + 1], wx.turns + ws.turns, [&](uint32_t turn) {
+    for_each_turn<NT>(a.ctrl->claims[bounce + 1], wx.turns + ws.turns, [&](uint32_t turn) {
         uint32_t begin, end;
         if (turn < wx.turns) {
             LaneStack<false, SL> st;

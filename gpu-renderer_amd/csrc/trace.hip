@@ -20,6 +20,8 @@ namespace {
 // chunks are used as powers of two (rounded down)
 uint32_t log2_floor(uint32_t v) { return 31u - (uint32_t)__builtin_clz(v); }
 
+constexpr int kCursorWords = kClaimSets * claim_stride<unsigned long long>();  // word 1 counts overflows
+
 __global__ void k_zero_u64(unsigned long long* p, int n) {
     if ((int)threadIdx.x < n) p[threadIdx.x] = 0ull;
 }
@@ -53,7 +55,7 @@ __global__ __launch_bounds__(NT) void k_trace_fast(SceneView sv, const gpr_ray* 
     st.template place<NT>(lds, spill);
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t lg = turn_log(n, gridDim.x * (NT / 64), chunk_log);
-    for_each_turn<NT, false>(cursor, (n + (1ull << lg) - 1) >> lg, [&](uint64_t turn) {
+    for_each_turn<NT>(cursor, (n + (1ull << lg) - 1) >> lg, [&](uint64_t turn) {
         const uint64_t end = min((turn + 1) << lg, n);
         for (uint64_t i = (turn << lg) + lane; i < end; i += 64) {
             gpr_hit h;
@@ -109,6 +111,7 @@ __global__ __launch_bounds__(NT) void k_trace_refill(SceneView sv, const gpr_ray
             uint64_t nb = pe, ne = pe;
             if (avail < cnt && !drained) {
                 unsigned long long b = 0;
+                // one counter: a claim hides behind the lanes still walking (8 counters 2.60 ms, one 2.56)
                 if (lane == 0) b = atomicAdd(cursor, (unsigned long long)chunk);
                 b = claimed_from + __shfl(b, 0, 64);
                 nb = b < n ? b : n;
@@ -181,7 +184,7 @@ __global__ __launch_bounds__(kQuadNT) void k_trace_quad(SceneView sv, const gpr_
     st.template place<kQuadNT>(lds, spill);
     const uint32_t quad = (threadIdx.x & 63) / 4;
     const uint32_t lg = min(turn_log(n, gridDim.x * (kQuadNT / 64), chunk_log), 4u);
-    for_each_turn<kQuadNT, false>(cursor, (n + (1ull << lg) - 1) >> lg, [&](uint64_t turn) {
+    for_each_turn<kQuadNT>(cursor, (n + (1ull << lg) - 1) >> lg, [&](uint64_t turn) {
         const uint64_t i = (turn << lg) + quad;
         if (quad < (1u << lg) && i < n) {
             gpr_hit h;
@@ -321,7 +324,7 @@ int ensure_resources(TraceResources& R) {
         threads = std::max(threads, (size_t)R.grid_quad[a] * kQuadNT / 4);  // a stack for every four lanes
     }
     GPR_TRY(R.spill.alloc(threads * kStackGlobal * sizeof(int2)));
-    GPR_TRY(R.cursor.alloc(4 * sizeof(unsigned long long)));
+    GPR_TRY(R.cursor.alloc(kCursorWords * sizeof(unsigned long long)));
     R.dev = dev;
     return GPR_OK;
 }
@@ -389,7 +392,7 @@ int launch_trace(const SceneView& sv, const gpr_ray* rays, gpr_hit* hits, uint64
         TraceResources* rp = nullptr;
         GPR_TRY(resources_for(st, &rp));
         unsigned long long* cur = rp->cursor.as<unsigned long long>();
-        hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, cur, 4);
+        hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(kCursorWords), 0, st, cur, kCursorWords);
         const dim3 grid((unsigned)std::min<uint64_t>(rp->grid_quad[any ? 1 : 0], n));
         const auto kernel = any ? k_trace_quad<true> : k_trace_quad<false>;
         hipLaunchKernelGGL(kernel, grid, dim3(kQuadNT), 0, st, sv, rays, hits, n, cur, rp->spill.as<int2>(), 4u);
@@ -404,7 +407,7 @@ int launch_trace(const SceneView& sv, const gpr_ray* rays, gpr_hit* hits, uint64
     TraceResources& R = *rp;
     const TraceVariant& v = trace_variant_at(k);
     unsigned long long* cur = R.cursor.as<unsigned long long>();
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, cur, 4);
+    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(kCursorWords), 0, st, cur, kCursorWords);
     const uint64_t want = n;  // a short batch is spread thin: a wave takes one ray at least
     const int kind = (refill ? 2 : 0) + (any ? 1 : 0);
     const TraceKernel ks[4] = {v.closest, v.any, v.closest_r, v.any_r};

@@ -623,40 +623,42 @@ GPR_D uint32_t turn_log(I n, uint32_t waves, uint32_t chunk_log) {
 }
 
 // Hands turns 0 .. n-1 to the waves of the grid and calls f(turn) for each.
-//  - Half of the turns are dealt out in order, the rest is claimed from the
-//    cursor as waves come free: claims are atomics on one address, which
-//    serialise at ~12 ns each on this chip, so claiming every 64 rays bounded
-//    the renderer's big passes.
+//  - Every wave is dealt its first turn and claims the others as it comes free.
+//    Claims are atomics that serialise at ~12 ns on one address, 131 us for the
+//    11,000 claims of a million rays; so there are kClaimSets counters, each
+//    for every kClaimSets-th turn and wave.  Neighbouring turns lie in
+//    different sets, so the sets run out together, and a wave ends with its own:
+//    looking through the others cost more than it evened out.
 //  - A short queue is spread thin over kSpreadWaves waves (four to a SIMD): a
 //    wave takes the union of its lanes' node steps and leaf tests, so thin
-//    waves finish sooner and the chip has room for them (turn_log).
-// Against a claim per 64 rays: 4 samples of the 1920x1080 sphere grid 14.9 ms
-// instead of 16.7 (15.4 with only the first turn dealt out, 15.3 with three
-// quarters), one sample 5.0 instead of 6.5; one sample of an 803x451 textured
-// scene 1.48 ms instead of 2.60 (1.85 unspread, 1.60 / 1.51 / 1.48 over 1024 /
-// 2048 / 4096 waves); 16 of the 256x256 Cornell box 1.61 instead of 2.37.
-// DEAL_HALF asks for a grid that is resident as a whole: a block that starts
-// when others have ended would run its dealt turns alone (a grid one block per
-// CU too large made 4M incoherent rays 24 % slower).  Without it only the first
-// turn is dealt out.
-template <int NT, bool DEAL_HALF, class I, class C, class F>
+//    waves finish sooner and the chip has room for them (turn_log): one sample
+//    of an 803x451 textured scene 1.85 ms unspread, 1.60 / 1.51 / 1.48 over 1024
+//    / 2048 / 4096 waves.
+// One counter with half of the turns dealt out beforehand, then 4 / 8 / 16 sets:
+// 16 samples of the 256x256 Cornell box 1319, then 734 / 685 / 688 us; 8 of the
+// 803x451 textured scene 2842, then 2525 / 2521 / 2523; 8 of a 500x300 sphere grid
+// 2256, then 2146 / 2125 / 2132; the batch of 12 scenes 40.5 ms, then 39.1 / 39.4
+// / 39.3.  8 sets with a search through the others' turns at the end: 1038,
+// 2875, 2327 us and 41.0 ms.
+constexpr uint32_t kClaimSets = 8;
+constexpr uint32_t kClaimLine = 128;  // bytes between two counters
+template <class C>
+GPR_HD constexpr uint32_t claim_stride() { return kClaimLine / sizeof(C); }
+// sets that `waves` waves claim from: every one needs a wave
+GPR_D uint32_t claim_sets(uint32_t waves) { return waves >= kClaimSets ? kClaimSets : 1u; }
+template <int NT, class I, class C, class F>
 GPR_D void for_each_turn(C* cursor, I n, F&& f) {
     const uint32_t waves = gridDim.x * (NT / 64);
-    uint32_t dealt = DEAL_HALF ? (uint32_t)(n / (2 * (I)waves)) : 1u;
-    const I claimed_from = (I)(dealt > 1 ? dealt : 1) * waves;
-    I t = __builtin_amdgcn_readfirstlane(blockIdx.x * (NT / 64) + threadIdx.x / 64);
-    while (t < n) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (NT / 64) + threadIdx.x / 64);
+    const uint32_t sets = claim_sets(waves), set = wave % sets;
+    C* mine = cursor + set * claim_stride<C>();
+    for (I t = wave; t < n;) {
         f(t);
-        if (dealt > 1) {
-            --dealt;
-            t += waves;
-        } else {
-            if (claimed_from >= n) break;
-            C got = 0;
-            if ((threadIdx.x & 63) == 0) got = atomicAdd(cursor, (C)1);
-            if constexpr (sizeof(I) == 4) t = claimed_from + __builtin_amdgcn_readfirstlane(got);
-            else t = claimed_from + (I)__shfl(got, 0, 64);
-        }
+        if (n <= waves) break;
+        C got = 0;
+        if ((threadIdx.x & 63) == 0) got = atomicAdd(mine, (C)1);
+        if constexpr (sizeof(I) == 4) t = waves + __builtin_amdgcn_readfirstlane(got) * sets + set;
+        else t = waves + (I)__shfl(got, 0, 64) * sets + set;
     }
 }
 
