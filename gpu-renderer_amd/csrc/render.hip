@@ -577,12 +577,12 @@ GPR_D void shadow_finish(const RenderArgs& a, const QueueView& q, uint32_t i, co
 }
 
 // A queue this short walks its rays with four lanes each (quad_trace): a launch
-// then takes as long as its longest walk.  Renders of 57,000 paths of the
-// textured scene and 60,000 of the sphere grid 1000 -> 890 and 1232 -> 1054 us, a
-// 300x200 frame 746 -> 650 us; 12-job batch 41.1 -> 40.6 ms, 16 served jobs 141
-// -> 138 ms (late bounces).  Lines at 2^17 / 2^18 entries: batch 40.4 / 41.4 ms,
-// but the 256x256 Cornell box, whose walks are short, 1.46 ms instead of 1.40.
-constexpr uint32_t kQuadEntries = 1u << 16;
+// then takes as long as its longest walk.  Never / up to 2^16 / 2^17 entries: 57,000
+// paths of the textured scene 1000 / 845 / 800 us, 60,000 of the sphere grid 1232 /
+// 1018 / 980, a 300x200 frame 746 / 620 / 593; 12-job batch 41.1 / 40.6 ms, then
+// with cheaper turns 39.4 / 39.0; 16 served jobs 141 / 137 ms.  3 * 2^15 entries:
+// 802, 1022, 620 us; 3 * 2^16: 801, 974, 594 us, but served jobs 138 ms for 136.5.
+constexpr uint32_t kQuadEntries = 1u << 17;
 // log2 of the entries of a turn: turn_log, or at most 16 where four lanes take one
 GPR_D uint32_t entries_log(uint32_t total, uint32_t waves, uint32_t chunk_log, bool quads) {
     const uint32_t lg = turn_log(total, waves, chunk_log);

@@ -50,9 +50,9 @@ def test_four_lanes_to_a_ray(ntri, n, any_hit):
     s.free()
 
 
-@pytest.mark.parametrize("name,w,h,spp", [("spheres", 256, 256, 4), ("textured", 257, 255, 3), ("spheres", 91, 90, 8)])
+@pytest.mark.parametrize("name,w,h,spp", [("spheres", 256, 256, 4), ("textured", 257, 255, 3), ("spheres", 91, 90, 8), ("spheres", 181, 182, 8)])
 def test_short_queues_of_a_render(name, w, h, spp):
-    # one sample a pass keeps the queues at or below 2^16 entries (four lanes to an entry), all of them in one exceed it
+    # one sample a pass keeps the queues below 2^17 entries (four lanes to an entry), all of them in one mostly exceed it
     import gpu_scenes as G
     s = gpr.Scene.sphere_grid(w, h, 6) if name == "spheres" else G.textured(w, h).commit()
     o = dict(max_depth=8, rr_start=3, seed=3)
