@@ -18,9 +18,9 @@
 //            halves of a histogram tile run on one XCD.
 //   local    one block per bucket staged in LDS: MSD split on the next 10 key
 //            bits into 1024 sub-buckets (~1 element each), then every
-//            composite is placed by its rank among its sub-bucket.  Buckets
-//            with a crowded sub-bucket, or too large for LDS, use LDS bitonic
-//            chunk sorts and pairwise merges.
+//            composite is placed by its rank among its sub-bucket.  A bucket
+//            too large for LDS is cut into pieces of whole sub-buckets, which
+//            the blocks take between them.
 // Every bucket block zeroes its digit total once it has read it, so each call
 // leaves the totals cleared for the next call in stream order: eager calls and
 // replays of captured graphs (of any number of sorts) may interleave freely.
@@ -55,6 +55,12 @@ constexpr int kSub = 1024;          // sub-buckets of the LDS MSD split
 constexpr int kSubMax = 48;         // largest sub-bucket sorted by one thread
 constexpr uint32_t kWin = 4;        // sub-bucket entries a rank reads at once
 static_assert(kSub % kLocalThreads == 0, "sub-bucket scan: whole counts per thread");
+constexpr uint32_t kWinStep = 1536;   // piece starts fall on sub-bucket starts past multiples of this
+constexpr uint32_t kMaxTodo = 16;     // ranges of a piece yet to do: a level takes one and adds three at most, of seven levels
+constexpr uint32_t kRankMax = 1024;   // largest sub-bucket placed by rank (O(size) LDS reads per entry)
+constexpr uint32_t kPieceMax = kWinStep + kRankMax;
+static_assert(kPieceMax + kSub / 2 <= 2 * kFastCap, "a piece and its sub-buckets' places must fit the LDS buffer");
+GPR_HD constexpr uint32_t pieces_of(uint32_t n) { return n > (uint32_t)kFastCap ? (n + kWinStep - 1) / kWinStep : 0u; }
 
 // Top-digit width: ~1K keys per bucket, between 1 and 11 bits.
 uint32_t digit_bits(uint32_t n) {
@@ -205,6 +211,7 @@ __global__ __launch_bounds__(kScatterThreads) void k_scatter(const uint32_t* __r
     __shared__ uint32_t lcnt[kMaxDigits];  // digit counts of the sub-tile, then local starts
     __shared__ unsigned long long stage[kSubTile];
     __shared__ uint32_t sh[2 * NT / 64];
+    __shared__ uint32_t pieces;
     const uint32_t sub = sub_of_block(blockIdx.x);
     const uint64_t b0 = (uint64_t)sub * kSubTile;
     if (b0 >= n) return;  // padding blocks of the XCD mapping
@@ -241,6 +248,7 @@ __global__ __launch_bounds__(kScatterThreads) void k_scatter(const uint32_t* __r
         }
     }
     for (uint32_t d = threadIdx.x; d < nd; d += NT) lcnt[d] = 0;
+    if (threadIdx.x == 0) pieces = 0;
     __syncthreads();
     // rank of every key among the sub-tile's keys of its digit
     uint32_t r[KPT];
@@ -269,7 +277,9 @@ __global__ __launch_bounds__(kScatterThreads) void k_scatter(const uint32_t* __r
             if ((uint32_t)x < per) {
                 lcnt[d0 + x] = lex;
                 gpos[d0 + x] = ex + p[x] + o[x] - lex;
-                if (sub == 0) bases[d0 + x] = make_uint2(ex, a[x]);
+                if (sub == 0) {
+                    bases[d0 + x] = make_uint2(ex, a[x]);
+                }
                 ex += a[x];
                 lex += l[x];
             }
@@ -295,224 +305,200 @@ __global__ __launch_bounds__(kScatterThreads) void k_scatter(const uint32_t* __r
                                __HIP_MEMORY_SCOPE_AGENT);
         }
     }
+    if (sub == 0) {
+        uint32_t large = 0;
+#pragma unroll
+        for (int x = 0; x < kPer; ++x) large += pieces_of(a[x]);
+        if (large) atomicAdd(&pieces, large);
+        __syncthreads();
+        if (threadIdx.x == 0) bases[kMaxDigits] = make_uint2(pieces, 0u);
+    }
 }
 
-GPR_D void bitonic_lds(unsigned long long* s, uint32_t P) {
-    for (uint32_t k = 2; k <= P; k <<= 1) {
-        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            for (uint32_t i = threadIdx.x; i < (P >> 1); i += kLocalThreads) {
-                const uint32_t a = ((i & ~(j - 1)) << 1) | (i & (j - 1));
-                const uint32_t b = a + j;
-                const unsigned long long x = s[a], y = s[b];
-                if ((x > y) == ((a & k) == 0)) {
-                    s[a] = y;
-                    s[b] = x;
-                }
-            }
+// f(entry) for the n entries at src, in 16-byte loads, kBatch of them in
+// flight per thread.
+template <class F>
+GPR_D void each_entry(const unsigned long long* src, uint32_t n, F&& f) {
+    constexpr uint32_t kBatch = 4;
+    const uint32_t head = (uint32_t)(reinterpret_cast<uintptr_t>(src) >> 3) & 1u;  // 1: the first pair starts before src
+    const ulonglong2* p = reinterpret_cast<const ulonglong2*>(src - head);
+    const uint32_t end = n + head, pairs = (end + 1) / 2;
+    for (uint32_t base = 0; base < pairs; base += kBatch * kLocalThreads) {
+        ulonglong2 v[kBatch];
+#pragma unroll
+        for (uint32_t j = 0; j < kBatch; ++j) {
+            const uint32_t i = base + j * kLocalThreads + threadIdx.x;
+            v[j] = i < pairs ? p[i] : make_ulonglong2(0, 0);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kBatch; ++j) {
+            const uint32_t e = 2 * (base + j * kLocalThreads + threadIdx.x);
+            if (e >= head && e < end) f(v[j].x);
+            if (e + 1 < end) f(v[j].y);
+        }
+    }
+}
+
+// A range of a bucket: the entries whose bits under `mask` are `value`, with
+// `base` entries of the bucket below them.
+struct SortNode {
+    unsigned long long mask, value;
+    uint32_t base;
+};
+struct PieceLds {
+    unsigned long long buf[2 * kFastCap];
+    uint32_t cnt[kSub], start[kSub + 1];
+    uint32_t sh[kLocalThreads / 64];
+    SortNode todo[kMaxTodo];
+    uint32_t ntodo;
+    unsigned long long all, any;  // AND and OR of a range's entries
+};
+// Piece q of a bucket of n composites at src (any order): what belongs at its
+// places q * kWinStep to (q + 1) * kWinStep, in whole sub-buckets.  The block
+// counts a range's sub-buckets, the bucket's own by the key bits below the top
+// digit.  Those of up to kRankMax entries that start in the piece it collects
+// in LDS and places by rank; larger ones that the piece overlaps are ranges of
+// their own, split by the highest 10 bits in which their entries differ
+// (composites are all different, so this ends).
+// The bucket is read twice for every piece, and three times more for a range
+// inside it.  That costs less than a split by one block with its windows one
+// after another, which made a bucket take the time of one compute unit, and no
+// block waits for another.   One
+// block a bucket against this: 1M / 399,952 / 20,000 keys in 64 clusters 11.1 ms /
+// 6,861 us / 305 us -> 427 / 266 / 52; 1M equal keys 58.4 -> 2.5 ms; a rebuild of the
+// 254K-triangle sphere grid 208 -> 190 us.  Uniform keys pay for the look at the
+// bucket sizes: 1M of them 18.35 -> 18.46 us.
+GPR_D void sort_piece(const unsigned long long* src, uint32_t n, uint32_t q, uint32_t sub_shift, uint32_t nsub,
+                      uint32_t* __restrict__ skeys, uint32_t* __restrict__ sidx, PieceLds& L) {
+    const uint32_t p0 = q * kWinStep, p1 = p0 + kWinStep;
+    uint32_t* at_of = reinterpret_cast<uint32_t*>(L.buf + kPieceMax);  // a sub-bucket's place in the buffer
+    __syncthreads();  // the LDS is free
+    if (threadIdx.x == 0) {
+        L.todo[0] = SortNode{0ull, 0ull, 0u};
+        L.ntodo = 1;
+    }
+    __syncthreads();
+    for (bool whole = true;; whole = false) {
+        const uint32_t left = L.ntodo;
+        if (left == 0) break;
+        const SortNode node = L.todo[left - 1];
+        __syncthreads();
+        for (uint32_t s = threadIdx.x; s < kSub; s += kLocalThreads) L.cnt[s] = 0;
+        if (threadIdx.x == 0) {
+            L.ntodo = left - 1;
+            L.all = ~0ull;
+            L.any = 0ull;
+        }
+        __syncthreads();
+        const auto inside = [&](unsigned long long v) { return (v & node.mask) == node.value; };
+        uint32_t shift = sub_shift, nd = nsub;
+        if (!whole) {
+            unsigned long long all = ~0ull, any = 0ull;
+            each_entry(src, n, [&](unsigned long long v) {
+                all &= inside(v) ? v : ~0ull;
+                any |= inside(v) ? v : 0ull;
+            });
+            atomicAnd(&L.all, all);
+            atomicOr(&L.any, any);
             __syncthreads();
+            const uint32_t top = 63u - (uint32_t)__clzll((long long)(L.all ^ L.any));
+            shift = top > 9u ? top - 9u : 0u;
+            nd = 2u << (top - shift);
         }
-    }
-}
-
-GPR_D uint32_t lower_bound_u64(const unsigned long long* a, uint32_t n, unsigned long long v) {
-    uint32_t lo = 0, hi = n;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (a[mid] < v) lo = mid + 1;
-        else hi = mid;
-    }
-    return lo;
-}
-
-// Sorts x[0, n) (composites) into skeys / sidx[0, n): LDS bitonic sorts of
-// 2048-entry chunks, then pairwise merges through y[0, n) (global scratch).
-// The general fallback: any size, any key distribution.
-GPR_D void sort_range_merge(unsigned long long* x, unsigned long long* y, uint32_t n, unsigned long long* buf,
-                            uint32_t* __restrict__ skeys, uint32_t* __restrict__ sidx) {
-    constexpr uint32_t kChunk = 2048;
-    for (uint32_t c0 = 0; c0 < n; c0 += kChunk) {
-        const uint32_t m = min(kChunk, n - c0);
-        for (uint32_t i = threadIdx.x; i < kChunk; i += kLocalThreads) buf[i] = i < m ? x[c0 + i] : ~0ull;
+        const auto digit = [&](unsigned long long v) { return (uint32_t)(v >> shift) & (nd - 1); };
+        each_entry(src, n, [&](unsigned long long v) {
+            if (!inside(v)) return;
+            // equal digits in a whole wave: one atomic
+            const uint32_t d = digit(v), d0 = __builtin_amdgcn_readfirstlane(d);
+            const unsigned long long here = __ballot(true);
+            if (__ballot(d == d0) != here) atomicAdd(&L.cnt[d], 1u);
+            else if ((threadIdx.x & 63) == (uint32_t)__builtin_ctzll(here)) atomicAdd(&L.cnt[d], (uint32_t)__popcll(here));
+        });
         __syncthreads();
-        bitonic_lds(buf, kChunk);
-        for (uint32_t i = threadIdx.x; i < m; i += kLocalThreads) x[c0 + i] = buf[i];
-        __syncthreads();
-    }
-    for (uint32_t w = kChunk; w < n; w <<= 1) {
-        for (uint32_t e = threadIdx.x; e < n; e += kLocalThreads) {
-            const uint32_t r0 = (e / (2 * w)) * (2 * w);
-            const uint32_t mid = min(r0 + w, n), end = min(r0 + 2 * w, n);
-            const unsigned long long v = x[e];
-            const uint32_t o = e < mid ? (e - r0) + lower_bound_u64(x + mid, end - mid, v)
-                                       : (e - mid) + lower_bound_u64(x + r0, mid - r0, v);
-            y[r0 + o] = v;
-        }
-        __syncthreads();
-        unsigned long long* t = x;
-        x = y;
-        y = t;
-    }
-    for (uint32_t i = threadIdx.x; i < n; i += kLocalThreads) {
-        const unsigned long long v = x[i];
-        skeys[i] = (uint32_t)(v >> 32);
-        sidx[i] = (uint32_t)v;
-    }
-    __syncthreads();
-}
-
-// First sub-bucket start >= pos (starts are non-decreasing; an empty
-// sub-bucket starts where the next one does), or n.
-GPR_D uint32_t first_start_at(const uint32_t* start, uint32_t nsub, uint32_t n, uint32_t pos) {
-    uint32_t lo = 0, hi = nsub;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (start[mid] < pos) lo = mid + 1;
-        else hi = mid;
-    }
-    return lo < nsub ? start[lo] : n;
-}
-
-constexpr uint32_t kWinStep = 1536;   // window starts fall on sub-bucket starts past multiples of this
-constexpr uint32_t kRankMax = 1024;   // largest sub-bucket placed by rank (O(size) LDS reads per entry)
-static_assert(kWinStep + kRankMax <= 2 * kFastCap, "a window must fit the LDS buffer");
-
-// A bucket of n composites at src (any order, any size): split by the
-// sub-bucket digit (key bits below the top digit) into dst = the bucket's
-// range of the scratch, then cut the split into windows of whole
-// consecutive sub-buckets (each starts at the first sub-bucket start at or
-// past a multiple of kWinStep, so it holds at most kWinStep + kRankMax - 1
-// entries when no sub-bucket exceeds kRankMax) and place every entry of a
-// window by its rank among its sub-bucket, all in LDS.  A window with a
-// sub-bucket above kRankMax is sorted by sort_range_merge, with src (free
-// after the split) as its scratch.
-GPR_D void large_bucket(unsigned long long* src, unsigned long long* dst, uint32_t n, uint32_t sub_shift,
-                        uint32_t nsub, uint32_t* __restrict__ skeys, uint32_t* __restrict__ sidx,
-                        unsigned long long* buf, uint32_t* cnt, uint32_t* start, uint32_t* sh, uint32_t* flag) {
-    // global reads in batches of kBatch per thread, all in flight before their first use
-    constexpr uint32_t kBatch = 8;
-    for (uint32_t s = threadIdx.x; s < kSub; s += kLocalThreads) cnt[s] = 0;
-    __syncthreads();
-    for (uint32_t base = 0; base < n; base += kBatch * kLocalThreads) {
-        unsigned long long v[kBatch];
+        constexpr int kQ = kSub / kLocalThreads;
+        uint32_t c[kQ], sum = 0, tot;
 #pragma unroll
-        for (uint32_t j = 0; j < kBatch; ++j) {
-            const uint32_t i = base + j * kLocalThreads + threadIdx.x;
-            v[j] = i < n ? src[i] : 0ull;
-        }
+        for (int k = 0; k < kQ; ++k) sum += c[k] = L.cnt[kQ * threadIdx.x + k];
+        const uint32_t size_end = scan_incl<kLocalThreads>(sum, L.sh, &tot);
+        // the sub-buckets that start in the piece, and the large ones that reach into it
+        uint32_t first = node.base + size_end - sum, mine = 0, at[kQ];
 #pragma unroll
-        for (uint32_t j = 0; j < kBatch; ++j)
-            if (base + j * kLocalThreads + threadIdx.x < n) atomicAdd(&cnt[(uint32_t)(v[j] >> sub_shift) & (nsub - 1)], 1u);
-    }
-    __syncthreads();
-    constexpr int kQ = kSub / kLocalThreads;
-    uint32_t cq[kQ], sq = 0;
-#pragma unroll
-    for (int k = 0; k < kQ; ++k) {
-        cq[k] = cnt[kQ * threadIdx.x + k];
-        sq += cq[k];
-    }
-    uint32_t tot;
-    uint32_t run = scan_incl<kLocalThreads>(sq, sh, &tot) - sq;
-    uint32_t* fill = reinterpret_cast<uint32_t*>(buf);  // buf is free during the split
-#pragma unroll
-    for (int k = 0; k < kQ; ++k) {
-        start[kQ * threadIdx.x + k] = run;
-        fill[kQ * threadIdx.x + k] = 0;
-        run += cq[k];
-    }
-    __syncthreads();
-    for (uint32_t base = 0; base < n; base += kBatch * kLocalThreads) {
-        unsigned long long v[kBatch];
-#pragma unroll
-        for (uint32_t j = 0; j < kBatch; ++j) {
-            const uint32_t i = base + j * kLocalThreads + threadIdx.x;
-            v[j] = i < n ? src[i] : 0ull;
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < kBatch; ++j) {
-            if (base + j * kLocalThreads + threadIdx.x < n) {
-                const uint32_t sb = (uint32_t)(v[j] >> sub_shift) & (nsub - 1);
-                dst[start[sb] + atomicAdd(&fill[sb], 1u)] = v[j];
+        for (int k = 0; k < kQ; ++k) {
+            const uint32_t d = kQ * threadIdx.x + k;
+            L.start[d] = first;
+            at[k] = ~0u;
+            if (c[k] > kRankMax) {
+                if (first < p1 && first + c[k] > p0)
+                    L.todo[atomicAdd(&L.ntodo, 1u)] =
+                        SortNode{node.mask | (unsigned long long)(nd - 1) << shift,
+                                 node.value | (unsigned long long)d << shift, first};
+            } else if (c[k] != 0 && first >= p0 && first < p1) {
+                at[k] = mine;
+                mine += c[k];
             }
+            first += c[k];
         }
-    }
-    __syncthreads();  // the split is in dst, seen by every thread of the block
-    const uint32_t nw = (n + kWinStep - 1) / kWinStep;
-    for (uint32_t w = 0; w < nw; ++w) {
-        const uint32_t lo = first_start_at(start, nsub, n, w * kWinStep);
-        const uint32_t hi = first_start_at(start, nsub, n, (w + 1) * kWinStep);
-        const uint32_t m = hi - lo;
+        if (threadIdx.x == kLocalThreads - 1) L.start[kSub] = first;
+        const uint32_t mine_end = scan_incl<kLocalThreads>(mine, L.sh, &tot);
+#pragma unroll
+        for (int k = 0; k < kQ; ++k) at_of[kQ * threadIdx.x + k] = at[k] == ~0u ? ~0u : at[k] + mine_end - mine;
+        const uint32_t m = tot;
+        __syncthreads();
         if (m == 0) continue;
-        if (threadIdx.x == 0) *flag = m > 2u * kFastCap ? 1u : 0u;
+        each_entry(src, n, [&](unsigned long long v) {
+            const uint32_t d = digit(v);
+            if (inside(v) && at_of[d] != ~0u) L.buf[at_of[d] + atomicSub(&L.cnt[d], 1u) - 1u] = v;
+        });
         __syncthreads();
-        if (*flag == 0) {
-            constexpr uint32_t kW = (2 * kFastCap + kLocalThreads - 1) / kLocalThreads;
-            unsigned long long v[kW];
-#pragma unroll
-            for (uint32_t j = 0; j < kW; ++j) {
-                const uint32_t i = j * kLocalThreads + threadIdx.x;
-                v[j] = i < m ? dst[lo + i] : 0ull;
-            }
-#pragma unroll
-            for (uint32_t j = 0; j < kW; ++j) {
-                const uint32_t i = j * kLocalThreads + threadIdx.x;
-                if (i < m) {
-                    buf[i] = v[j];
-                    if (cnt[(uint32_t)(v[j] >> sub_shift) & (nsub - 1)] > kRankMax) *flag = 1u;
-                }
-            }
-        }
-        __syncthreads();
-        if (*flag != 0) {
-            sort_range_merge(dst + lo, src + lo, m, buf, skeys + lo, sidx + lo);
-            continue;
-        }
         for (uint32_t j = threadIdx.x; j < m; j += kLocalThreads) {
-            const unsigned long long v = buf[j];
-            const uint32_t sb = (uint32_t)(v >> sub_shift) & (nsub - 1);
-            const uint32_t b = start[sb] - lo, c = cnt[sb];
+            const unsigned long long v = L.buf[j];
+            const uint32_t d = digit(v), b = at_of[d];
             // 8 independent LDS reads per step: the loop is bound by LDS
             // latency, not by the compares
+            const uint32_t e = L.start[d + 1] - L.start[d];
             uint32_t rank = 0, x = 0;
-            for (; x + 8 <= c; x += 8) {
+            for (; x + 8 <= e; x += 8) {
                 unsigned long long a[8];
 #pragma unroll
-                for (int u = 0; u < 8; ++u) a[u] = buf[b + x + u];
+                for (int u = 0; u < 8; ++u) a[u] = L.buf[b + x + u];
 #pragma unroll
                 for (int u = 0; u < 8; ++u) rank += a[u] < v ? 1u : 0u;
             }
-            for (; x < c; ++x) rank += buf[b + x] < v ? 1u : 0u;
-            skeys[start[sb] + rank] = (uint32_t)(v >> 32);
-            sidx[start[sb] + rank] = (uint32_t)v;
+            for (; x < e; ++x) rank += L.buf[b + x] < v ? 1u : 0u;
+            __hip_atomic_store(&skeys[L.start[d] + rank], (uint32_t)(v >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&sidx[L.start[d] + rank], (uint32_t)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        __syncthreads();  // buf is reloaded by the next window
+        __syncthreads();
     }
 }
 
-// ---- local: one bucket per block, LDS MSD split + rank inside each sub-bucket
-__global__ __launch_bounds__(kLocalThreads) void k_local(uint32_t shift, uint32_t* __restrict__ acc,
+// ---- local: one bucket per block, LDS MSD split + rank inside each
+// sub-bucket; then the block's share of the pieces of the large buckets
+__global__ __launch_bounds__(kLocalThreads, 8) void k_local(uint32_t shift, uint32_t nd, uint32_t* __restrict__ acc,
                                                          const uint2* __restrict__ bases,
-                                                         unsigned long long* __restrict__ tmp,
-                                                         unsigned long long* __restrict__ alt,
+                                                         const unsigned long long* __restrict__ tmp,
                                                          uint32_t* __restrict__ skeys,
                                                          uint32_t* __restrict__ sidx) {
-    __shared__ unsigned long long buf[2 * kFastCap];  // A | B
-    __shared__ uint32_t cnt[kSub];
-    __shared__ uint32_t start[kSub];
-    __shared__ uint32_t sh[kLocalThreads / 64];
+    __shared__ PieceLds L;
+    unsigned long long* buf = L.buf;  // A | B
+    uint32_t* cnt = L.cnt;
+    uint32_t* start = L.start;
+    uint32_t* sh = L.sh;
     __shared__ uint32_t crowded;
+    __shared__ uint32_t piece[3];  // first slot and size of its bucket, number in the bucket
     const uint32_t d = blockIdx.x;
     // the bucket's base and size, as the scatter pass computed them
     const uint2 bn = bases[d];
     const uint32_t b0 = bn.x, n = bn.y;
+    const uint32_t pieces = bases[kMaxDigits].x;  // of all buckets
     // the reservation counters start from zero in the next call
     if (threadIdx.x < kGroups) acc[acc_at(d, threadIdx.x)] = 0u;
-    if (n == 0) return;
-    unsigned long long* src = tmp + b0;
+    if (n == 0 && __builtin_expect(pieces == 0, 1)) return;
+    const unsigned long long* src = tmp + b0;
     const uint32_t sub_bits = min(10u, shift);
     const uint32_t nsub = 1u << sub_bits;
     const uint32_t sub_shift = 32 + shift - sub_bits;
-    if (n <= (uint32_t)kFastCap) {
+    if (n != 0 && n <= (uint32_t)kFastCap) {
         unsigned long long* A = buf;
         unsigned long long* B = buf + kFastCap;
         // all loads in flight before the first LDS use
@@ -586,26 +572,50 @@ __global__ __launch_bounds__(kLocalThreads) void k_local(uint32_t shift, uint32_
                     __hip_atomic_store(&sidx[b0 + i], (uint32_t)w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
             }
-            return;
+            if (__builtin_expect(pieces == 0, 1)) return;
+        } else {
+            sort_piece(src, n, 0, sub_shift, nsub, skeys + b0, sidx + b0, L);
         }
     }
-    // Oversized bucket, or a crowded sub-bucket: a second MSD split on the
-    // same next key bits, through the scratch `alt`, then windows of
-    // consecutive sub-buckets staged in LDS and placed by rank.
-    large_bucket(src, alt + b0, n, sub_shift, nsub, skeys + b0, sidx + b0, buf, cnt, start, sh, &crowded);
+    constexpr int kDigits = kMaxDigits / kLocalThreads;  // digits per thread at most
+    const uint32_t per = nd >= (uint32_t)kLocalThreads ? nd / kLocalThreads : 1u;
+    for (uint32_t w = d; w < pieces; w += nd) {
+        uint2 l[kDigits];
+        uint32_t sum = 0, tot;
+#pragma unroll
+        for (int x = 0; x < kDigits; ++x) {
+            const uint32_t i = threadIdx.x * per + x;
+            l[x] = (uint32_t)x < per && i < nd ? bases[i] : make_uint2(0u, 0u);
+            sum += pieces_of(l[x].y);
+        }
+        __syncthreads();  // sh and piece are free
+        uint32_t first = scan_incl<kLocalThreads>(sum, sh, &tot) - sum;
+#pragma unroll
+        for (int x = 0; x < kDigits; ++x) {
+            const uint32_t k = pieces_of(l[x].y);
+            if (w - first < k) {
+                piece[0] = l[x].x;
+                piece[1] = l[x].y;
+                piece[2] = w - first;
+            }
+            first += k;
+        }
+        __syncthreads();
+        const uint32_t p0 = piece[0];
+        sort_piece(tmp + p0, piece[1], piece[2], sub_shift, nsub, skeys + p0, sidx + p0, L);
+    }
 }
 
 struct Layout {
     uint32_t* acc;
-    uint2* bases;     // per bucket: first slot, size
+    uint2* bases;     // per bucket: first slot, size; then the pieces of all large buckets
     uint32_t* off;
     unsigned long long* tmp;
-    unsigned long long* alt;
 };
 // Byte offsets of the scratch arrays for n keys, each on a 256-B boundary
 // (constexpr: the no-allocation entry point sizes its fixed array with it).
 struct Offsets {
-    size_t acc, bases, off, tmp, alt, total;
+    size_t acc, bases, off, tmp, total;
 };
 constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 constexpr Offsets offsets(uint32_t n) {
@@ -614,10 +624,9 @@ constexpr Offsets offsets(uint32_t n) {
     Offsets o{};
     o.acc = 0;
     o.bases = align256(o.acc + 4ull * kAccWords);
-    o.off = align256(o.bases + 8ull * kMaxDigits);
+    o.off = align256(o.bases + 8ull * (kMaxDigits + 1));
     o.tmp = align256(o.off + 4ull * kMaxDigits * kSubs * ntiles);
-    o.alt = align256(o.tmp + 8ull * nk);
-    o.total = o.alt + 8ull * nk + 256;
+    o.total = align256(o.tmp + 8ull * nk) + 256;
     return o;
 }
 size_t layout(uint32_t n, char* base, Layout* L) {
@@ -627,7 +636,6 @@ size_t layout(uint32_t n, char* base, Layout* L) {
         L->bases = reinterpret_cast<uint2*>(base + o.bases);
         L->off = reinterpret_cast<uint32_t*>(base + o.off);
         L->tmp = reinterpret_cast<unsigned long long*>(base + o.tmp);
-        L->alt = reinterpret_cast<unsigned long long*>(base + o.alt);
     }
     return o.total;
 }
@@ -662,8 +670,8 @@ int sort_pairs(const uint32_t* keys, uint32_t* skeys, uint32_t* sidx, uint32_t n
     const uint32_t nsub_blocks = div_up(ntiles, kXcds) * kXcds * kSubs;
     hipLaunchKernelGGL(k_scatter, dim3(nsub_blocks), dim3(kScatterThreads), 0, st, keys, n, shift, nd,
                        L.acc, L.off, L.bases, L.tmp);
-    hipLaunchKernelGGL(k_local, dim3(nd), dim3(kLocalThreads), 0, st, shift, L.acc, L.bases, L.tmp,
-                       L.alt, skeys, sidx);
+    hipLaunchKernelGGL(k_local, dim3(nd), dim3(kLocalThreads), 0, st, shift, nd, L.acc, L.bases, L.tmp,
+                       skeys, sidx);
     GPR_HIP(hipGetLastError());
     return GPR_OK;
 }
@@ -673,7 +681,7 @@ int sort_pairs(const uint32_t* keys, uint32_t* skeys, uint32_t* sidx, uint32_t n
 // ---- the sort without allocation ------------------------------------------
 // A fixed device array holds the scratch of sorts of up to kNoAllocMaxKeys
 // keys, so gpr_sort_pairs_device_noalloc calls neither hipMalloc nor hipFree.
-// Each GPU holds its own copy of the array until the process ends (18.9 MB);
+// Each GPU holds its own copy of the array until the process ends (10.5 MB);
 // every call on a GPU shares it.
 namespace {
 constexpr uint32_t kNoAllocMaxKeys = 1u << 20;

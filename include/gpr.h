@@ -253,7 +253,7 @@ int gpr_sort_pairs_device(const uint32_t* keys, uint32_t* sorted_keys, uint32_t*
  * reference: it is for callers that cannot allocate device memory (code under
  * hipGraph capture, serving loops, harnesses that forbid hipMalloc).  Same
  * arguments and results as gpr_sort_pairs_device; its scratch is a fixed
- * device array of 18.9 MB per GPU, held until the process ends, so n is at
+ * device array of 10.5 MB per GPU, held until the process ends, so n is at
  * most 1,048,576 (larger n fails with GPR_ERR_INVALID).  Every call on one GPU
  * shares that array: calls that overlap on one GPU (different streams or
  * threads without ordering between them) race and give wrong results. */
