@@ -27,6 +27,7 @@
 // path, so the read-modify-write needs no atomics).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -1450,6 +1451,10 @@ int engine_set_scenes(Engine* e, const std::vector<SceneView>& views, hipStream_
 }
 
 namespace {
+// Blocks of a configuration's traversal kernels whose walks may overflow to `bytes`.
+uint32_t blocks_of_spill(int kidx, uint64_t bytes) {
+    return (uint32_t)(bytes / (pass_kernel_table(kidx).nt * kStackGlobal * sizeof(int2)));
+}
 // Launch grids cover `size` paths (the pass's size class), not the capacity:
 // a small pass launches small grids.
 int record_pass(Engine* e, uint32_t depth, int kidx, uint32_t chunk, uint32_t size, float4* fb, bool terms,
@@ -1476,7 +1481,8 @@ int record_pass(Engine* e, uint32_t depth, int kidx, uint32_t chunk, uint32_t si
         RenderArgs a = pass;
         const uint32_t n = set_part(a, size, parts, part, true, e->side_spill.as<int2>());
         const hipStream_t ps = part ? e->side.s : st;
-        const dim3 tg(std::min<uint32_t>(e->grid[kidx], div_up(n, pk.nt))), tb(pk.nt);
+        const uint32_t most = blocks_of_spill(kidx, part ? e->side_spill.bytes : e->spill.bytes);
+        const dim3 tg(std::min({(uint32_t)e->grid[kidx], most, div_up(n, pk.nt)})), tb(pk.nt);
         hipLaunchKernelGGL(k_gen<true>, dim3(div_up(n, 256)), dim3(256), 0, ps, a);
         hipLaunchKernelGGL(pk.ext_primary, tg, tb, 0, ps, a, 0u);
         for (uint32_t b = 0; b < depth; ++b) {
@@ -1494,18 +1500,18 @@ int record_pass(Engine* e, uint32_t depth, int kidx, uint32_t chunk, uint32_t si
 }  // namespace
 
 namespace {
-// Stack overflow area of the second part's walks.
-uint64_t side_bytes(const Engine* e, int kidx) {
-    return (uint64_t)e->grid[kidx] * pass_kernel_table(kidx).nt * kStackGlobal * sizeof(int2);
-}
 // Whether a pass can run as two parts: the second one's area is there, or can
 // be allocated (once, at its largest, as captured passes hold its address).
+// The grid of the second part is what the area holds (record_pass): a server
+// reserves it for one configuration, and others have up to 1.75 times its threads.
+// 16 requests with 64-thread blocks and 8 entries 154 ms in one part, 147-151 so,
+// 149-150 with an area for all of them.
 bool side_ready(Engine* e, int kidx) {
     if (e->side_grows && !e->side_spill.p) {
         e->side_grows = false;
         if (e->side_spill.alloc(e->spill.bytes) != GPR_OK) (void)hipGetLastError();  // the failed allocation
     }
-    return e->side_spill.bytes >= side_bytes(e, kidx) && e->side.make() == GPR_OK;
+    return blocks_of_spill(kidx, e->side_spill.bytes) > 0 && e->side.make() == GPR_OK;
 }
 // Launch size class of a pass: its paths rounded up to a power of two.
 uint32_t size_class(const Engine* e, uint64_t paths) {
@@ -1581,7 +1587,8 @@ void engine_limit_terms(Engine* e, uint64_t bytes) {
 
 uint64_t engine_side_bytes(const Engine* e) {
     if (parts_for(e->capacity, true) == 1) return 0;
-    return side_bytes(e, pass_kernel_index(TraceCfg{256, 16, 64, 0, 0}));
+    const int kidx = pass_kernel_index(TraceCfg{256, 16, 64, 0, 0});
+    return (uint64_t)e->grid[kidx] * pass_kernel_table(kidx).nt * kStackGlobal * sizeof(int2);
 }
 int engine_reserve_side(Engine* e) {
     if (e->side_spill.alloc(engine_side_bytes(e)) == GPR_OK) return GPR_OK;
