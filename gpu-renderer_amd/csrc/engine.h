@@ -51,9 +51,10 @@ size_t engine_device_bytes(const Engine* e);
 int engine_set_scenes(Engine* e, const std::vector<SceneView>& views, hipStream_t st);
 // Term lists of passes of more than one sample a job.  They grow on use, up to
 // the limit (0 bytes: never); engine_reserve_terms allocates them at once
-// instead.
+// instead and returns the bytes they take: all that were offered, or none where
+// they are too few for a pass of two samples or the device has no room.
 void engine_limit_terms(Engine* e, uint64_t bytes);
-int engine_reserve_terms(Engine* e, uint64_t bytes);
+uint64_t engine_reserve_terms(Engine* e, uint64_t bytes);
 // Large passes run as two parts side by side; the second one's traversal stacks
 // overflow to an area of their own.  engine_limit_terms lets it be allocated on
 // use; engine_reserve_side allocates it (engine_side_bytes) at once.

@@ -1596,16 +1596,16 @@ int engine_reserve_side(Engine* e) {
     return GPR_ERR_OOM;
 }
 
-int engine_reserve_terms(Engine* e, uint64_t bytes) {
+uint64_t engine_reserve_terms(Engine* e, uint64_t bytes) {
     const uint64_t paths = std::min<uint64_t>(e->capacity, kPassPaths);  // one term count (a byte) each
-    if (bytes <= 64 * paths) return GPR_OK;
+    if (bytes <= 64 * paths) return 0;
     if (e->nterm.alloc(paths) != GPR_OK || e->terms.alloc(bytes - paths) != GPR_OK) {
         (void)hipGetLastError();  // the failed allocation
         e->nterm.release();
-        return GPR_ERR_OOM;
+        return 0;
     }
     e->term_limit = bytes - paths;
-    return GPR_OK;
+    return bytes;
 }
 
 namespace {

@@ -660,10 +660,7 @@ int gpr_server_create(const gpr_server_opts* o, gpr_server** out) {
     if (side > 0 && rest > frames + side && rest - frames - side >= kTermBytesPerPath * o->capacity &&
         engine_reserve_side(s->eng) == GPR_OK)
         rest -= side;
-    if (rest > frames) {
-        const uint64_t terms = std::min(rest - frames, kServerTermBytes);
-        if (engine_reserve_terms(s->eng, terms) == GPR_OK) rest -= terms;
-    }
+    if (rest > frames) rest -= engine_reserve_terms(s->eng, std::min(rest - frames, kServerTermBytes));
     const uint64_t fb_pixels = std::min<uint64_t>(rest / 16, (1ull << 31) - 1);
     GPR_TRY(s->arena.mem.alloc(std::max<uint64_t>(o->arena_bytes, 256)));
     GPR_TRY(s->fb.alloc(16 * fb_pixels));

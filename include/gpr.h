@@ -436,14 +436,18 @@ int gpr_batch_free(gpr_batch* b);
 
 typedef struct gpr_server gpr_server;
 typedef struct {
-    uint64_t hbm_budget;  /* device bytes for arena + queues + frame buffers */
+    uint64_t hbm_budget;  /* device bytes for arena + queues + frame buffers + what passes of several samples need */
     uint64_t arena_bytes; /* part of the budget for scenes */
     uint32_t capacity;    /* paths per pass */
     uint32_t max_jobs;    /* jobs in flight, <= 1024 */
 } gpr_server_opts;
-/* Starts the server's loop thread.  Frame buffers of admitted requests come
- * out of hbm_budget - arena_bytes - the engine's queues; a request waits until
- * its frame buffer fits and a job slot is free. */
+/* Starts the server's loop thread.  Of hbm_budget - arena_bytes - the engine's
+ * queues, the frame buffers of admitted requests get 64 bytes a path of the
+ * capacity (four full passes) or all there is.  What is left goes to passes of
+ * several samples a job, to the second half of large passes (up to 400 MB, if
+ * lists of terms still fit) and to lists of terms (up to 2.4 GB, if more than 64
+ * bytes a path remain), and the rest to frame buffers again.  A request waits
+ * until its frame buffer fits and a job slot is free. */
 int gpr_server_create(const gpr_server_opts* opts, gpr_server** out);
 int gpr_server_add_scene(gpr_server* s, const gpr_scene* scene, uint32_t* id);
 /* Queue a request; returns at once with a ticket.  GPR_ERR_BUDGET if the

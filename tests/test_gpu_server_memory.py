@@ -36,3 +36,32 @@ def test_a_configured_server_keeps_its_two_parts(cfg):
         for g in got:
             assert np.array_equal(g.view(np.uint32), want.view(np.uint32))
     srv.free()
+
+
+# budgets from the smallest accepted one up: none, a few and many bytes a path beyond the queues and four passes of frames
+@pytest.mark.parametrize("bytes_a_path", [17, 40, 70, 100, 127, 140, 300])
+def test_a_server_uses_its_whole_budget(bytes_a_path):
+    import torch
+    arena, capacity = 1 << 20, 1 << 22
+
+    def used(budget):
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        srv = gpr.Server(budget, arena, capacity=capacity, max_jobs=4)
+        after = torch.cuda.mem_get_info()[0]
+        srv.free()
+        return before - after
+
+    lo, hi = 0, 4 << 30  # the smallest accepted budget: arena, queues and a frame of the capacity
+    while hi - lo > 1 << 16:
+        mid = (lo + hi) // 2
+        try:
+            gpr.Server(mid, arena, capacity=capacity, max_jobs=4).free()
+            hi = mid
+        except gpr.GprError:
+            lo = mid
+    budget = hi - 16 * capacity + bytes_a_path * capacity
+    got = used(budget)
+    print(f"[server] {bytes_a_path} B a path: budget {budget >> 20} MiB, in use {got >> 20}", flush=True)
+    # allocations are whole 2-MiB pages, some twenty of them; streams and events take a few more
+    assert budget - (48 << 20) < got < budget + (64 << 20)
