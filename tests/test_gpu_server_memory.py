@@ -65,3 +65,15 @@ def test_a_server_uses_its_whole_budget(bytes_a_path):
     print(f"[server] {bytes_a_path} B a path: budget {budget >> 20} MiB, in use {got >> 20}", flush=True)
     # allocations are whole 2-MiB pages, some twenty of them; streams and events take a few more
     assert budget - (48 << 20) < got < budget + (64 << 20)
+
+
+# the smallest budgets that servers of these capacities were accepted with before passes had two parts and eight claim
+# counters, with 1 MiB of arena and 256 compute units
+@pytest.mark.parametrize("capacity,budget", [(1000, 2289165), (10000, 11689485), (65536, 68484621), (131072, 135724557),
+                                             (262144, 270204429), (500000, 482566669), (655360, 522649101),
+                                             (1048576, 624098829), (1310720, 691731981), (4194304, 1435696653)])
+def test_small_budgets_are_accepted(capacity, budget):
+    import torch
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the stack overflow area depends on the number of compute units")
+    gpr.Server(budget, 1 << 20, capacity=capacity, max_jobs=4).free()
