@@ -1330,9 +1330,17 @@ struct SideStream {
         if (joined) (void)hipEventDestroy(joined);
     }
 };
+// Device memory that is free.  On a nearly full device the runtime's figure can
+// fall below zero and wrap.
+int free_bytes(uint64_t* out) {
+    size_t free = 0, total = 0;
+    GPR_HIP(hipMemGetInfo(&free, &total));
+    *out = free <= total ? free : 0;
+    return GPR_OK;
+}
+uint64_t queue_bytes(uint32_t n, bool with_job) { return (uint64_t)n * (16 * 4 + 4 + 8 + (with_job ? 4 : 0)) + 8 * 256; }
 int alloc_queue(DevBuf& mem, QueueView& q, uint32_t n, bool with_job) {
-    const size_t per = 16 * 4 + 4 + 8 + (with_job ? 4 : 0);
-    GPR_TRY(mem.alloc((size_t)n * per + 8 * 256));
+    GPR_TRY(mem.alloc(queue_bytes(n, with_job)));
     char* p = mem.as<char>();
     size_t off = 0;
     auto take = [&](size_t bytes) {
@@ -1731,6 +1739,16 @@ struct PassWork {
     QueueView q[3];
     uint32_t paths = 0, depth = 0;
     uint64_t gen = 0;  // of the buffers; graphs captured with older ones are dropped
+    // the smallest buffers whose allocation failed, and the memory free then (these
+    // buffers given back): as large ones are not tried again before more is free
+    uint64_t refused = 0, refused_free = 0;
+    uint64_t held() const {
+        return qmem[0].bytes + qmem[1].bytes + qmem[2].bytes + terms.bytes + nterm.bytes;
+    }
+    void release_pass() {
+        for (DevBuf* b : {&qmem[0], &qmem[1], &qmem[2], &terms, &nterm}) b->release();
+        paths = depth = 0;
+    }
 };
 namespace {
 std::mutex g_work_mu;
@@ -1904,24 +1922,42 @@ int pass_graph(gpr_renderer* r, uint32_t log_s, uint32_t parts, hipGraphExec_t* 
 
 namespace {
 // Makes the stream's pass buffers hold `paths` paths of r's depth (w.mu held,
-// no pass in flight).
+// no pass in flight).  Buffers that cannot fit leave the present ones as they
+// are; if memory runs out all the same, nothing is kept of either.
 int grow_work(gpr_renderer* r, PassWork& w, uint32_t paths) {
+    if (w.paths >= paths && w.terms.bytes >= 16ull * paths * max_terms(r->opts.max_depth)) return GPR_OK;
+    uint64_t free = 0;
+    GPR_TRY(free_bytes(&free));
+    free += w.held();
+    const auto bytes = [](uint32_t n, uint32_t depth) {
+        return 3 * queue_bytes(pass_entries(n, false), false) + 16ull * n * max_terms(depth) + n;
+    };
     const uint32_t depth = std::max(w.depth, r->opts.max_depth);
     const uint32_t n = std::max(w.paths, paths);
     // a deeper render after a larger one: not both at once if that breaks the bound
-    const bool both = n * path_bytes(depth) <= kPassBytes;
+    const bool both = n * path_bytes(depth) <= kPassBytes && bytes(n, depth) <= free;
     const uint32_t np = both ? n : paths, nd = both ? depth : r->opts.max_depth;
-    if (w.paths >= paths && w.terms.bytes >= 16ull * paths * max_terms(r->opts.max_depth)) return GPR_OK;
-    w.paths = w.depth = 0;
+    const uint64_t need = bytes(np, nd);
+    const bool tried = w.refused && need >= w.refused && free < w.refused_free + (64ull << 20);
+    if (tried || need > free) return fail(GPR_ERR_OOM, "no device memory for a pass of several samples");
     {
         std::lock_guard<std::mutex> lk(g_work_mu);
         w.gen = ++g_work_gen;
     }
     // given back first, so that the old and the new buffers never exist together
-    for (DevBuf* b : {&w.qmem[0], &w.qmem[1], &w.qmem[2], &w.terms, &w.nterm}) b->release();
-    for (int k = 0; k < 3; ++k) GPR_TRY(alloc_queue(w.qmem[k], w.q[k], pass_entries(np, false), false));
-    GPR_TRY(w.terms.alloc(16ull * np * max_terms(nd)));
-    GPR_TRY(w.nterm.alloc(np));
+    w.release_pass();
+    int rc = GPR_OK;
+    for (int k = 0; k < 3 && rc == GPR_OK; ++k) rc = alloc_queue(w.qmem[k], w.q[k], pass_entries(np, false), false);
+    if (rc == GPR_OK) rc = w.terms.alloc(16ull * np * max_terms(nd));
+    if (rc == GPR_OK) rc = w.nterm.alloc(np);
+    if (rc != GPR_OK) {
+        (void)hipGetLastError();  // the failed allocation
+        w.release_pass();
+        w.refused = need;
+        w.refused_free = free;
+        return rc;
+    }
+    if (need >= w.refused) w.refused = 0;
     w.paths = np;
     w.depth = nd;
     return GPR_OK;
@@ -1936,10 +1972,7 @@ uint32_t plan_passes(gpr_renderer* r, PassWork& w, uint32_t spp) {
     while (k < kMaxLogS && (2u << k) <= spp && ((uint64_t)r->npix << (k + 1)) <= kPassPaths &&
            ((uint64_t)r->npix << (k + 1)) * path_bytes(r->opts.max_depth) <= kPassBytes)
         ++k;
-    while (k > 0 && grow_work(r, w, r->npix << k) != GPR_OK) {
-        (void)hipGetLastError();  // the failed allocation
-        --k;
-    }
+    while (k > 0 && grow_work(r, w, r->npix << k) != GPR_OK) --k;
     if (k > 0 && r->work_gen != w.gen) {
         r->drop_graphs();
         r->work_gen = w.gen;
