@@ -1619,12 +1619,20 @@ uint64_t engine_reserve_terms(Engine* e, uint64_t bytes) {
 }
 
 namespace {
-// Term lists for a pass of `size` paths; false (and none larger from then on)
-// where the device has no room for them.
+// Term lists for a pass of `size` paths; false (and none as large from then on)
+// where the device has no room for them.  Lists that cannot fit leave the
+// present ones as they are.
 int grow_terms(Engine* e, uint32_t size, uint32_t depth, hipStream_t st, bool* ok) {
     const uint64_t need = 16ull * size * max_terms(depth);
     *ok = true;
     if (need <= e->terms.bytes && size <= e->nterm.bytes) return GPR_OK;
+    uint64_t free = 0;
+    GPR_TRY(free_bytes(&free));
+    if (need + size > free + e->terms.bytes + e->nterm.bytes) {
+        e->term_limit = need - 1;
+        *ok = false;
+        return GPR_OK;
+    }
     GPR_HIP(hipStreamSynchronize(st));  // passes in flight use the old lists
     for (size_t g = e->graphs.size(); g-- > 0;)
         if (e->graphs[g].first.terms) {
@@ -1635,7 +1643,7 @@ int grow_terms(Engine* e, uint32_t size, uint32_t depth, hipStream_t st, bool* o
         (void)hipGetLastError();
         e->terms.release();
         e->nterm.release();
-        e->term_limit = 0;
+        e->term_limit = need - 1;
         *ok = false;
     }
     return GPR_OK;
@@ -1652,23 +1660,24 @@ int engine_fill_pass(Engine* e, std::vector<EngineJob>& jobs, const std::vector<
         while (s < k && (2u << s) <= left[i]) ++s;
         return s;
     };
-    uint32_t best = 0, size = 0;
-    for (uint32_t k = 1; k <= kMaxLogS; ++k) {
-        uint64_t paths = 0;
-        bool any = false;
-        for (size_t i = 0; i < jobs.size(); ++i) {
-            const uint32_t s = samples(i, k);
-            any = any || s == k;
-            paths += (uint64_t)jobs[i].npix << s;
+    for (bool ok = false; !ok;) {
+        uint32_t best = 0, size = 0;
+        for (uint32_t k = 1; k <= kMaxLogS; ++k) {
+            uint64_t paths = 0;
+            bool any = false;
+            for (size_t i = 0; i < jobs.size(); ++i) {
+                const uint32_t s = samples(i, k);
+                any = any || s == k;
+                paths += (uint64_t)jobs[i].npix << s;
+            }
+            if (!any || paths > most || 16ull * size_class(e, paths) * max_terms(depth) > e->term_limit) break;
+            best = k;
+            size = size_class(e, paths);
         }
-        if (!any || paths > most || 16ull * size_class(e, paths) * max_terms(depth) > e->term_limit) break;
-        best = k;
-        size = size_class(e, paths);
+        if (best == 0) return GPR_OK;
+        GPR_TRY(grow_terms(e, size, depth, st, &ok));  // where it fails, the limit is below this pass
+        for (size_t i = 0; ok && i < jobs.size(); ++i) jobs[i].log_s = samples(i, best);
     }
-    if (best == 0) return GPR_OK;
-    bool ok = false;
-    GPR_TRY(grow_terms(e, size, depth, st, &ok));
-    for (size_t i = 0; ok && i < jobs.size(); ++i) jobs[i].log_s = samples(i, best);
     return GPR_OK;
 }
 
