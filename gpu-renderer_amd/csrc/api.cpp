@@ -687,8 +687,7 @@ int trace_host_pipelined(gpr_scene* s, const SceneView& sv, const gpr_ray* rays,
             GPR_HIP(hipMemcpyAsync(dr + off, rays + off, m * sizeof(gpr_ray), hipMemcpyHostToDevice, cin));
             GPR_HIP(hipEventRecord(ev[c], cin));
             GPR_HIP(hipStreamWaitEvent(st, ev[c], 0));
-            GPR_TRY(launch_trace(sv, dr + off, dh + off, m, flags, nullptr, st, s->trace_nt, s->trace_sl,
-                                 s->trace_chunk, s->trace_refill));
+            GPR_TRY(launch_scene_trace(s, sv, dr + off, dh + off, m, flags, nullptr, st));
             GPR_TRY(trace_overflow_accumulate(dov.as<unsigned long long>(), st));
             GPR_HIP(hipEventRecord(ev[nch + c], st));
             if (c > 0) GPR_TRY(copy_out(c - 1));
@@ -749,8 +748,7 @@ int gpr_trace(gpr_scene* s, const gpr_ray* rays, gpr_hit* hits, uint64_t n, uint
         return GPR_OK;
     }
     if (flags & GPR_TRACE_DEVICE_PTRS)
-        return launch_trace(sv, rays, hits, n, flags, stats, stream(), s->trace_nt, s->trace_sl, s->trace_chunk,
-                            s->trace_refill);
+        return launch_scene_trace(s, sv, rays, hits, n, flags, stats, stream());
     TraceStaging* sg = staging_for_stream();
     std::lock_guard<std::mutex> lk(sg->mu);
     DevBuf& dr = sg->rays;
@@ -760,8 +758,7 @@ int gpr_trace(gpr_scene* s, const gpr_ray* rays, gpr_hit* hits, uint64_t n, uint
     if (!(flags & GPR_TRACE_REF_ORDER) && n > kHostChunk)
         return trace_host_pipelined(s, sv, rays, hits, n, flags, dr.as<gpr_ray>(), dh.as<gpr_hit>(), sg->ov);
     GPR_HIP(hipMemcpyAsync(dr.p, rays, n * sizeof(gpr_ray), hipMemcpyHostToDevice, stream()));
-    GPR_TRY(launch_trace(sv, dr.as<gpr_ray>(), dh.as<gpr_hit>(), n, flags, stats, stream(), s->trace_nt,
-                         s->trace_sl, s->trace_chunk, s->trace_refill));
+    GPR_TRY(launch_scene_trace(s, sv, dr.as<gpr_ray>(), dh.as<gpr_hit>(), n, flags, stats, stream()));
     GPR_HIP(hipMemcpyAsync(hits, dh.p, n * sizeof(gpr_hit), hipMemcpyDeviceToHost, stream()));
     GPR_HIP(hipStreamSynchronize(stream()));
     unsigned long long ov = 0;
@@ -780,6 +777,7 @@ int gpr_trace_set_cfg(gpr_scene* s, const gpr_trace_cfg* c) {
     s->trace_sl = (int)c->stack;
     s->trace_chunk = (int)c->chunk;
     s->trace_refill = c->refill ? 1 : 0;
+    s->trace_pinned = true;
     return GPR_OK;
 }
 
@@ -825,6 +823,7 @@ int gpr_trace_tune(gpr_scene* s, const gpr_ray* rays, uint64_t n, uint32_t flags
     s->trace_sl = (int)res[0].stack;
     s->trace_chunk = (int)res[0].chunk;
     s->trace_refill = (int)res[0].refill;
+    s->trace_pinned = false;
     if (nout) *nout = (uint32_t)std::min<size_t>(cap, res.size());
     if (out)
         for (uint32_t k = 0; k < cap && k < res.size(); ++k) out[k] = res[k];

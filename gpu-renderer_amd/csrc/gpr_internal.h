@@ -215,6 +215,7 @@ struct gpr_scene {
     float r2c[16];
     uint64_t last_nv = 0, last_nt = 0;
     int trace_nt = 0, trace_sl = 0, trace_chunk = 0, trace_refill = 0;  // BVH4 traversal launch configuration (nt 0: by batch)
+    bool trace_pinned = false;  // set by the caller: short batches take it too
     gpr::SceneView view() const;
 };
 
@@ -234,6 +235,9 @@ int sort_prepare(void* scratch, size_t bytes, hipStream_t st);
 int launch_trace(const SceneView& sv, const gpr_ray* rays, gpr_hit* hits, uint64_t n, uint32_t flags,
                  unsigned long long* stats, hipStream_t st, int nt = 0, int sl = 0, int chunk = 0, int refill = 0);
 bool trace_cfg_valid(int nt, int sl, int chunk);
+// launch_trace as the scene is configured
+int launch_scene_trace(const gpr_scene* s, const SceneView& sv, const gpr_ray* rays, gpr_hit* hits, uint64_t n,
+                       uint32_t flags, unsigned long long* stats, hipStream_t st);
 int launch_trace_stats(const SceneView& sv, const gpr_ray* rays, uint64_t n, bool any, unsigned long long* stats,
                        hipStream_t st);
 int trace_release_stream(hipStream_t st);

@@ -375,6 +375,17 @@ void trace_default_cfg(uint64_t n, bool any, int& nt, int& sl, int& chunk, int& 
 }
 }  // namespace
 
+// A tuned shape is one of a lane to a ray, also where it was found on a short batch:
+// those keep the four lanes.  2,000 / 131,072 rays at 1M triangles, us: not tuned 97 /
+// 266; with the shape tuned on 4M rays 172 / 355, on themselves 126 / 303; now 96 / 264
+// either way.
+int launch_scene_trace(const gpr_scene* s, const SceneView& sv, const gpr_ray* rays, gpr_hit* hits, uint64_t n,
+                       uint32_t flags, unsigned long long* stats, hipStream_t st) {
+    const bool by_batch = !s->trace_pinned && n <= kQuadRays;
+    return launch_trace(sv, rays, hits, n, flags, stats, st, by_batch ? 0 : s->trace_nt, s->trace_sl, s->trace_chunk,
+                        s->trace_refill);
+}
+
 int launch_trace(const SceneView& sv, const gpr_ray* rays, gpr_hit* hits, uint64_t n, uint32_t flags,
                  unsigned long long* stats, hipStream_t st, int nt, int sl, int chunk, int refill) {
     if (n == 0) return GPR_OK;

@@ -288,7 +288,9 @@ int gpr_trace(gpr_scene* s, const gpr_ray* rays, gpr_hit* hits, uint64_t n, uint
  * rays (flags: GPR_TRACE_DEVICE_PTRS, optionally GPR_TRACE_ANY): block size
  * {64,128,256,512} x LDS stack {8,16,32} x chunk {64,128,256} x per-lane ray
  * refill {off, on}; the fastest is
- * kept for the scene's later gpr_trace calls.  Results do not depend on the
+ * kept for the scene's later gpr_trace calls of more than 131,072 rays (shorter
+ * batches walk a ray with four lanes, as on a scene that was not tuned; a
+ * configuration from gpr_trace_set_cfg holds for them too).  Results do not depend on the
  * configuration.  No counterpart in the reference (its traversal launch shape
  * is fixed, pathtracer_kernel.h:235-246). */
 int gpr_trace_tune(gpr_scene* s, const gpr_ray* rays, uint64_t n, uint32_t flags, gpr_trace_cfg* out,
