@@ -188,9 +188,11 @@ GPR_D int32_t split_weight(const uint32_t* __restrict__ sk, uint32_t n, const ui
 // or invalidate is needed although the eight XCD L2 caches are not coherent
 // with each other; device-scope release / acquire on the RMW would add both
 // on every arrival (measured 16x slower at 1M triangles).  Values read back
-// are range-checked, and k_export_ref checks every parent box against the
-// union of its children's, so a protocol failure raises the error word
-// instead of indexing out of bounds or producing a wrong tree silently.
+// are range-checked, and the layout kernels check every parent box against the
+// union of its children's (k_layout inside a block, and that a block's own
+// subtrees have the boxes that were published; k_layout_top above), so a protocol
+// failure raises the error word instead of indexing out of bounds or producing a
+// wrong tree silently.
 GPR_D void pub(uint32_t* p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 GPR_D uint32_t get(uint32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 GPR_D void pub8(uint64_t* p, uint64_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -210,8 +212,10 @@ GPR_D void get2(uint64_t* p, float& a, float& b) {
 // The layout pass builds the same subtrees again from the triangle records
 // rather than reading 60 bytes a node back.  Both passes are bound by memory:
 // random reads of the positions in the first, 180 MB of layouts written in the
-// second.  Tree, refit and layouts of a 1M-triangle soup take 176 us
+// second.  Tree, refit and layouts of a 1M-triangle soup take 168 us
 // instead of the 559 of one published climb per leaf and a kernel per layout.
+// Weights fit 16 bits; with 32 a block of k_layout took 41,008 bytes of LDS, three
+// to a CU instead of four: 80.7 us without its checks, 82.6 with them, now 75.8.
 constexpr uint16_t kNoNode = 0xffff;
 // Node codes inside a block: internal node of split j is j, leaf i is kTreeB + i.
 struct TreeShared {
@@ -220,7 +224,7 @@ struct TreeShared {
     uint16_t ch[2][kTreeB];
     uint16_t lo[kTreeB], hi[kTreeB];  // leaf range
     uint32_t cnt[kTreeB];             // arrivals: 2 = built here
-    int32_t w[kTreeB + 1];            // w[j]: weight of the split before leaf j, -1 before the first and after the last
+    int16_t w[kTreeB + 1];            // w[j]: weight of the split before leaf j, -1 before the first and after the last
 };
 // Where a thread's climb ended: the local subtree it holds, and whether that
 // subtree is a root of its block's forest.
@@ -333,7 +337,7 @@ __global__ __launch_bounds__(kTreeB) void k_tree(const float* __restrict__ pos, 
     for (uint32_t j = threadIdx.x; j <= m; j += kTreeB) {
         const bool inside = (j > 0 || before) && (j < m || after);
         const int32_t v = inside ? split_weight(sk, n, keys, s - before, nkeys - 1, s + j - 1) : -1;
-        S.w[j] = v;
+        S.w[j] = (int16_t)v;
         if (j > 0) w[s + j - 1] = v;
     }
     const Climb c = local_tree(S, n, s, m, lo, hi);
@@ -480,6 +484,10 @@ GPR_D void put_ref(gpr_ref_node* __restrict__ ref, uint32_t nn, uint32_t at, con
     o[1] = make_float4(b[4], b[5], __uint_as_float(idx), __uint_as_float(leaf));
 }
 
+// Bound `q` (lox loy loz hix hiy hiz) of the union of a left and a right child.
+GPR_D float union_of(int q, float l, float r) { return q < 3 ? fmin_h(l, r) : fmax_h(l, r); }
+GPR_D bool same_bits(float a, float b) { return __float_as_uint(a) == __float_as_uint(b); }
+
 // Layouts of the nodes built inside blocks: reference nodes, BVH4 nodes, and
 // for the published nodes above what they need of the subtrees below them.
 __global__ __launch_bounds__(kTreeB) void k_layout(uint32_t n, const TriRec* __restrict__ tris,
@@ -508,7 +516,7 @@ __global__ __launch_bounds__(kTreeB) void k_layout(uint32_t n, const TriRec* __r
         tri = __float_as_uint(c.y);
         tri_bounds(q, lo, hi);
     }
-    for (uint32_t j = i; j <= m; j += kTreeB) S.w[j] = s + j > 0 ? w[s + j - 1] : -1;
+    for (uint32_t j = i; j <= m; j += kTreeB) S.w[j] = (int16_t)(s + j > 0 ? w[s + j - 1] : -1);
     const Climb c = local_tree(S, n, s, m, lo, hi);
     if (c.root) {
         uint32_t l = 0, d = 0;
@@ -516,6 +524,12 @@ __global__ __launch_bounds__(kTreeB) void k_layout(uint32_t n, const TriRec* __r
             const uint32_t p = (uint32_t)((int64_t)s + c.parent);
             l = left[p] + (c.as_left ? 1u : 0u);
             d = depth[p] + 1;
+            // the box that k_tree published is this build's
+            const float2* b = reinterpret_cast<const float2*>(box + 6ull * node_id(c.code, s, n));
+            const float2 x = b[0], y = b[1], z = b[2];
+            if (!(same_bits(x.x, c.lo.x) && same_bits(x.y, c.lo.y) && same_bits(y.x, c.lo.z) && same_bits(y.y, c.hi.x) &&
+                  same_bits(z.x, c.hi.y) && same_bits(z.y, c.hi.z)))
+                atomicOr(&bs->err, 2u);
         }
         s_left[c.code] = (uint16_t)l;
         s_depth[c.code] = (uint16_t)d;
@@ -586,6 +600,14 @@ __global__ __launch_bounds__(kTreeB) void k_layout(uint32_t n, const TriRec* __r
         }
         reinterpret_cast<float4*>(out + base + (w >> 3))[piece] = make_float4(v[0], v[1], v[2], v[3]);
     }
+    // every parent's box against its children's
+    if (inner) {
+        const uint32_t c0 = S.ch[0][i], c1 = S.ch[1][i];
+        bool same = c0 < 2 * kTreeB && c1 < 2 * kTreeB;
+#pragma unroll
+        for (int q = 0; q < 6; ++q) same = same && same_bits(union_of(q, S.box[q][c0], S.box[q][c1]), S.box[q][i]);
+        if (!same) atomicOr(&bs->err, 2u);
+    }
     if (c.root && c.code < kTreeB) {
         const uint32_t id = s + c.code;
         if ((s_depth[c.code] & 1u) == 0) {
@@ -624,9 +646,8 @@ __global__ __launch_bounds__(kB) void k_layout_top(uint32_t n, const uint32_t* _
             continue;
         }
         if (piece < 6) {
-            const float a = box[6ull * c[0] + piece], b = box[6ull * c[1] + piece];
-            const float u = piece < 3 ? fmin_h(a, b) : fmax_h(a, b);
-            if (__float_as_uint(u) != __float_as_uint(box[6ull * x + piece])) atomicOr(&bs->err, 2u);
+            const float u = union_of(piece, box[6ull * c[0] + piece], box[6ull * c[1] + piece]);
+            if (!same_bits(u, box[6ull * x + piece])) atomicOr(&bs->err, 2u);
         } else if (piece == 6) {
             put_ref(ref, nn, 2 * (uint32_t)ends[2ull * x] + lf, box + 6ull * x, 2 * (x + 1) + lf, 0u, bs);
         }
