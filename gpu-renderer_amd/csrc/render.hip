@@ -394,56 +394,56 @@ GPR_D float power_heur(float a, float b) {
     return a / (a + b);
 }
 
-// Walks a segmented queue in turns of 2^lg entries; every member is uniform.
+// Walks a segmented queue in turns of 2^lg entries.  Uniform: written member by
+// member and chosen from as scalars.  With arrays the compiler kept the walk in each
+// lane's scratch memory (44 B; 92 in k_trace) or, in k_shade and the 32-entry shapes,
+// in 11 KB of LDS: 16 samples of the 256x256 Cornell box 753 us, now 701; 8 of the
+// 803x451 textured scene 2610 and 2521; the batch 40.0 ms and 38.0, 16 served jobs
+// 150 and 138.
 struct SegWalk {
-    uint32_t n[kMaxSegs], first[kMaxSegs];  // a segment's entries, and the turn it starts at
+    uint32_t n0, n1, n2, n3;  // entries of the segments
+    uint32_t f1, f2, f3;      // the turns that they start at (the first one at 0)
     uint32_t turns, cap, lg;
+    GPR_D uint32_t turns_of(uint32_t n) const { return (n + (1u << lg) - 1) >> lg; }
     GPR_D void init(uint32_t seg_cap, uint32_t log_turn) {
         cap = seg_cap;
         lg = log_turn;
-        turns = 0;
-#pragma unroll
-        for (uint32_t g = 0; g < kMaxSegs; ++g) {
-            first[g] = turns;
-            turns += (n[g] + (1u << lg) - 1) >> lg;
-        }
+        f1 = turns_of(n0);
+        f2 = f1 + turns_of(n1);
+        f3 = f2 + turns_of(n2);
+        turns = f3 + turns_of(n3);
     }
-    GPR_D uint32_t total() const {
-        uint32_t t = 0;
-#pragma unroll
-        for (uint32_t g = 0; g < kMaxSegs; ++g) t += n[g];
-        return t;
-    }
+    GPR_D uint32_t total() const { return n0 + n1 + n2 + n3; }
     GPR_D void range(uint32_t turn, uint32_t& begin, uint32_t& end) const {
         // the last segment that starts at or before the turn (empty ones before it start there too)
-        uint32_t g = 0, f = first[0], m = n[0];
-#pragma unroll
-        for (uint32_t k = 1; k < kMaxSegs; ++k) {
-            const bool later = first[k] <= turn;
-            g = later ? k : g;
-            f = later ? first[k] : f;
-            m = later ? n[k] : m;
-        }
+        const auto uni = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane(v); };
+        const uint32_t s1 = uni(f1), s2 = uni(f2), s3 = uni(f3), m0 = uni(n0), m1 = uni(n1), m2 = uni(n2), m3 = uni(n3);
+        const bool after1 = turn >= s1, after2 = turn >= s2, after3 = turn >= s3;
+        const uint32_t g = after3 ? 3u : after2 ? 2u : after1 ? 1u : 0u;
+        const uint32_t f = after3 ? s3 : after2 ? s2 : after1 ? s1 : 0u;
+        const uint32_t m = after3 ? m3 : after2 ? m2 : after1 ? m1 : m0;
         const uint32_t off = (turn - f) << lg;
         begin = g * cap + off;
         end = g * cap + min(off + (1u << lg), m);
     }
 };
+static_assert(kMaxSegs == 4, "a walk has four segments");
 // Entries of the primary queue (one segment of all paths), or of what bounce
 // `bounce` appended.
 enum QueueKind { kPrimary, kScatter, kShadow };
 template <QueueKind KIND, bool MULTI>
+GPR_D uint32_t seg_count(const RenderArgs& a, uint32_t bounce, uint32_t g) {
+    if constexpr (KIND == kPrimary) return g == 0 ? npaths_of<MULTI>(a) : 0u;
+    if (g >= a.nseg) return 0u;
+    const unsigned long long v = *seg_at(a, bounce, g);
+    return __builtin_amdgcn_readfirstlane(KIND == kShadow ? (uint32_t)(v >> 32) : (uint32_t)v);
+}
+template <QueueKind KIND, bool MULTI>
 GPR_D void seg_counts(const RenderArgs& a, uint32_t bounce, SegWalk& w) {
-#pragma unroll
-    for (uint32_t g = 0; g < kMaxSegs; ++g) {
-        w.n[g] = 0;
-        if constexpr (KIND == kPrimary) {
-            if (g == 0) w.n[g] = npaths_of<MULTI>(a);
-        } else if (g < a.nseg) {
-            const unsigned long long v = *seg_at(a, bounce, g);
-            w.n[g] = __builtin_amdgcn_readfirstlane(KIND == kShadow ? (uint32_t)(v >> 32) : (uint32_t)v);
-        }
-    }
+    w.n0 = seg_count<KIND, MULTI>(a, bounce, 0);
+    w.n1 = seg_count<KIND, MULTI>(a, bounce, 1);
+    w.n2 = seg_count<KIND, MULTI>(a, bounce, 2);
+    w.n3 = seg_count<KIND, MULTI>(a, bounce, 3);
 }
 // Calls f(i) for the entries of a queue, a turn's lanes together.
 template <QueueKind KIND, bool MULTI, int NT, class F>
@@ -1423,6 +1423,10 @@ int engine_create(int device, uint32_t capacity, uint32_t max_jobs, Engine** out
         const PassKernels& pk = pass_kernel_table(k);
         int per_cu = 0;
         GPR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pk.trace, pk.nt, 0));
+        // Blocks of 256 threads and more: four waves a SIMD though five fit.  Batch of
+        // 12 scenes / burst of 16 requests, four waves and five: 256x16 40.4 / 144 ms
+        // and 42.4 / 148, but 64x8 41.5 / 151 and 40.3 / 146, 128x16 40.8 / 149 and 41.1 / 146.
+        if (pk.nt >= 256) per_cu = std::min(per_cu, 1024 / pk.nt);
         // more persistent threads than queue entries would only idle
         e->grid[k] = std::max(1, std::min<int>(cus * std::max(1, per_cu), (int)div_up(capacity, pk.nt)));
         threads = std::max(threads, (size_t)e->grid[k] * pk.nt);
@@ -1845,8 +1849,8 @@ RenderArgs make_args(gpr_renderer* r, uint32_t log_s) {
 }
 
 // Block size and LDS stack entries per lane of the single-scene renderer's
-// traversal.  12 entries keep the LDS of a closest-hit block at 24 KB, six
-// blocks to a CU as its registers allow; 8 / 12 / 16 entries: 8 samples of the
+// traversal.  12 entries take 24 KB of LDS a block, room for six to a CU; the
+// registers of both kernels allow five.  8 / 12 / 16 entries: 8 samples of the
 // textured scene 5.03 / 4.85 / 4.88 ms, 4 of the sphere grid 16.7 / 16.7 / 17.1.
 constexpr int kRenderNT = 256, kRenderSL = 12;
 
