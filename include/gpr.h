@@ -316,7 +316,8 @@ int gpr_trace_overflow_count(uint64_t* count);
  * host-buffer traces keep for the calling thread's device and hip_stream
  * (NULL = null stream), after synchronizing that stream; the next call on the
  * stream allocates them again.  For applications that create streams per
- * request or per thread; no other call may use the stream meanwhile.  No
+ * request or per thread; no other call may use the stream meanwhile.  What the
+ * renderers of a stream share (gpr_render) goes with the last of them instead.  No
  * counterpart in the reference (one stream). */
 int gpr_release_stream(void* hip_stream);
 
@@ -334,7 +335,13 @@ typedef struct {
 } gpr_render_opts;
 /* PathTracer(filename) + init() (pathtracer.cu:8-39). */
 int gpr_renderer_create(gpr_scene* s, const gpr_render_opts* opts, gpr_renderer** out);
-/* spp x PathTracer::render() (pathtracer.cu:41-150). */
+/* spp x PathTracer::render() (pathtracer.cu:41-150).
+ * In PCG mode a call of several samples renders up to 64 at once, in passes of at
+ * most 2^23 paths.  Their queues and term lists (229 + 16 * (2 * max_depth + 1)
+ * bytes a path, 6 GB at most) and a second stack overflow area (250 MB) are shared by
+ * the renderers of one (device, stream) and freed with the last of them; where the
+ * device has no room for them, passes hold fewer samples.  The image does not
+ * depend on it. */
 int gpr_render(gpr_renderer* r, uint32_t spp);
 /* Linear radiance sum and per-pixel sample count (FrameBuffer, framebuffer.h:33-70). */
 int gpr_renderer_read(gpr_renderer* r, float* rgb_sum, uint32_t* sample_num);
@@ -412,14 +419,15 @@ typedef struct {
     uint64_t arena_bytes; /* device bytes for the scene arena (see gpr_scene_arena_bytes) */
     uint32_t capacity;    /* paths per pass (queue entries); >= the largest job's pixel count */
     uint32_t max_jobs;    /* jobs per pass, <= 1024 */
-} gpr_batch_opts;
+} gpr_batch_opts; /* besides these, passes of several samples hold term lists of up to 4 GB and a second stack
+                   * overflow area of up to 400 MB, as far as the device has room for them */
 /* Device bytes a committed scene takes in an arena. */
 int gpr_scene_arena_bytes(const gpr_scene* s, uint64_t* bytes);
 int gpr_batch_create(const gpr_batch_opts* opts, gpr_batch** out);
 /* Copy a committed scene into the arena (the scene may be freed afterwards). */
 int gpr_batch_add_scene(gpr_batch* b, const gpr_scene* s, uint32_t* id);
 int gpr_batch_add_job(gpr_batch* b, const gpr_job* job, uint32_t* id);
-/* Autotune the traversal configuration on the batch's own first pass (block
+/* Autotune the traversal configuration on one sample of the jobs of the batch's first pass (block
  * size {64,128,256,512} x LDS stack {8,16,32} x chunk {64..512}, plus the
  * reference layout); best first in out[0..n), n <= cap. */
 int gpr_batch_tune(gpr_batch* b, gpr_trace_cfg* out, uint32_t cap, uint32_t* n);
