@@ -743,9 +743,11 @@ def main():
                      "bytes_formula": "32 ray + 16 hit + 128 * BVH4 node fetches + 48 * triangle tests, per ray, "
                                       "counted on the device (gpr_trace_bvh4_stats)",
                      "mean_bvh4_nodes": round(n_node4, 3), "mean_tri_tests": round(n_tri4, 3),
-                     "limiter": "VALU issue (79 % busy, 39 % of lanes active per instruction) and node-fetch "
-                                "latency (L2 hit 29.6 %); 2.9 TB/s of L2-to-fabric traffic, mostly from the "
+                     "limiter": "VALU issue (82 % busy, 42 % of lanes active per instruction) and node-fetch "
+                                "latency (L2 hit 29.4 %); 3.2 TB/s of L2-to-fabric traffic, mostly from the "
                                 "Infinity Cache: not HBM bandwidth",
+                     "frac_note": "bytes counted per node fetch and triangle test over the HBM peak; caches serve "
+                                  "most of them",
                      "reference_order_diagnostic": {"bytes_per_ray": round(bytes_per_ray_ref, 2),
                                                     "mean_nodes": round(n_node, 3), "mean_tris": round(n_tri, 3),
                                                     "formula": "32 + 16 + 32 * nodes + 36 * tris of the "
@@ -765,8 +767,10 @@ def main():
         "anyhit_roofline": {"bytes_per_ray": round(bytes_per_ray_any, 2),
                             "achieved_gbs": round(bytes_per_ray_any * N_RAYS / (ms_any * 1e-3) / 1e9, 1),
                             "frac": round(bytes_per_ray_any * N_RAYS / (ms_any * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-                            "note": "node / triangle counts of the immediate-leaf walk; the timed kernel "
-                                    "postpones leaves into wave-wide rounds"},
+                            "note": "bytes counted per node fetch and triangle test over the HBM peak; caches "
+                                    "serve most of them, so frac is no share of HBM bandwidth and can pass 1; "
+                                    "counts of the immediate-leaf walk (the timed kernel postpones leaves into "
+                                    "wave-wide rounds)"},
         "closest_hit_fraction": round(hit_frac, 4),
         "stack_overflow_rays": int(overflow),
         "build_ms": {"bounds_morton": round(build_ms[0], 4), "sort": round(build_ms[1], 4),

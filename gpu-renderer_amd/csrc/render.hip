@@ -1,10 +1,11 @@
 // render.hip -- wavefront path tracer on gfx950 (PathTracer::render,
 // src/renderer/pathtracer.cu:41-150, kernels of src/renderer/pathtracer_kernel.h).
 //
-// One sample of every pixel is a fixed launch sequence with no host round
-// trip:  gen -> extend(primary) -> max_depth x { shade -> trace } -> flush
-// -> finish.  Queue sizes live on the device; each kernel reads the size it
-// consumes and early-exits, so the whole sample can be replayed as a hipGraph.
+// A pass of 1 to 64 samples of every pixel is a fixed launch sequence with no host
+// round trip:  gen -> extend(primary) -> max_depth x { shade -> trace } -> flush
+// -> accum (several samples) -> finish, as two such chains side by side where it is
+// large.  Queue sizes live on the device; each kernel reads the size it
+// consumes and early-exits, so the whole pass can be replayed as a hipGraph.
 //
 //   gen     primary rays (InitRandom/NextRandom jitter or PCG32), queue A
 //   extend  closest hit of the primary queue
