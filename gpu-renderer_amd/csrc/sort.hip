@@ -72,17 +72,19 @@ GPR_HD constexpr uint32_t pieces_of(uint32_t n) {
 
 // Every piece reads its whole bucket, so a bucket of m keys costs m * m / step
 // reads.  From kWideMin on most buckets are cut, and with larger pieces a uniform
-// bucket is one; from kRadixMin on the passes cost less than pieces of uniform
-// keys once did, and never more.  Us for uniform keys / keys of 64 clusters, with one
-// block a bucket, pieces of 1536, of 6144, and the passes:
-//    3.1M  uniform  65.9   64.8   62.1          clusters  23319    1749    919
-//    3.2M           75.2   75.3   67.8
-//    4.2M           87.5   84.2   76.1  123              24552   12070   7861   134
-//    8.4M          164    162    139    226              34883   64732  17655   228
-//   14.7M          409    369    308    360              59632  192758  56740   370
-//   16.8M          492    461    354    409              76429  237178          426
-//   67M           2263   3022   2026   1761
-// 4.2M equal keys 285 ms, 65.2 ms, 16.0 ms, 123 us.
+// bucket is one; from kRadixMin on the passes cost less than the pieces of 1536 did
+// for uniform keys, and larger pieces more than one block a bucket did for clustered
+// ones.  Us for uniform keys and keys of 64 clusters, with one block a bucket, pieces
+// of 1536, of 6144, and the passes:
+//          uniform                     clusters
+//    3.0M    55    51    60   110     19934    1528    1300   115
+//    3.2M    75    76    68   112     25288    1868    1459   119
+//    4.2M    88    84    76   124     24499   12175    7770   127
+//    8.4M   164   162   140   217     35059   63632   17815   228
+//   15.7M   446   417   332   397     61723  211131   62331   412
+//   16.8M   492   459   356   413     76482  238898   60209   423
+//   67.1M  2258  3022  2080  1758
+// 4.2M equal keys: 288 ms, 64 ms, 15.9 ms, 116 us.
 constexpr uint32_t kWideMin = 3u << 20, kRadixMin = 15u << 20;
 
 // Top-digit width: ~1K keys per bucket, between 1 and 11 bits.
